@@ -6,22 +6,19 @@
 // merge the partials in chunk order (deterministic). z = L / T as the
 // reference computes logits ./ temperature (src/ModelCPU.jl:1130-1132).
 //
-// Probabilities, their sums and every prefix sum of the draws are fp64:
-// exp((double)z - max) with the exponent's argument exact, sums and scans
-// in double. A draw over 151936 entries of mass ~1e-5 each moves when the
-// cumulative sum errs by a fraction of one entry's mass; fp32 sums err by
-// ~1e-7 of the total, which moved ~0.4 % of residual draws against the
-// exact prefix sums, fp64 ones by ~1e-15.
+// Probabilities, their sums and every prefix sum of the draws are fp64 sums
+// of per-entry fp32 exponentials whose argument is exact (ExpZ: relative
+// error ~1e-7, independent across entries). A draw over 151936 entries of
+// mass ~1e-5 each moves when the cumulative sum errs by a fraction of one
+// entry's mass; fp32 sums err by ~1e-7 of the total, which moved ~0.4 % of
+// residual draws against the exact prefix sums, fp64 ones by ~1e-15.
 //
 // Acceptance (src/SpeculativeDecoding.jl:75-104 with explicit uniforms) runs
-// as four launches: statistics of every target and draft row; one wave per
-// verify step for the ratio tests (lane i judges draft i); per (chunk, step)
-// sums of the sampling weights (residual or bonus distribution); and one
-// workgroup per step that locates u * S by a chunk prefix, then a round
-// prefix, then a wave scan inside the chunk. Every partial sum is formed in
-// one fixed order, and the running value C_j at the last entry of a round
-// or chunk equals the prefix the next level starts from, so the search
-// always lands inside the level it selected.
+// as three launches: statistics of every target and draft row; per (chunk,
+// step) the ratio tests (every chunk's workgroup repeats them, the first
+// publishes) and the chunk's sum of the sampling weights (residual or bonus
+// distribution); and one workgroup per step that locates u * S by a chunk
+// prefix and a scan inside the chunk. Every sum has one fixed order.
 #include "common.h"
 
 namespace {
@@ -41,6 +38,44 @@ __device__ __forceinline__ double dexp(float z, float m) {
     const float e = expf(d);
     return (double)(e > 0.f && e < __builtin_huge_valf() ? fmaf(e, err, e) : e);
 }
+
+// The same over many entries of one row: exp(x / T - m) for m at or above
+// every x / T, ~15 VALU instructions an entry where the division and dexp
+// take ~45 (the statistics of 576 rows of 151936 took 191 us, bound by
+// them). z = x / T by a reciprocal and two fma corrections (RN but for
+// quotients within 2^-24 ulp of a rounding boundary); then z log2 e - M, M =
+// m log2 e, without a rounding before the fraction: M = Mh + Ml with Mh on a
+// grid g on which n + Mh is exact for every integer n in reach, so fma(z,
+// log2 e, -(n + Mh)) rounds once, at a result below 1. An entry 230 below
+// the maximum (-Inf among them) is clamped there: its exp is 0 in fp32
+// either way. NaN stays NaN. Outside 2^-60 <= T <= 2^60 and |m| <= 2^20
+// (fast false: a huge or infinite m has no such grid) the division and dexp
+// are used.
+struct ExpZ {
+    float T, rT, m, xlim, Mh, Ml;
+    bool fast;
+    __device__ __forceinline__ ExpZ(float T_, float m_) : T(T_), m(m_) {
+        fast = T >= 0x1p-60f && T <= 0x1p60f && fabsf(m) <= 0x1p20f;
+        rT = 1.0f / T;
+        xlim = (m - 230.0f) * T;
+        const int il = fast ? ilogbf(fabsf(m) + 256.0f) : 8;
+        const double Md = (double)m * 1.4426950408889634074;
+        Mh = (float)ldexp(rint(ldexp(Md, 22 - il)), il - 22);  // (below 2^24 steps of g = 2^(il - 22))
+        Ml = (float)(Md - (double)Mh);
+    }
+    // (only when fast)
+    __device__ __forceinline__ float quick(float x) const {
+        constexpr float L = 0x1.715476p+0f, LLO = 0x1.4ae0cp-26f;  // log2 e = L + LLO
+        x = x < xlim ? xlim : x;
+        const float q = x * rT;
+        const float z = __builtin_fmaf(__builtin_fmaf(-q, T, x), rT, q);
+        const float n = __builtin_rintf(__builtin_fmaf(z, L, -Mh));
+        float f = __builtin_fmaf(z, L, -(n + Mh));
+        f = __builtin_fmaf(z, LLO, f - Ml);
+        return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
+    }
+    __device__ __forceinline__ double slow(float x) const { return dexp(x / T, m); }
+};
 // exp(m2 - m) in double for rescaling a partial sum (a few per row).
 __device__ __forceinline__ double rescale(float m2, float m) { return exp((double)m2 - (double)m); }
 
@@ -55,20 +90,6 @@ __device__ __forceinline__ MS make_ms(float m, double s) {
     r.pad = 0.f;
     r.s = s;
     return r;
-}
-
-// (m, s) merged with (m2, s2): the smaller maximum's sum rescaled. The same
-// bits whichever argument comes first (a single exp, then a commutative
-// add); a NaN or +Inf entry makes the sum NaN, as exp(Inf - Inf) does.
-__device__ __forceinline__ void merge_ms(float &m, double &s, float m2, double s2) {
-    if (m2 == -__builtin_huge_valf()) return;
-    if (m == -__builtin_huge_valf()) { m = m2; s = s2; return; }
-    if (m >= m2) {
-        s = s + s2 * rescale(m2, m);
-    } else {
-        s = s * rescale(m, m2) + s2;
-        m = m2;
-    }
 }
 
 // Cross-lane moves on the VALU (DPP) and, across rows, one swizzle or
@@ -95,110 +116,143 @@ template <int O> __device__ __forceinline__ double partner_d(double v) {
     return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
-// Butterfly merge of one (max, sum) pair per lane (levels 1, 2, 4, 8, 16,
-// 32 as above); merge_ms is symmetric, so both partners compute the same
-// bits and every lane ends with the same value.
-template <int O> __device__ __forceinline__ void merge_level(float &m, double &s) {
-    const float m2 = partner<O>(m);
-    const double s2 = partner_d<O>(s);
-    merge_ms(m, s, m2, s2);
+// Butterfly sum / maximum over a wave (every lane gets the result).
+__device__ __forceinline__ double wave_sum_d(double v) {
+    v += partner_d<1>(v);
+    v += partner_d<2>(v);
+    v += partner_d<4>(v);
+    v += partner_d<8>(v);
+    v += partner_d<16>(v);
+    v += partner_d<32>(v);
+    return v;
 }
-__device__ __forceinline__ MS wave_merge_pairs(float m, double s) {
-    merge_level<1>(m, s);
-    merge_level<2>(m, s);
-    merge_level<4>(m, s);
-    merge_level<8>(m, s);
-    merge_level<16>(m, s);
-    merge_level<32>(m, s);
-    return make_ms(m, s);
+__device__ __forceinline__ float wave_max_f(float v) {
+    v = fmaxf(v, partner<1>(v));
+    v = fmaxf(v, partner<2>(v));
+    v = fmaxf(v, partner<4>(v));
+    v = fmaxf(v, partner<8>(v));
+    v = fmaxf(v, partner<16>(v));
+    v = fmaxf(v, partner<32>(v));
+    return v;
 }
 
-// Block-wide (max, sum) merge of per-thread pairs.
-__device__ void block_merge_ms(float &m, double &s, MS *sh) {
-    const MS wv = wave_merge_pairs(m, s);
-    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-    if (l == 0) sh[w] = wv;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float M = sh[0].m;
-        double S = sh[0].s;
-        for (int i = 1; i < (int)(blockDim.x >> 6); i++) merge_ms(M, S, sh[i].m, sh[i].s);
-        sh[0] = make_ms(M, S);
+// A chunk's entries over the workgroup: wave w holds the 1024 entries from
+// 1024 w, in PER / 4 rounds of 4 consecutive entries a lane (16-byte loads
+// at any 4-byte alignment), so index order is (wave, round, lane, entry).
+constexpr int PER = CHUNK / NT;  // 16 entries per thread
+constexpr int PR = PER / 4;      // rounds
+__device__ __forceinline__ int entry0(int r) {
+    return (threadIdx.x >> 6) * (CHUNK / 4) + r * 256 + 4 * (threadIdx.x & 63);
+}
+// Entries past V read `fill`.
+__device__ __forceinline__ void load_chunk(const float *__restrict__ src, int c, int V, float fill, float (&x)[PER]) {
+    const int j0 = c * CHUNK;
+    if (j0 + CHUNK <= V) {
+#pragma unroll
+        for (int r = 0; r < PR; r++) __builtin_memcpy(&x[4 * r], src + j0 + entry0(r), 16);
+    } else {
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            const int j = j0 + entry0(i / 4) + (i & 3);
+            x[i] = j < V ? src[j] : fill;
+        }
     }
-    __syncthreads();
-    m = sh[0].m;
-    s = sh[0].s;
-    __syncthreads();
 }
 
 // partial[row][chunk] = (max z, sum exp(z - max)). Rows [0, rows1) come from
 // L1 at temperature T1, except every period-th row (r % period == period - 1,
 // the bonus row of a verify step) at T_last; rows [rows1, ..) come from L2 at
-// T2. Entry c * CHUNK + i * NT + t is thread t's i-th value.
-constexpr int PER = CHUNK / NT;  // 16 entries per thread
+// T2. With parent (a draft tree of rows1 nodes, target rows then draft rows)
+// only the rows of nodes that are some node's parent are formed: the walk
+// reads no others.
+// One maximum over the workgroup's raw logits (the division by T > 0 keeps
+// the order), then every exponential against it: no rescaling exp per thread
+// and merge level. Bound by HBM and VALU together: 576 rows of 151936 (350
+// MB) 191 -> TBD us.
+constexpr int TREE_FILTER = 4 * NT;  // (parents read per workgroup: at most 4 loads a thread)
 __global__ __launch_bounds__(NT) void stats_partial_kernel(const float *__restrict__ L1, int rows1, float T1,
                                                            float T_last, int period, const float *__restrict__ L2,
-                                                           float T2, int V, int nchunk, MS *__restrict__ part) {
-    __shared__ MS sh[NT / 64];
-    const int chunk = blockIdx.x, row = blockIdx.y;
+                                                           float T2, int V, int nchunk,
+                                                           const int32_t *__restrict__ parent,
+                                                           MS *__restrict__ part) {
+    __shared__ float sm[NT / 64];
+    __shared__ double ss[NT / 64];
+    const int chunk = blockIdx.x, row = blockIdx.y, wave = threadIdx.x >> 6;
     const bool first = row < rows1;
+    if (parent != nullptr) {
+        const int node = first ? row : row - rows1;
+        bool used = false;
+        for (int i = threadIdx.x; i < rows1; i += NT) used |= i > node && parent[i] == node;
+        if (!__syncthreads_or(used)) return;
+    }
     const float Tr = first ? ((period > 0 && row % period == period - 1) ? T_last : T1) : T2;
     const float *src = first ? L1 + (size_t)row * V : L2 + (size_t)(row - rows1) * V;
-    const int j0 = chunk * CHUNK;
-    float z[PER];
+    float x[PER];
+    load_chunk(src, chunk, V, -__builtin_huge_valf(), x);
+    float m = x[0];
 #pragma unroll
-    for (int i = 0; i < PER; i++) {
-        const int j = j0 + i * NT + threadIdx.x;
-        z[i] = j < V ? src[j] / Tr : -__builtin_huge_valf();
-    }
-    float m = -__builtin_huge_valf();
+    for (int i = 1; i < PER; i++) m = fmaxf(m, x[i]);
+    m = wave_max_f(m);
+    if ((threadIdx.x & 63) == 0) sm[wave] = m;
+    __syncthreads();
+    m = sm[0];
 #pragma unroll
-    for (int i = 0; i < PER; i++) m = fmaxf(m, z[i]);
+    for (int w = 1; w < NT / 64; w++) m = fmaxf(m, sm[w]);
+    m = fmaxf(m, -__builtin_huge_valf()) / Tr;  // (all NaN: -Inf)
     double s = 0.0;
     if (m > -__builtin_huge_valf()) {
+        const ExpZ E(Tr, m);
+        if (E.fast) {
 #pragma unroll
-        for (int i = 0; i < PER; i++) s += dexp(z[i], m);
+            for (int i = 0; i < PER; i++) s += (double)E.quick(x[i]);
+        } else {
+#pragma unroll 1
+            for (int i = 0; i < PER; i++) {
+                const int j = chunk * CHUNK + entry0(i / 4) + (i & 3);
+                s += E.slow(j < V ? src[j] : -__builtin_huge_valf());
+            }
+        }
     }
-    block_merge_ms(m, s, sh);
-    if (threadIdx.x == 0) part[(size_t)row * nchunk + chunk] = make_ms(m, s);
+    s = wave_sum_d(s);
+    if ((threadIdx.x & 63) == 0) ss[wave] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) part[(size_t)row * nchunk + chunk] = make_ms(m, ((ss[0] + ss[1]) + ss[2]) + ss[3]);
 }
 
-// Sequential merge of a row's chunk partials (chunk order), the loads issued
-// eight at a time.
-__device__ __forceinline__ MS merge_row(const MS *part, int nchunk) {
-    float m = -__builtin_huge_valf();
-    double s = 0.0;
-    for (int c = 0; c < nchunk; c += 8) {
-        MS v[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = part[min(c + j, nchunk - 1)];
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-            if (c + j < nchunk) merge_ms(m, s, v[j].m, v[j].s);
-    }
-    return make_ms(m, s);
-}
-
-// Merge of a row's chunk partials by one wave: lane l folds chunks l, l+64,
-// ... in order, then the butterfly.
-__device__ __forceinline__ MS wave_merge_row(const MS *part, int nchunk) {
+// A row's statistics from its chunk partials, by one wave: the maximum, then
+// each partial's sum rescaled to it (one exp a partial). p0, p1: this lane's
+// partials lane and lane + 64 (m = -Inf past the end); chunks past 128 are
+// read here.
+__device__ __forceinline__ MS wave_merge(const MS &p0, const MS &p1, const MS *__restrict__ part, int nchunk) {
     const int lane = threadIdx.x & 63;
-    float m = -__builtin_huge_valf();
+    const float ninf = -__builtin_huge_valf();
+    float m = fmaxf(p0.m, p1.m);
+    for (int c = lane + 128; c < nchunk; c += 64) m = fmaxf(m, part[c].m);
+    m = wave_max_f(m);
     double s = 0.0;
-    for (int c = lane; c < nchunk; c += 64) {
+    if (p0.m > ninf) s = p0.s * rescale(p0.m, m);
+    if (nchunk > 64 && p1.m > ninf) s += p1.s * rescale(p1.m, m);
+    for (int c = lane + 128; c < nchunk; c += 64) {
         const MS p = part[c];
-        merge_ms(m, s, p.m, p.s);
+        if (p.m > ninf) s += p.s * rescale(p.m, m);
     }
-    return wave_merge_pairs(m, s);
+    return make_ms(m, wave_sum_d(s));
+}
+__device__ __forceinline__ MS load_part(const MS *__restrict__ part, int c, int nchunk) {
+    return c < nchunk ? part[c] : make_ms(-__builtin_huge_valf(), 0.0);
 }
 
-__global__ void stats_merge_kernel(const MS *__restrict__ part, int rows, int nchunk, float *__restrict__ zmax,
-                                   float *__restrict__ zsum) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= rows) return;
-    const MS ms = merge_row(part + (size_t)r * nchunk, nchunk);
-    zmax[r] = ms.m;
-    zsum[r] = (float)ms.s;
+// One wave per row.
+__global__ __launch_bounds__(NT) void stats_merge_kernel(const MS *__restrict__ part, int rows, int nchunk,
+                                                         float *__restrict__ zmax, float *__restrict__ zsum) {
+    const int r = blockIdx.x * (NT / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (r >= rows) return;  // (whole waves)
+    const MS *p = part + (size_t)r * nchunk;
+    const MS ms = wave_merge(load_part(p, lane, nchunk), load_part(p, lane + 64, nchunk), p, nchunk);
+    if (lane == 0) {
+        zmax[r] = ms.m;
+        zsum[r] = (float)ms.s;
+    }
 }
 
 // Sampling distribution of one draw of a verify step, set by the ratio
@@ -283,10 +337,7 @@ __device__ void decide_block(const float *__restrict__ tgt, const float *__restr
             const int r = min(r0 + b * DECIDE_WAVES, nrows - 1);
             const MS *row = r <= k ? Pt + (size_t)r * nchunk : Pd + (size_t)(r - k - 1) * nchunk;
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int c = lane + 64 * h;
-                pv[b][h] = c < nchunk ? row[c] : make_ms(-__builtin_huge_valf(), 0.0);
-            }
+            for (int h = 0; h < 2; h++) pv[b][h] = load_part(row, lane + 64 * h, nchunk);
         }
         if (r0 == 0 && has0 && x0 >= 0 && x0 < V) {
             lx0 = Lt[(size_t)lane * V + x0];
@@ -296,16 +347,8 @@ __device__ void decide_block(const float *__restrict__ tgt, const float *__restr
         for (int b = 0; b < 8; b++) {
             const int r = r0 + b * DECIDE_WAVES;
             if (r >= nrows) break;
-            MS v;
-            if (nchunk <= 128) {
-                float m = -__builtin_huge_valf();
-                double sm = 0.0;
-                merge_ms(m, sm, pv[b][0].m, pv[b][0].s);
-                merge_ms(m, sm, pv[b][1].m, pv[b][1].s);
-                v = wave_merge_pairs(m, sm);
-            } else {
-                v = wave_merge_row(r <= k ? Pt + (size_t)r * nchunk : Pd + (size_t)(r - k - 1) * nchunk, nchunk);
-            }
+            const MS v = wave_merge(pv[b][0], pv[b][1],
+                                    r <= k ? Pt + (size_t)r * nchunk : Pd + (size_t)(r - k - 1) * nchunk, nchunk);
             if (lane == 0) ms[r] = v;
         }
     }
@@ -396,49 +439,62 @@ __device__ void decide_block(const float *__restrict__ tgt, const float *__restr
     __syncthreads();
 }
 
-// Sampling weights of the PER x NT entries of chunk c: thread t holds entries
-// c * CHUNK + r * NT + t (r < PER) of w and, for the standard residual, of p.
-// Per round r: wave inclusive scans, round total R_r = ((T0 + T1) + T2) + T3
-// of the four wave totals.
-struct ChunkScan {
-    double cw[PER];  // wave-inclusive scans of the weights
-    double R[PER];   // round totals (uniform)
-};
-
-__device__ void chunk_scan(const Decision &D, const float *lt, const float *ld, int V, int c, bool use_p,
-                           ChunkScan &cs, double *sh /* [PER][4] */) {
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-    // every load of the chunk in flight before any arithmetic
-    float lv[PER], dv[PER];
+// Sampling weights of the thread's PER entries of chunk c (load_chunk's
+// order): p (use_p, kind 0) or the residual.
+__device__ __forceinline__ void chunk_weights(const Decision &D, const float *__restrict__ lt,
+                                              const float *__restrict__ ld, int V, int c, bool use_p,
+                                              double (&w)[PER]) {
+    // (no fma of the two products: equal rows leave a residual of exactly 0)
+#pragma clang fp contract(off)
     const bool need_q = !use_p && D.kind == 1;
+    float x[PER], y[PER];
+    load_chunk(lt, c, V, -__builtin_huge_valf(), x);
+    if (need_q) load_chunk(ld, c, V, -__builtin_huge_valf(), y);
+    const ExpZ P(D.Tp, D.mp);
+    if (P.fast) {
 #pragma unroll
-    for (int r = 0; r < PER; r++) {
-        const int j = min(c * CHUNK + r * NT + t, V - 1);
-        lv[r] = lt[j];
-        dv[r] = need_q ? ld[j] : 0.f;
+        for (int i = 0; i < PER; i++) w[i] = (double)P.quick(x[i]) * D.isp;
+    } else {
+#pragma unroll
+        for (int i = 0; i < PER; i++) w[i] = P.slow(x[i]) * D.isp;
     }
+    if (need_q) {
+        const ExpZ Q(D.Tq, D.mq);
+        if (Q.fast) {
 #pragma unroll
-    for (int r = 0; r < PER; r++) {
-        const int j = c * CHUNK + r * NT + t;
-        double w = 0.0;
-        if (j < V) {
-            const double p = dexp(lv[r] / D.Tp, D.mp) * D.isp;
-            if (use_p || D.kind == 0) w = p;
-            else w = fmax(p - (D.kind == 1 ? dexp(dv[r] / D.Tq, D.mq) * D.isq : D.qs), 0.0);
+            for (int i = 0; i < PER; i++) w[i] = fmax(w[i] - (double)Q.quick(y[i]) * D.isq, 0.0);
+        } else {
+#pragma unroll
+            for (int i = 0; i < PER; i++) w[i] = fmax(w[i] - Q.slow(y[i]) * D.isq, 0.0);
         }
-        cs.cw[r] = wave_scan(w);
-        if (lane == 63) sh[r * 4 + wave] = cs.cw[r];
-    }
-    __syncthreads();
+    } else if (!use_p && D.kind == 2) {
 #pragma unroll
-    for (int r = 0; r < PER; r++) cs.R[r] = ((sh[r * 4] + sh[r * 4 + 1]) + sh[r * 4 + 2]) + sh[r * 4 + 3];
+        for (int i = 0; i < PER; i++) w[i] = fmax(w[i] - D.qs, 0.0);
+    }
+    if ((c + 1) * CHUNK > V) {  // (a scalar q or a NaN row would leave weights past the end)
+#pragma unroll
+        for (int i = 0; i < PER; i++)
+            if (c * CHUNK + entry0(i / 4) + (i & 3) >= V) w[i] = 0.0;
+    }
+}
+
+// The chunk's sum of weights (sh: NT / 64 doubles; ends with the sum in
+// every thread, sh free again).
+__device__ __forceinline__ double chunk_sum(const double (&w)[PER], double *sh) {
+    double s = 0.0;
+#pragma unroll
+    for (int r = 0; r < PR; r++) s += (w[4 * r] + w[4 * r + 1]) + (w[4 * r + 2] + w[4 * r + 3]);
+    s = wave_sum_d(s);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
     __syncthreads();
+    s = ((sh[0] + sh[1]) + sh[2]) + sh[3];
+    __syncthreads();
+    return s;
 }
 
 // The decision of verify step `step` (decide_block, computed by every
 // workgroup; the first one publishes it), then csum[step][slot][c] = the
-// sum of w over chunk c: the sequential sum of its round totals (grid: x
-// chunk, y step, z draw slot).
+// sum of w over chunk c (grid: x chunk, y step, z draw slot).
 __global__ __launch_bounds__(NT) void decide_sum_kernel(const float *__restrict__ tgt, const float *__restrict__ drf,
                                                         const int32_t *__restrict__ draft_tok, int k, int V, float T,
                                                         const float *__restrict__ u_acc,
@@ -448,7 +504,7 @@ __global__ __launch_bounds__(NT) void decide_sum_kernel(const float *__restrict_
                                                         const int32_t *__restrict__ bonus_pre,
                                                         int32_t *__restrict__ out_tok, int32_t *__restrict__ out_n,
                                                         Decision *__restrict__ dec, double *__restrict__ csum) {
-    __shared__ double sh[PER * 4];
+    __shared__ double sh[NT / 64];
     __shared__ MS ms[DECIDE_MAX_ROWS];
     __shared__ Decision s_dec[2];
     const int c = blockIdx.x, step = blockIdx.y;
@@ -459,123 +515,126 @@ __global__ __launch_bounds__(NT) void decide_sum_kernel(const float *__restrict_
     if (D.kind < 0 || D.kind == 3) return;
     const float *lt = tgt + ((size_t)step * (k + 1) + D.prow) * V;
     const float *ld = D.kind == 1 ? drf + ((size_t)step * k + D.qrow) * V : nullptr;
-    ChunkScan cs;
-    chunk_scan(D, lt, ld, V, c, false, cs, sh);
-    double sw = 0.0;
-#pragma unroll
-    for (int r = 0; r < PER; r++) sw += cs.R[r];
+    double w[PER];
+    chunk_weights(D, lt, ld, V, c, false, w);
+    const double sw = chunk_sum(w, sh);
     if (threadIdx.x == 0) csum[slot * nchunk + c] = sw;
 }
 
-// First j with u * S <= C_j, where C_j = before(chunk) + (P_r + (off_w +
-// scan)): chunk prefix, then round prefix, then lane. When the weights sum
-// to zero the standard mode draws from p (its chunk sums are formed here, in
-// the same order), the reference mode returns V - 1.
+// First j with u * S <= C_j: the chunk by a prefix over the chunk sums (a
+// wave scan, repeated by every wave: 64 chunks a round), then the entry by
+// scans inside the chunk, C_j = before(chunk) + (the sums of the rounds
+// before it in the chunk) + (the lanes before it, then its own entries).
+// When the weights sum to zero the standard mode draws from p (its chunk
+// sums are formed here), the reference mode returns V - 1; so does a u * S
+// no chunk reaches (NaN weights, u above 1).
 constexpr int MAX_CHUNKS = 1024;
 __global__ __launch_bounds__(NT) void sample_kernel(const float *__restrict__ tgt, const float *__restrict__ drf,
                                                     int k, int V, const Decision *__restrict__ dec, int nchunk,
                                                     const double *__restrict__ csum,
                                                     const int32_t *__restrict__ bonus_pre,
                                                     int32_t *__restrict__ out_tok) {
-    __shared__ double sh[PER * 4];
+    __shared__ double sh[PER];
     __shared__ double s_psum[MAX_CHUNKS];
-    __shared__ double s_csum[MAX_CHUNKS];
-    __shared__ double s_before, s_target;
-    __shared__ int s_chunk, s_usep, s_tok;
-    __shared__ int s_first[NT / 64];
+    __shared__ int s_hit[NT / 64], s_last[NT / 64];
     const int step = blockIdx.x, t = threadIdx.x, wave = t >> 6, lane = t & 63;
     const size_t slot = (size_t)step * gridDim.y + blockIdx.y;
+    const double *cw = csum + slot * nchunk;
+    double c0 = lane < nchunk ? cw[lane] : 0.0;  // (a slot without a draw: read, not used)
     const Decision D = dec[slot];
     if (D.kind < 0) return;
+    int32_t *out = out_tok + (size_t)step * (k + 1) + D.pos;
     if (D.kind == 3) {
-        if (t == 0) out_tok[(size_t)step * (k + 1) + D.pos] = bonus_pre[step];
+        if (t == 0) *out = bonus_pre[step];
         return;
     }
-    const double *cw = csum + slot * nchunk;
     const float *lt = tgt + ((size_t)step * (k + 1) + D.prow) * V;
     const float *ld = D.kind == 1 ? drf + ((size_t)step * k + D.qrow) * V : nullptr;
-    for (int c = t; c < nchunk; c += NT) s_csum[c] = cw[c];
-    __syncthreads();
-    if (t == 0) {
-        double S = 0.0;
-        for (int c = 0; c < nchunk; c++) S += s_csum[c];
-        s_usep = 0;
-        s_tok = -1;
-        if (!(S > 0.0)) {
-            if (D.fallback == 1) s_usep = 1;
-            else s_tok = V - 1;
+    const double *src = cw;
+    bool usep = false;
+    // the running sum through chunk b + lane, given the sum before chunk b
+    auto round = [&](int b, double carry) {
+        const int c = b + lane;
+        return carry + wave_scan(b == 0 ? c0 : c < nchunk ? src[c] : 0.0);
+    };
+    auto total = [&]() {
+        double carry = 0.0;
+        for (int b = 0; b < nchunk; b += 64) carry = __shfl(round(b, carry), 63);
+        return carry;
+    };
+    double w[PER];
+    double S = total();
+    if (!(S > 0.0)) {
+        if (D.fallback != 1) {
+            if (t == 0) *out = V - 1;
+            return;
         }
-    }
-    __syncthreads();
-    if (s_tok >= 0) {
-        if (t == 0) out_tok[(size_t)step * (k + 1) + D.pos] = s_tok;
-        return;
-    }
-    const bool usep = s_usep != 0;
-    ChunkScan cs;
-    if (usep) {
+        usep = true;
         for (int c = 0; c < nchunk; c++) {
-            chunk_scan(D, lt, ld, V, c, true, cs, sh);
-            if (t == 0) {
-                double sp = 0.0;
-#pragma unroll
-                for (int r = 0; r < PER; r++) sp += cs.R[r];
-                s_psum[c] = sp;
-            }
+            chunk_weights(D, lt, ld, V, c, true, w);
+            const double sp = chunk_sum(w, sh);
+            if (t == 0) s_psum[c] = sp;
         }
         __syncthreads();
+        src = s_psum;
+        c0 = lane < nchunk ? s_psum[lane] : 0.0;
+        S = total();
     }
-    if (t == 0) {
-        double S = 0.0;
-        for (int c = 0; c < nchunk; c++) S += usep ? s_psum[c] : s_csum[c];
-        const double target = (double)D.u * S;
-        double before = 0.0;
-        int chunk = nchunk - 1;
-        for (int c = 0; c < nchunk; c++) {
-            const double nb = before + (usep ? s_psum[c] : s_csum[c]);
-            if (target <= nb) { chunk = c; break; }
-            before = nb;
+    const double target = (double)D.u * S;
+    double before = 0.0;
+    int c = -1;
+    for (int b = 0; b < nchunk && c < 0; b += 64) {
+        const double cum = round(b, before);
+        const uint64_t hit = __ballot(b + lane < nchunk && target <= cum);
+        const int f = hit ? __ffsll((unsigned long long)hit) - 1 : 64;
+        if (f > 0) before = __shfl(cum, f - 1);
+        if (f < 64) c = b + f;
+    }
+    if (c < 0) {
+        if (t == 0) *out = V - 1;
+        return;
+    }
+    chunk_weights(D, lt, ld, V, c, usep, w);
+    double inc[PR];  // inclusive scans over the lanes of the rounds' sums
+#pragma unroll
+    for (int r = 0; r < PR; r++) {
+        inc[r] = wave_scan((w[4 * r] + w[4 * r + 1]) + (w[4 * r + 2] + w[4 * r + 3]));
+        if (lane == 63) sh[wave * PR + r] = inc[r];
+    }
+    __syncthreads();
+    for (int i = 0; i < wave * PR; i++) before += sh[i];
+    int hit = CHUNK, last = -1;
+#pragma unroll
+    for (int r = 0; r < PR; r++) {
+        double run = __shfl_up(inc[r], 1);
+        if (lane == 0) run = 0.0;
+        const int j = entry0(r);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            run += w[4 * r + e];
+            if (target <= before + run && hit == CHUNK) hit = j + e;
+            if (w[4 * r + e] > 0.0) last = j + e;
         }
-        s_before = before;
-        s_target = target;
-        s_chunk = chunk;
+        before += sh[wave * PR + r];
     }
-    __syncthreads();
-    const int c = s_chunk;
-    const double before = s_before, target = s_target;
-    chunk_scan(D, lt, ld, V, c, usep, cs, sh);
-    // round: first r with target <= before + P_{r+1}
-    double P = 0.0, Pr = 0.0;
-    int rr = -1;
-#pragma unroll
-    for (int r = 0; r < PER; r++) {
-        const double Pn = P + cs.R[r];
-        if (rr < 0 && target <= before + Pn) { rr = r; Pr = P; }
-        P = Pn;
+    for (int o = 32; o > 0; o >>= 1) {
+        hit = min(hit, __shfl_xor(hit, o));
+        last = max(last, __shfl_xor(last, o));
     }
-    if (rr < 0) {  // unreachable: the chunk total bounds the target
-        rr = PER - 1;
-        Pr = P - cs.R[PER - 1];
+    if (lane == 0) {
+        s_hit[wave] = hit;
+        s_last[wave] = last;
     }
-    double cw_rr = 0.0;
-#pragma unroll
-    for (int r = 0; r < PER; r++)
-        if (r == rr) cw_rr = cs.cw[r];
-    if (lane == 63) sh[wave] = cw_rr;
-    __syncthreads();
-    double off = 0.0;
-    for (int w = 0; w < wave; w++) off += sh[w];
-    const double C = before + (Pr + (off + cw_rr));
-    const int j = c * CHUNK + rr * NT + t;
-    const bool hit = j < V && target <= C;
-    const uint64_t m = __ballot(hit);
-    if (lane == 0) s_first[wave] = m ? (wave * 64 + __ffsll((unsigned long long)m) - 1) : NT;
     __syncthreads();
     if (t == 0) {
-        int f = NT;
-        for (int w = 0; w < NT / 64; w++) f = min(f, s_first[w]);
-        const int tok = min(c * CHUNK + rr * NT + (f < NT ? f : NT - 1), V - 1);
-        out_tok[(size_t)step * (k + 1) + D.pos] = tok;
+        // (the scan inside the chunk can end a rounding step below the sum
+        // that selected it: then the chunk's last entry of positive weight)
+        int h = CHUNK, l = -1;
+        for (int i = 0; i < NT / 64; i++) {
+            h = min(h, s_hit[i]);
+            l = max(l, s_last[i]);
+        }
+        *out = min(c * CHUNK + (h < CHUNK ? h : l >= 0 ? l : CHUNK - 1), V - 1);
     }
 }
 
@@ -621,71 +680,163 @@ __global__ __launch_bounds__(NT) void argmax_partial_kernel(const float *__restr
     }
 }
 
-__global__ void greedy_kernel(const float2 *__restrict__ part, int nchunk, const int32_t *__restrict__ draft_tok,
-                              int steps, int k, int32_t *__restrict__ out_n, int32_t *__restrict__ out_argmax) {
-    const int step = blockIdx.x * blockDim.x + threadIdx.x;
-    if (step >= steps) return;
+// One wave per step: each row's first argmax over its chunks (lane l takes
+// chunks l, l + 64, ..), then the matching prefix of the drafts.
+__global__ __launch_bounds__(64) void greedy_kernel(const float2 *__restrict__ part, int nchunk,
+                                                    const int32_t *__restrict__ draft_tok, int k,
+                                                    int32_t *__restrict__ out_n, int32_t *__restrict__ out_argmax) {
+    const int step = blockIdx.x, lane = threadIdx.x;
     int n = 0;
     bool go = true;
+#pragma unroll 4
     for (int i = 0; i <= k; i++) {
         const float2 *p = part + ((size_t)step * (k + 1) + i) * nchunk;
-        float bv = p[0].x;
-        int bi = __float_as_int(p[0].y);
-        for (int c = 1; c < nchunk; c++)  // chunks ascend: the strict order keeps the first
-            if (beats(p[c].x, bv)) { bv = p[c].x; bi = __float_as_int(p[c].y); }
-        if (out_argmax) out_argmax[(size_t)step * (k + 1) + i] = bi;
+        float bv = -__builtin_huge_valf();
+        int bi = 0x7fffffff;
+        for (int c = lane; c < nchunk; c += 64) {
+            const float2 v = p[c];
+            if (first_of(v.x, __float_as_int(v.y), bv, bi)) { bv = v.x; bi = __float_as_int(v.y); }
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            const float v2 = __shfl_xor(bv, o);
+            const int i2 = __shfl_xor(bi, o);
+            if (first_of(v2, i2, bv, bi)) { bv = v2; bi = i2; }
+        }
+        if (out_argmax && lane == 0) out_argmax[(size_t)step * (k + 1) + i] = bi;
         if (i < k && go) {
             if (bi == draft_tok[(size_t)step * k + i]) n++;
             else go = false;
         }
     }
-    out_n[step] = n;
+    if (lane == 0) out_n[step] = n;
 }
 
-// Tree walk: the workgroup first merges the statistics of every row (target
-// rows then draft rows) into ms, then tests every node in parallel (the test
-// of node i reads only its parent's rows and its own token: pass = u_i <
-// min(1, p/q)), then one thread walks the nodes in index order (parent[i] <
-// i) with integers only: st[i] = depth of i if i and all its ancestors
-// passed, else -1; the deepest accepted node, smallest index on ties, ends
-// the path. Node state lives in LDS up to TREE_LDS nodes (in the workspace
-// beyond that).
+// Tree walk by one workgroup: the statistics of every parent's target and
+// draft row are merged (one wave a row) into ms, then every node is tested in
+// parallel (the test of node i reads only its parent's rows and its own
+// token: pass = u_i < min(1, p/q)), then its depth, or that it or an
+// ancestor failed, comes from pointer jumping over the parents (parent[i] <
+// i; log2 of the depth rounds): dep[i] sums 1 per node that passed and
+// TREE_FAIL per failure from i to its ancestor anc[i]. The deepest accepted
+// node, smallest index on ties, ends the path. Node state lives in LDS up to
+// TREE_LDS nodes; a larger tree is walked by one thread from the workspace.
+// (One thread walking 64 nodes in LDS, each row merged by one thread: 29 us;
+// now TBD us.)
+constexpr int TREE_NT = 1024;
 constexpr int TREE_LDS = 4096;
-__global__ __launch_bounds__(NT) void tree_kernel(const float *__restrict__ tgt, const float *__restrict__ drf,
-                                                  const int32_t *__restrict__ tok, const int32_t *__restrict__ parent,
-                                                  int n, int V, float T, const float *__restrict__ u,
-                                                  const MS *__restrict__ part, int nchunk, MS *__restrict__ ms,
-                                                  int32_t *__restrict__ out_path, int32_t *__restrict__ out_len,
-                                                  int32_t *__restrict__ wsi) {
-    __shared__ int32_t s_par[TREE_LDS], s_st[TREE_LDS];
-    __shared__ int8_t s_pass[TREE_LDS];
+constexpr int TREE_FAIL = -(1 << 24);
+__global__ __launch_bounds__(TREE_NT) void tree_kernel(const float *__restrict__ tgt, const float *__restrict__ drf,
+                                                       const int32_t *__restrict__ tok,
+                                                       const int32_t *__restrict__ parent, int n, int V, float T,
+                                                       const float *__restrict__ u, const MS *__restrict__ part,
+                                                       int nchunk, MS *__restrict__ ms,
+                                                       int32_t *__restrict__ out_path, int32_t *__restrict__ out_len,
+                                                       int32_t *__restrict__ wsi) {
+    constexpr int NPT = TREE_LDS / TREE_NT;
+    __shared__ int32_t s_par[TREE_LDS], s_anc[TREE_LDS], s_dep[TREE_LDS];
+    __shared__ uint8_t s_used[TREE_LDS];
+    __shared__ int s_best[TREE_NT / 64];
+    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
     const bool in_lds = n <= TREE_LDS;
-    int32_t *par = in_lds ? s_par : wsi;
-    int32_t *st = in_lds ? s_st : wsi + n;
-    int8_t *pass = in_lds ? s_pass : (int8_t *)(wsi + 2 * n);
-    for (int r = threadIdx.x; r < 2 * n; r += blockDim.x) ms[r] = merge_row(part + (size_t)r * nchunk, nchunk);
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const int p = parent[i];
-        const int x = tok[i];
-        par[i] = p;
-        int8_t r = 1;  // (the root is accepted)
-        if (i > 0) {
-            if (p < 0 || p >= i || x < 0 || x >= V) {
-                r = -1;  // malformed node: reported as out_len = -1
-            } else {
-                const MS pt = ms[p];
-                const MS pd = ms[n + p];
-                const double pp = dexp(tgt[(size_t)p * V + x] / T, pt.m) / pt.s;
-                const double qq = dexp(drf[(size_t)p * V + x] / T, pd.m) / pd.s;
-                const double ratio = qq > 0.0 ? fmin(1.0, pp / qq) : 1.0;
-                r = (double)u[i] < ratio ? 1 : 0;
-            }
+    if (in_lds) {
+        for (int i = t; i < n; i += TREE_NT) s_used[i] = 0;
+        __syncthreads();
+        for (int i = t; i < n; i += TREE_NT) {
+            const int p = i > 0 ? parent[i] : 0;
+            s_par[i] = p;
+            if (i > 0 && p >= 0 && p < i) s_used[p] = 1;
         }
-        pass[i] = r;
+        __syncthreads();
+    }
+    for (int r = wave; r < 2 * n; r += TREE_NT / 64) {
+        if (in_lds && !s_used[r < n ? r : r - n]) continue;
+        const MS *p = part + (size_t)r * nchunk;
+        const MS v = wave_merge(load_part(p, lane, nchunk), load_part(p, lane + 64, nchunk), p, nchunk);
+        if (lane == 0) ms[r] = v;
     }
     __syncthreads();
-    if (threadIdx.x != 0) return;
+    // 1 passed, 0 failed, -1 malformed
+    auto test = [&](int i, int p) {
+        if (i == 0) return 1;  // (the root is accepted)
+        const int x = tok[i];
+        if (p < 0 || p >= i || x < 0 || x >= V) return -1;
+        const MS pt = ms[p];
+        const MS pd = ms[n + p];
+        const double pp = dexp(tgt[(size_t)p * V + x] / T, pt.m) / pt.s;
+        const double qq = dexp(drf[(size_t)p * V + x] / T, pd.m) / pd.s;
+        const double ratio = qq > 0.0 ? fmin(1.0, pp / qq) : 1.0;
+        return (double)u[i] < ratio ? 1 : 0;
+    };
+    if (in_lds) {
+        int dep[NPT], anc[NPT];
+        bool bad = false, more = false;
+#pragma unroll
+        for (int j = 0; j < NPT; j++) {
+            const int i = t + j * TREE_NT;
+            dep[j] = 0;
+            anc[j] = 0;
+            if (i < n && i > 0) {
+                const int p = s_par[i], r = test(i, p);
+                bad |= r < 0;
+                dep[j] = r > 0 ? 1 : TREE_FAIL;
+                anc[j] = r < 0 ? 0 : p;
+                more |= anc[j] != 0;
+            }
+        }
+        if (__syncthreads_or(bad)) {
+            if (t == 0) *out_len = -1;
+            return;
+        }
+        while (__syncthreads_or(more)) {
+#pragma unroll
+            for (int j = 0; j < NPT; j++) {
+                const int i = t + j * TREE_NT;
+                if (i < n) {
+                    s_dep[i] = dep[j];
+                    s_anc[i] = anc[j];
+                }
+            }
+            __syncthreads();
+            more = false;
+#pragma unroll
+            for (int j = 0; j < NPT; j++) {
+                const int a = anc[j];
+                if (a != 0) {
+                    dep[j] = max(dep[j] + s_dep[a], TREE_FAIL);
+                    anc[j] = s_anc[a];
+                    more |= anc[j] != 0;
+                }
+            }
+        }
+        int best = 0;  // depth * TREE_LDS + (TREE_LDS - 1 - index), at least the root's
+#pragma unroll
+        for (int j = 0; j < NPT; j++) {
+            const int i = t + j * TREE_NT;
+            if (i < n && dep[j] >= 0) best = max(best, dep[j] * TREE_LDS + (TREE_LDS - 1 - i));
+        }
+        for (int o = 32; o > 0; o >>= 1) best = max(best, __shfl_xor(best, o));
+        if (lane == 0) s_best[wave] = best;
+        __syncthreads();
+        if (t != 0) return;
+        for (int w = 1; w < TREE_NT / 64; w++) best = max(best, s_best[w]);
+        const int len = best / TREE_LDS + 1;
+        int v = TREE_LDS - 1 - best % TREE_LDS;
+        for (int d = len - 1; d >= 0; d--) {
+            out_path[d] = v;
+            v = d > 0 ? s_par[v] : 0;
+        }
+        *out_len = len;
+        return;
+    }
+    int32_t *par = wsi, *st = wsi + n;
+    int8_t *pass = (int8_t *)(wsi + 2 * n);
+    for (int i = t; i < n; i += TREE_NT) {
+        const int p = parent[i];
+        par[i] = p;
+        pass[i] = (int8_t)test(i, p);
+    }
+    __syncthreads();
+    if (t != 0) return;
     st[0] = 0;
     int best = 0;
     for (int i = 1; i < n; i++) {
@@ -720,13 +871,14 @@ hipError_t launch_stats(const float *L, int rows, int V, float T, float T_last, 
                         hipStream_t st) {
     if (rows <= 0) return hipSuccess;
     const int nc = accept_nchunk(V);
-    stats_partial_kernel<<<dim3(nc, rows), NT, 0, st>>>(L, rows, T, T_last, period, L, T, V, nc, (MS *)part);
+    stats_partial_kernel<<<dim3(nc, rows), NT, 0, st>>>(L, rows, T, T_last, period, L, T, V, nc, nullptr,
+                                                             (MS *)part);
     return hipGetLastError();
 }
 
 hipError_t launch_stats_merge(const void *part, int rows, int V, float *zmax, float *zsum, hipStream_t st) {
     const int nc = accept_nchunk(V);
-    stats_merge_kernel<<<(rows + 63) / 64, 64, 0, st>>>((const MS *)part, rows, nc, zmax, zsum);
+    stats_merge_kernel<<<(rows + NT / 64 - 1) / (NT / 64), NT, 0, st>>>((const MS *)part, rows, nc, zmax, zsum);
     return hipGetLastError();
 }
 
@@ -751,7 +903,7 @@ hipError_t launch_spec_accept(const float *tgt, const float *drf, const int32_t 
     Decision *dec = (Decision *)(part + (size_t)steps * (2 * k + 1) * nc);
     double *csum = (double *)(dec + (size_t)steps * nd);
     stats_partial_kernel<<<dim3(nc, steps * (2 * k + 1)), NT, 0, st>>>(tgt, steps * (k + 1), Tr, T, k + 1,
-                                                                      drf, Tr, V, nc, part);
+                                                                      drf, Tr, V, nc, nullptr, part);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     decide_sum_kernel<<<dim3(nc, steps, nd), NT, 0, st>>>(tgt, drf, draft_tok, k, V, T, u_acc, u_res, u_bonus,
@@ -770,7 +922,7 @@ hipError_t launch_argmax_partial(const float *L, int rows, int V, float2 *part, 
 hipError_t launch_greedy(const float2 *part, int V, const int32_t *draft_tok, int steps, int k, int32_t *out_n,
                          int32_t *out_argmax, hipStream_t st) {
     const int nc = accept_nchunk(V);
-    greedy_kernel<<<(steps + 63) / 64, 64, 0, st>>>(part, nc, draft_tok, steps, k, out_n, out_argmax);
+    greedy_kernel<<<steps, 64, 0, st>>>(part, nc, draft_tok, k, out_n, out_argmax);
     return hipGetLastError();
 }
 
@@ -786,9 +938,10 @@ hipError_t launch_tree(const float *tgt, const float *drf, const int32_t *tok, c
     MS *part = (MS *)ws;
     MS *ms = part + (size_t)2 * n * nc;
     int32_t *wsi = (int32_t *)(ms + 2 * n);
-    stats_partial_kernel<<<dim3(nc, 2 * n), NT, 0, st>>>(tgt, n, T, T, 0, drf, T, V, nc, part);
+    stats_partial_kernel<<<dim3(nc, 2 * n), NT, 0, st>>>(tgt, n, T, T, 0, drf, T, V, nc,
+                                                            n <= TREE_FILTER ? parent : nullptr, part);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    tree_kernel<<<1, NT, 0, st>>>(tgt, drf, tok, parent, n, V, T, u, part, nc, ms, out_path, out_len, wsi);
+    tree_kernel<<<1, TREE_NT, 0, st>>>(tgt, drf, tok, parent, n, V, T, u, part, nc, ms, out_path, out_len, wsi);
     return hipGetLastError();
 }
