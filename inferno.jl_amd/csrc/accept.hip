@@ -168,7 +168,7 @@ __device__ __forceinline__ void load_chunk(const float *__restrict__ src, int c,
 // One maximum over the workgroup's raw logits (the division by T > 0 keeps
 // the order), then every exponential against it: no rescaling exp per thread
 // and merge level. Bound by HBM and VALU together: 576 rows of 151936 (350
-// MB) 191 -> TBD us.
+// MB) 191 -> 63 us (5.5 TB/s).
 constexpr int TREE_FILTER = 4 * NT;  // (parents read per workgroup: at most 4 loads a thread)
 __global__ __launch_bounds__(NT) void stats_partial_kernel(const float *__restrict__ L1, int rows1, float T1,
                                                            float T_last, int period, const float *__restrict__ L2,
@@ -721,7 +721,7 @@ __global__ __launch_bounds__(64) void greedy_kernel(const float2 *__restrict__ p
 // node, smallest index on ties, ends the path. Node state lives in LDS up to
 // TREE_LDS nodes; a larger tree is walked by one thread from the workspace.
 // (One thread walking 64 nodes in LDS, each row merged by one thread: 29 us;
-// now TBD us.)
+// now 8 us.)
 constexpr int TREE_NT = 1024;
 constexpr int TREE_LDS = 4096;
 constexpr int TREE_FAIL = -(1 << 24);
