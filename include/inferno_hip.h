@@ -467,12 +467,11 @@ int ihip_sample(const float *logits_dev, int rows, int V, float T, int top_k,
  * aligned; 4104 bytes per 4096 logits of each row plus 49408 per row):
  * plain draws (T > 0, no top-k, top-p or min-p: the speculative defaults)
  * spread each row over workgroups of 4096 logits (their softmax
- * statistics, then the draw inside the round that holds u); so do top-k
- * from 1 to 64 at V <= 262144 (each chunk's top-k, then the row's among
- * them: the tokens of ihip_sample), top-p and / or min-p without top-k
- * (the threshold's histograms merged per row), a larger top-k (its
- * threshold by count, the kept entries compacted, then ihip_sample's
- * candidate draw: its tokens; above 4096, ihip_sample's threshold path),
+ * statistics, then the draw inside the round that holds u); so do top-k up to
+ * 4096 and top-p (each chunk's threshold histogram and candidate list,
+ * then one workgroup per row for the threshold and the draw: with top-k
+ * ihip_sample's tokens; a top-k above 4096 takes ihip_sample's path),
+ * min-p (the chunks' kept sums)
  * and T = 0 (each chunk's first argmax: the tokens of ihip_sample). The
  * same limits and the same softmax_sample
  * (src/ModelCPU.jl:1123-1200) and the same contract: draws match the exact

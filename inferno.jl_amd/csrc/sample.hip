@@ -25,9 +25,9 @@
 //  * the threshold's refinement passes run over the first pass's bucket
 //    gathered into LDS when it holds at most 4096 elements.
 //  * with a workspace, every setting spreads each row over workgroups of
-//    one round (chunk statistics, each chunk's argmax, top-k candidates,
-//    threshold histograms, kept sums or kept entries), and one workgroup
-//    per row finishes each stage from them.
+//    one round (chunk statistics, each chunk's argmax, threshold histograms
+//    and candidate lists, kept sums), and one workgroup per row finishes
+//    each stage from them.
 // Sums and scans are trees, where the reference accumulates sequentially:
 // the drawn token can differ only where u falls within rounding of a CDF
 // step.
@@ -61,12 +61,73 @@ __device__ __forceinline__ float okey_inv(uint32_t k) {
 }
 
 // ---- block primitives (16 waves), fixed reduction trees
+// Cross-lane moves of the butterflies on the VALU: the value of lane l ^ O (O
+// = 8: a rotation by 8 within a row of 16; 4: row shifts by 4, each into the
+// half rows that take it; 2, 1: quad permutes; 32, 16: swap_op). The levels
+// and pairs of the reductions are those of shfl_xor.
+template <int CTRL, int BANKS = 0xF> __device__ __forceinline__ float dpp(float old, float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, old), __builtin_bit_cast(int, v),
+                                                                 CTRL, 0xF, BANKS, false));
+}
+template <int O> __device__ __forceinline__ float lane_xor(float v) {
+    if constexpr (O == 8) return dpp<0x128>(v, v);                              // row_ror:8
+    if constexpr (O == 4) return dpp<0x114, 0xA>(dpp<0x104, 0x5>(v, v), v);     // row_shl:4, row_shr:4
+    if constexpr (O == 2) return dpp<0x4E>(v, v);                               // quad_perm [2,3,0,1]
+    return dpp<0xB1>(v, v);                                                     // quad_perm [1,0,3,2]
+}
+// v of lane l combined with lane l ^ 32 (16): the two halves (rows) of a swap
+// of v with itself hold one operand each.
+template <int O, class F> __device__ __forceinline__ float swap_op(float v, F &&f) {
+    const uint32_t x = __builtin_bit_cast(uint32_t, v);
+    if constexpr (O == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+        return f(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+    } else {
+        const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        return f(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+    }
+}
+template <class F> __device__ __forceinline__ float wave_reduce(float v, F &&f) {
+    v = swap_op<32>(v, f);
+    v = swap_op<16>(v, f);
+    v = f(v, lane_xor<8>(v));
+    v = f(v, lane_xor<4>(v));
+    v = f(v, lane_xor<2>(v));
+    return f(v, lane_xor<1>(v));
+}
 __device__ __forceinline__ float wave_sum(float v) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
+    return wave_reduce(v, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ float wave_max(float v) {
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
+    return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
+}
+// The same over integers (any order gives the same sum).
+template <int O> __device__ __forceinline__ uint32_t lane_xor_u(uint32_t v) {
+    return __builtin_bit_cast(uint32_t, lane_xor<O>(__builtin_bit_cast(float, v)));
+}
+__device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v) {
+    auto join = [](uint32_t lo, uint32_t hi) { return ((unsigned long long)hi << 32) | lo; };
+    const auto l32 = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+    const auto h32 = __builtin_amdgcn_permlane32_swap((uint32_t)(v >> 32), (uint32_t)(v >> 32), false, false);
+    v = join(l32[0], h32[0]) + join(l32[1], h32[1]);
+    const auto l16 = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
+    const auto h16 = __builtin_amdgcn_permlane16_swap((uint32_t)(v >> 32), (uint32_t)(v >> 32), false, false);
+    v = join(l16[0], h16[0]) + join(l16[1], h16[1]);
+    v += join(lane_xor_u<8>((uint32_t)v), lane_xor_u<8>((uint32_t)(v >> 32)));
+    v += join(lane_xor_u<4>((uint32_t)v), lane_xor_u<4>((uint32_t)(v >> 32)));
+    v += join(lane_xor_u<2>((uint32_t)v), lane_xor_u<2>((uint32_t)(v >> 32)));
+    v += join(lane_xor_u<1>((uint32_t)v), lane_xor_u<1>((uint32_t)(v >> 32)));
+    return v;
+}
+// Inclusive scan over the 64 lanes: row shifts inside each row of 16, then
+// the rows' totals (row 0 into 1, 2 into 3; 0 and 1 into 2 and 3).
+__device__ __forceinline__ uint32_t wave_scan_u(uint32_t v) {
+    v += __builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, true);  // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, true);  // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, true);  // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, true);  // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, true);  // row_bcast:15 into rows 1, 3
+    v += __builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, true);  // row_bcast:31 into rows 2, 3
     return v;
 }
 __device__ __forceinline__ int wave_min_i(int v) {
@@ -506,14 +567,87 @@ __device__ __forceinline__ bool above_threshold(float z, int j, float zmax, uint
     return k > tau || (k == tau && j < tie_lim);
 }
 
+// draw_candidates for at most 64 of them, one a lane of one wave: the same
+// values in the same order (a block sum of one wave's values is that wave's
+// sum, a sorted slot the count of the candidates before it), without the
+// ~30 barriers of the block form (sort 21, sums and scans 2-3 each), which
+// were most of an 18 us draw of 40 candidates.
+__device__ void draw_candidates_wave(int n, const SampleArgs &a, float ur, int V, const int *s_cidx, float *s_cp,
+                                     int *s_sort, int32_t *out_row) {
+    const int l = threadIdx.x;
+    // first_cdf_hit over slots 4 l + e of the first 16 lanes
+    auto cdf_hit = [&](const float (&v)[4], float u) {
+        float c[4], run = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            run += v[e];
+            c[e] = run;
+        }
+        float inc = run;
+        for (int o = 1; o < 64; o <<= 1) {
+            const float y = __shfl_up(inc, o);
+            if (l >= o) inc += y;
+        }
+        const float ex = inc - run;
+        int hit = INT_MAX;
+#pragma unroll
+        for (int e = 3; e >= 0; e--)
+            if (4 * l + e < n && u <= ex + c[e]) hit = 4 * l + e;
+        return wave_min_i(hit);
+    };
+    const bool in = l < n;
+    const float z = in ? s_cp[l] : -__builtin_huge_valf();
+    const float zmax = wave_max(z);  // (all lanes)
+    const float w = in ? pexp(z - zmax) : 0.f;
+    const float S = wave_sum(w);
+    float p = in ? w / S : 0.f;
+    float v[4];
+    if (a.top_p < 1.0f) {
+        int rank = 0;
+        for (int j = 0; j < n; j++) {
+            const float pj = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p), j));
+            rank += pj > p || (pj == p && j < l);
+        }
+        if (in) {
+            s_cp[l] = p;
+            s_sort[rank] = l;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = 4 * l + e < n ? s_cp[s_sort[4 * l + e]] : 0.f;
+        const int cut = cdf_hit(v, a.top_p);
+        if (cut != INT_MAX && rank > cut) p = 0.f;
+        const float total = wave_sum(p);
+        if (total > 0.f) p = p / total;
+    }
+    if (a.min_p > 0.f) {
+        const float thr = wave_max(fmaxf(p, 0.f)) * a.min_p;
+        if (p < thr) p = 0.f;
+        const float total = wave_sum(p);
+        if (total > 0.f) p = p / total;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    if (in) s_cp[l] = p;
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = 4 * l + e < n ? s_cp[4 * l + e] : 0.f;
+    const int slot = cdf_hit(v, ur);
+    if (l == 0) *out_row = slot == INT_MAX ? V - 1 : s_cidx[slot];
+}
+
 // The draw over n top-k candidates in LDS in index order (s_cidx: token
 // ids, s_cp: z = L / T; s_sort: scratch), shared by draft_sample_kernel and
 // the spread top-k draw: softmax over the candidates (the rest are
 // exp(-Inf) = 0), top-p by a bitonic sort of their probabilities, min-p,
 // then the inverse CDF in index order.
+// (n <= 64: by wave 0 alone, draw_candidates_wave.)
 __device__ void draw_candidates(int n, const SampleArgs &a, float ur, int V, int *s_cidx, float *s_cp, int *s_sort,
                                 float *s_redf, int *s_redi, int32_t *out_row) {
     const int t = threadIdx.x;
+    if (n <= 64) {
+        if (t < 64) draw_candidates_wave(n, a, ur, V, s_cidx, s_cp, s_sort, out_row);
+        return;
+    }
     // softmax over the candidates (the rest are exp(-Inf) = 0)
     float lm = -__builtin_huge_valf();
     for (int i = t; i < n; i += SNT) lm = fmaxf(lm, s_cp[i]);
@@ -1041,14 +1175,13 @@ __global__ __launch_bounds__(SNT) void draft_sample_kernel(const float *__restri
 
 // Workspace of the spread draws: float2 part[rows][nround] (each round's
 // (max, sum exp(z - max))), then a slot of SLOT_BYTES per round of each row
-// (top-k: float cz[SK_SPREAD], int32 ci[SK_SPREAD], int32 cn; top-p: uint32
-// hist[256], uint64 mass[256]; top-p / min-p: float csum at SLOT_CSUM), then
-// ROW_BYTES per row (top-p: the selection state and the gathered threshold
-// bucket: uint32 keys, float z, int32 index, SK_MAX each).
+// (a threshold: uint64 hist[256], at SLOT_LIST the candidate list; top-p /
+// min-p: float sums at SLOT_CSUM, once the list is no longer read), then
+// ROW_BYTES per row (a threshold: the selection state).
 constexpr int SLOT_BYTES = 4096;
+constexpr int SLOT_LIST = 2048;
 constexpr int SLOT_CSUM = 3072;
-constexpr int ROW_GATHER = 256;
-constexpr size_t ROW_BYTES = ROW_GATHER + (size_t)SK_MAX * 12;
+constexpr size_t ROW_BYTES = 256 + (size_t)SK_MAX * 12;
 struct SpreadWs {
     float2 *part;
     uint8_t *slots, *rows;
@@ -1058,60 +1191,122 @@ struct SpreadWs {
 };
 
 // The row's softmax statistics from its rounds' partials (a fixed order: the
-// same bits in every kernel); false for a degenerate row, whose reference
+// same bits in every kernel, each wave by itself: the sums of 64 rounds at a
+// time, then the sum of those); false for a degenerate row, whose reference
 // probabilities are all NaN (the draw returns the last index): no finite
 // maximum (all -Inf, or a +Inf) or a NaN entry anywhere (a round's sum is
 // NaN then). The reference's top-k keeps a NaN (its descending sortperm
 // puts NaN first) and its maximum is then NaN, so this holds with top-k
 // too. count (a top-k threshold, whose softmax is over the kept entries
 // only): S = 1.
-__device__ bool row_stats(const float2 *pr, int nround, float *s_redf, float &zmax, float &S, bool count = false) {
-    const int t = threadIdx.x;
-    float lm = -__builtin_huge_valf(), nan = 0.f;
-    for (int i = t; i < nround; i += SNT) {
+__device__ bool row_stats(const float2 *pr, int nround, float &zmax, float &S, bool count = false) {
+    const int l = threadIdx.x & 63;
+    const float ninf = -__builtin_huge_valf();
+    const float2 p0 = l < nround ? pr[l] : make_float2(ninf, 0.f);
+    float lm = p0.x;
+    bool nan = p0.y != p0.y;
+    for (int i = l + 64; i < nround; i += 64) {
         const float2 p = pr[i];
         lm = fmaxf(lm, p.x);
-        if (p.y != p.y) nan = 1.f;
+        nan |= p.y != p.y;
     }
-    zmax = block_max(lm, s_redf);
-    const bool has_nan = block_max(nan, s_redf) > 0.f;
-    float ls = 0.f;
-    if (zmax > -__builtin_huge_valf())
-        for (int i = t; i < nround; i += SNT) {
-            const float2 p = pr[i];
-            if (p.x > -__builtin_huge_valf()) ls += p.y * pexp(p.x - zmax);
-        }
-    S = block_sum(ls, s_redf);
-    const bool finite_max = zmax > -__builtin_huge_valf() && zmax < __builtin_huge_valf();
+    zmax = wave_max(lm);
+    const bool has_nan = __ballot(nan) != 0ull;
+    const bool finite_max = zmax > ninf && zmax < __builtin_huge_valf();
     if (count) {
         S = 1.0f;
         return finite_max && !has_nan;
     }
+    float acc = 0.f;
+    if (zmax > ninf)
+        for (int v = 0; 64 * v < nround; v++) {
+            const int i = 64 * v + l;
+            const float2 p = v == 0 ? p0 : i < nround ? pr[i] : make_float2(ninf, 0.f);
+            const float sv = wave_sum(p.x > ninf ? p.y * pexp(p.x - zmax) : 0.f);
+            if (l == v) acc = sv;
+        }
+    S = wave_sum(acc);
     return finite_max && !has_nan && S > 0.f && S < __builtin_huge_valf();
 }
 
-// (max, sum exp(z - max)) of round blockIdx.x of row blockIdx.y: part[row][round].
-__global__ __launch_bounds__(SNT) void chunk_stats_kernel(const float *__restrict__ L, int V, float invT,
-                                                          float2 *__restrict__ part) {
-    __shared__ float s_red[2 * SNW];
-    const int r = blockIdx.x, row = blockIdx.y, nround = gridDim.x;
-    float z[4];
-    bool in;
-    load_round(L + (size_t)row * V, V, r, invT, z, in);
-    float m = -__builtin_huge_valf();
-    if (in)
+// The chunk kernels (one workgroup per round of a row): CNT threads of 16
+// entries. Wave w holds the entries of the one-row kernel's waves 4 w .. 4 w
+// + 3 (v = 4 w + r: entries 256 v + 4 lane + e), so a sum over r = one of
+// its waves, then over the 16 of them, is block_sum's. (1024 threads of 4
+// entries waited on barriers: 64 rows' statistics 16.8 us, 9.3 with 256.)
+constexpr int CNT = 256;
+constexpr int CNW = CNT / 64;
+constexpr int CR = SROUND / (4 * CNT);  // groups of 4 entries per thread
+__device__ __forceinline__ int chunk_entry(int r) {  // the first entry of group r
+    return (CR * (int)(threadIdx.x >> 6) + r) * 256 + 4 * (int)(threadIdx.x & 63);
+}
+// Round c of a row: z = L * (1 / T), -Inf past V (load_round's values; 16-byte
+// loads at any 4-byte alignment).
+__device__ __forceinline__ void load_chunk(const float *__restrict__ row, int V, int c, float invT, float (&z)[CR][4]) {
+    const float *src = row + (size_t)c * SROUND;
+    const int n = V - c * SROUND;
+    if (n >= SROUND) {
 #pragma unroll
-        for (int e = 0; e < 4; e++) m = fmaxf(m, z[e]);
-    m = block_max(m, s_red);
-    float sw = 0.f;
-    if (in)
+        for (int r = 0; r < CR; r++) __builtin_memcpy(z[r], src + chunk_entry(r), 16);
+    } else {
+#pragma unroll
+        for (int r = 0; r < CR; r++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int j = chunk_entry(r) + e;
+                z[r][e] = j < n ? src[j] : -__builtin_huge_valf();
+            }
+    }
+    if (invT != 1.0f) {
+#pragma unroll
+        for (int r = 0; r < CR; r++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) z[r][e] = z[r][e] * invT;
+    }
+}
+// block_sum of the one-row kernel's 16 waves' values (v[r]: this thread's
+// value in wave CR w + r); the sum in thread 0 (wave 0).
+__device__ __forceinline__ float chunk_sum(float (&v)[CR], float *red /* [SNW] */) {
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+#pragma unroll
+    for (int r = 0; r < CR; r++) {
+        v[r] = wave_sum(v[r]);
+        if (l == 0) red[CR * w + r] = v[r];
+    }
+    __syncthreads();
+    return wave_sum(l < SNW ? red[l] : 0.f);
+}
+
+// (max, sum exp(z - max)) of round blockIdx.x of row blockIdx.y: part[row][round].
+__global__ __launch_bounds__(CNT) void chunk_stats_kernel(const float *__restrict__ L, int V, float invT,
+                                                          float2 *__restrict__ part) {
+    __shared__ float s_m[CNW], s_red[SNW];
+    const int c = blockIdx.x, row = blockIdx.y, nround = gridDim.x;
+    float z[CR][4];
+    load_chunk(L + (size_t)row * V, V, c, invT, z);
+    float m = -__builtin_huge_valf();
+#pragma unroll
+    for (int r = 0; r < CR; r++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) m = fmaxf(m, z[r][e]);
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6] = m;
+    __syncthreads();
+    m = s_m[0];
+#pragma unroll
+    for (int w = 1; w < CNW; w++) m = fmaxf(m, s_m[w]);
+    float sw[CR];
+#pragma unroll
+    for (int r = 0; r < CR; r++) {
+        sw[r] = 0.f;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            if (z[e] != z[e]) sw = __builtin_nanf("");  // (flags the row even when m is -Inf)
-            else if (m > -__builtin_huge_valf()) sw += pexp(z[e] - m);
+            if (z[r][e] != z[r][e]) sw[r] = __builtin_nanf("");  // (flags the row even when m is -Inf)
+            else if (m > -__builtin_huge_valf()) sw[r] += pexp(z[r][e] - m);
         }
-    sw = block_sum(sw, s_red);
-    if (threadIdx.x == 0) part[(size_t)row * nround + r] = make_float2(m, sw);
+    }
+    const float sum = chunk_sum(sw, s_red);
+    if (threadIdx.x == 0) part[(size_t)row * nround + c] = make_float2(m, sum);
 }
 
 // The draw of row blockIdx.x from its rounds' statistics: the row's max and
@@ -1132,7 +1327,7 @@ __global__ __launch_bounds__(SNT) void chunk_draw_kernel(const float *__restrict
     const float ur = u[row];
     const float2 *pr = part + (size_t)row * nround;
     float zmax, S;
-    if (!row_stats(pr, nround, s_redf, zmax, S) || ur != ur) {
+    if (!row_stats(pr, nround, zmax, S) || ur != ur) {
         if (t == 0) out[row] = V - 1;
         return;
     }
@@ -1193,28 +1388,41 @@ __global__ __launch_bounds__(SNT) void chunk_draw_kernel(const float *__restrict
 // (its key and index as float bits) into part[row][chunk], then one
 // workgroup per row takes the first of those; an exact order, so the
 // tokens are the one-workgroup kernel's.
-__global__ __launch_bounds__(SNT) void chunk_argmax_kernel(const float *__restrict__ L, int V,
+__global__ __launch_bounds__(CNT) void chunk_argmax_kernel(const float *__restrict__ L, int V,
                                                            float2 *__restrict__ part) {
-    __shared__ uint32_t s_k[SNW];
-    __shared__ int s_i[SNW];
+    __shared__ uint32_t s_k[CNW];
+    __shared__ int s_i[CNW];
     const int c = blockIdx.x, row = blockIdx.y, t = threadIdx.x, nround = gridDim.x;
-    float z[4];
-    bool in;
-    load_round(L + (size_t)row * V + (size_t)c * SROUND, min(SROUND, V - c * SROUND), 0, 1.0f, z, in);
+    float z[CR][4];
+    load_chunk(L + (size_t)row * V, V, c, 1.0f, z);
     uint32_t bk = 0u;
     int bi = INT_MAX;
-    if (in)
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const uint32_t k = jl_key(z[e]);
-            if (k > bk) {
+    for (int r = 0; r < CR; r++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {  // (the thread's entries in index order)
+            const uint32_t k = jl_key(z[r][e]);
+            const int j = c * SROUND + chunk_entry(r) + e;
+            if (k > bk && j < V) {
                 bk = k;
-                bi = c * SROUND + 4 * t + e;
+                bi = j;
             }
         }
-    uint32_t best;
-    const int first = block_argmax_key(bk, bi, s_k, s_i, &best);
-    if (t == 0) part[(size_t)row * nround + c] = make_float2(__uint_as_float(best), __int_as_float(first));
+    uint32_t best = wave_max_u(bk);
+    int first = wave_min_i(bk == best ? bi : INT_MAX);
+    if ((t & 63) == 0) {
+        s_k[t >> 6] = best;
+        s_i[t >> 6] = first;
+    }
+    __syncthreads();
+    if (t == 0) {
+        for (int w = 1; w < CNW; w++)  // (the waves in index order: the first best stays)
+            if (s_k[w] > best) {
+                best = s_k[w];
+                first = s_i[w];
+            }
+        part[(size_t)row * nround + c] = make_float2(__uint_as_float(best), __int_as_float(first));
+    }
 }
 
 __global__ __launch_bounds__(SNT) void argmax_draw_kernel(int V, const float2 *__restrict__ part,
@@ -1237,450 +1445,553 @@ __global__ __launch_bounds__(SNT) void argmax_draw_kernel(int V, const float2 *_
     if (t == 0) out[row] = first == INT_MAX ? 0 : first;
 }
 
-// Spread top-k (1 <= K <= SK_SPREAD, V <= SPART_ROUNDS rounds): every
-// chunk's own top-K by the one-row kernel's order (the row maximum's bucket,
-// then the key; ties lowest index first), then one workgroup per row picks
-// the row's top-K from the chunks' candidates by the same order. The union
-// of the chunks' top-K holds the row's, and it is in index order, so the
-// draw over the kept candidates is the one-row kernel's.
-constexpr int SK_SPREAD = 64;
+// Spread thresholds: top-k (the k-th largest z, by count) and top-p (where
+// the probability mass from the top reaches top_p), by the one-row kernel's
+// rules (buckets below the row maximum, then the key; ties lowest index
+// first). After the statistics, one launch over the rounds:
+//  * hist[256] of the round: per bucket the count and the 2^-40 mass packed as
+//    mass << 13 | count (one LDS atomic an entry, a copy of the array per
+//    wave). Entries that cannot be kept are left out of it: for top-k <= 256
+//    those in buckets past one whose thread maxima up to it number k (at
+//    least k entries of this round are larger); for top-p <= 1 - 1e-4 those
+//    of probability below (1 - top_p) / (2 V): the mass past the threshold
+//    element exceeds 0.99 (1 - top_p) and no entry there is above it, so it
+//    is at least 0.99 (1 - top_p) / V, ln 1.98 above the cut, more than a
+//    bucket's width: the threshold's bucket is counted in full.
+//  * the candidate list: (z, index) of its entries up to bucket `last`, the
+//    largest that leaves at most LIST_MAX of them, in index order.
+// Then one workgroup per row merges the histograms to the threshold's bucket,
+// takes that bucket's entries from the lists (from the row, for a round whose
+// list ends before it), finds the threshold among them, and draws: top-k
+// over the kept entries (draw_candidates), top-p by the rounds' kept masses
+// (the buckets above the threshold's, plus its kept entries), then inside
+// the round u falls in. Two launches after the statistics where there were
+// two (top-k <= 64), seven (larger) and five (top-p): 64 rows of 151936 at
+// top-p 0.9 95 -> 38 us (histograms 32 -> 14, pick + gather + select + sums +
+// draw 52 -> 15), one row at top-k 40 + top-p 28.5 -> 18.6 us.
+enum : int { SEL_SELECT = 0, SEL_ALL = 1, SEL_DEGEN = 2 };
+struct RowSel {
+    int mode;
+    uint32_t zb, tau;
+    int tie_lim;
+    float zmax, S;
+};
+constexpr int LIST_MAX = 336;  // entries: 16 bytes of header, z[LIST_MAX], uint16 index in the round [LIST_MAX]
+constexpr int CBITS = 13;      // count bits of a packed bucket (a round holds 4096 entries)
+struct ListHead { int n, last; };
 
-// Chunk blockIdx.x of row blockIdx.y: its top-K candidates (z and token id,
-// index order) to cz / ci [row][chunk][SK_SPREAD], their count to cn.
-__global__ __launch_bounds__(SNT) void chunk_topk_kernel(const float *__restrict__ L, int V, float invT, int K,
-                                                         SpreadWs ws) {
-    __shared__ float s_redf[2 * SNW];
-    __shared__ uint32_t s_redu[SNW];
-    __shared__ uint32_t s_hist[256];
-    __shared__ unsigned long long s_mass[256];
-    __shared__ uint32_t s_sel[2];
-    __shared__ unsigned long long s_selm[2];
-    __shared__ uint32_t s_ck[SK_MAX];
-    __shared__ float s_cz[SK_MAX];
-    __shared__ int s_ncnt;
-    const int c = blockIdx.x, row = blockIdx.y, t = threadIdx.x, nround = gridDim.x;
-    const float2 *part = ws.part;
-    float lm = -__builtin_huge_valf();
-    for (int i = t; i < nround; i += SNT) lm = fmaxf(lm, part[(size_t)row * nround + i].x);
-    const float zm = block_max(lm, s_redf);
-    const float *Lc = L + (size_t)row * V + (size_t)c * SROUND;
-    const int Vc = min(SROUND, V - c * SROUND);
-    Select R;
-    select_threshold<false>(Lc, Vc, 1, invT, zm, 1.f, (unsigned long long)K, s_hist, s_mass, s_sel, s_selm, s_ck,
-                            s_cz, &s_ncnt, R);
-    const uint32_t zb = R.zb, tau = R.tau;
-    const int rem = (int)R.rem;
-    float z[4];
-    bool in;
-    load_round(Lc, Vc, 0, invT, z, in);
-    bool g[4], q[4];
-    uint32_t ng = 0, nq = 0;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const uint32_t b = zbin(z[e], zm);
-        const uint32_t k = okey(z[e]);
-        g[e] = in && (R.all || b < zb || (b == zb && k > tau));
-        q[e] = in && !R.all && b == zb && k == tau;
-        ng += g[e];
-        nq += q[e];
+template <bool COUNT>
+__global__ __launch_bounds__(CNT) void chunk_hist_kernel(const float *__restrict__ L, int V, float invT, int top_k,
+                                                         float top_p, SpreadWs ws) {
+    __shared__ unsigned long long s_h[CNW][256];
+    __shared__ uint32_t s_tm[256];
+    __shared__ int s_wn[CNW];
+    const int c = blockIdx.x, row = blockIdx.y, t = threadIdx.x, wave = t >> 6, lane = t & 63;
+    float z[CR][4];
+    load_chunk(L + (size_t)row * V, V, c, invT, z);
+    float zmax, S;
+    const bool ok = row_stats(ws.part + (size_t)row * ws.nround, ws.nround, zmax, S, COUNT);
+    if (c == 0 && t == 0) {
+        RowSel *rs = (RowSel *)ws.rowb(row);
+        rs->mode = ok ? SEL_SELECT : SEL_DEGEN;
+        rs->zmax = zmax;
+        rs->S = S;
     }
-    uint32_t tot;
-    const uint32_t ex = block_excl_scan_u(ng | (nq << 16), s_redu, tot);
-    const int eq_before = (int)(ex >> 16);
-    int pos = (int)(ex & 0xffffu) + min(max(rem, 0), eq_before);
-    int er = eq_before;
-    uint8_t *sl = ws.slot(row, c);
-    float *cz = (float *)sl;
-    int32_t *ci = (int32_t *)(sl + SK_SPREAD * 4);
+    if (!ok) return;  // (the whole workgroup)
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-        if (g[e] || (q[e] && er < rem)) {
-            if (pos < SK_SPREAD) {
-                cz[pos] = z[e];
-                ci[pos] = c * SROUND + 4 * t + e;
-            }
-            pos++;
+    for (int w = 0; w < CNW; w++) s_h[w][t] = 0;
+    const int n = V - c * SROUND;  // entries of the row from this round on
+    float zcut = -__builtin_huge_valf();  // (top-p: entries below it are left out)
+    uint32_t bcut = 255u;                 // (top-k: buckets past it are)
+    // the buckets 4 lane .. 4 lane + 3 of a wave: how many leading buckets
+    // hold at most `most` entries together (every wave by itself)
+    auto leading = [&](const uint32_t (&h)[4], uint32_t most) {
+        uint32_t cum[4], run = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            run += h[j];
+            cum[j] = run;
         }
-        if (q[e]) er++;
+        const uint32_t inc = wave_scan_u(run);
+        int k = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) k += __popcll(__ballot(inc - run + cum[j] <= most));
+        return k;
+    };
+    if constexpr (COUNT) {
+        s_tm[t] = 0;
+        __syncthreads();
+        if (top_k <= CNT) {
+            float tm = z[0][0];
+#pragma unroll
+            for (int r = 0; r < CR; r++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) tm = fmaxf(tm, z[r][e]);
+            if (chunk_entry(0) < n) atomicAdd(&s_tm[zbin(tm, zmax)], 1u);
+            __syncthreads();
+            const uint32_t h[4] = {s_tm[4 * lane], s_tm[4 * lane + 1], s_tm[4 * lane + 2], s_tm[4 * lane + 3]};
+            bcut = min(255, leading(h, (uint32_t)top_k - 1));  // (the first bucket whose prefix reaches k)
+        }
+    } else {
+        if (top_p <= 1.0f - 1e-4f) zcut = zmax + logf(0.5f * (1.0f - top_p) / (float)V * S) - 1e-3f;
+        __syncthreads();
     }
-    if (t == 0)
-        *(int32_t *)(sl + SK_SPREAD * 8) = min((int)(tot & 0xffffu) + min(max(rem, 0), (int)(tot >> 16)), SK_SPREAD);
+    const float invS = 1.0f / S;
+    uint32_t bk[CR][4];
+    bool in[CR][4];
+#pragma unroll
+    for (int r = 0; r < CR; r++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            bk[r][e] = zbin(z[r][e], zmax);
+            in[r][e] = chunk_entry(r) + e < n && (COUNT ? bk[r][e] <= bcut : z[r][e] >= zcut);
+            if (in[r][e])
+                atomicAdd(&s_h[wave][bk[r][e]],
+                          COUNT ? 1ull : (mass_fx(z[r][e], zmax, invS) << CBITS) + 1ull);
+        }
+    __syncthreads();
+    unsigned long long hs = s_h[0][t];
+#pragma unroll
+    for (int w = 1; w < CNW; w++) hs += s_h[w][t];
+    uint8_t *sl = ws.slot(row, c);
+    ((unsigned long long *)sl)[t] = hs;
+    s_tm[t] = (uint32_t)hs & ((1u << CBITS) - 1u);
+    __syncthreads();
+    const uint32_t h[4] = {s_tm[4 * lane], s_tm[4 * lane + 1], s_tm[4 * lane + 2], s_tm[4 * lane + 3]};
+    const int last = leading(h, LIST_MAX) - 1;
+    // places in index order: (wave, group, lane, entry)
+    int pos[CR], wn = 0;
+#pragma unroll
+    for (int r = 0; r < CR; r++) {
+        int before = 0, all = 0;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            in[r][e] = in[r][e] && (int)bk[r][e] <= last;
+            const uint64_t m = __ballot(in[r][e]);
+            before += __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+            all += __popcll(m);
+        }
+        pos[r] = wn + before;
+        wn += all;
+    }
+    if (lane == 0) s_wn[wave] = wn;
+    __syncthreads();
+    int base = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < CNW; w++) {
+        base += w < wave ? s_wn[w] : 0;
+        total += s_wn[w];
+    }
+    uint8_t *ls = sl + SLOT_LIST;
+    if (t == 0) *(ListHead *)ls = ListHead{total, last};
+    float *lz = (float *)(ls + 16);
+    uint16_t *li = (uint16_t *)(ls + 16 + 4 * LIST_MAX);
+#pragma unroll
+    for (int r = 0; r < CR; r++) {
+        int q = base + pos[r];
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (in[r][e]) {  // (total <= LIST_MAX)
+                lz[q] = z[r][e];
+                li[q] = (uint16_t)(chunk_entry(r) + e);
+                q++;
+            }
+    }
 }
 
-// select_threshold over the n slots of z in LDS whose id is >= 0 (MASS
-// off): the bucket of pass A, its keys gathered into ck (n entries), then
-// refine_threshold; R.all when fewer than target.
-__device__ void select_lds(const float *z, const int *id, int n, float zmax, unsigned long long target,
-                           uint32_t *hist, uint32_t *sel, unsigned long long *selm, uint32_t *ck, int *ncnt,
-                           Select &R) {
-    const int t = threadIdx.x;
-    R.zb = 255u;
-    R.tau = 0u;
-    R.rem = target;
-    R.cnt = 0;
-    R.all = false;
-    if (t < 256) hist[t] = 0;
-    if (t == 0) *ncnt = 0;
-    __syncthreads();
-    for (int i = t; i < n; i += SNT)
-        if (id[i] >= 0) atomicAdd(&hist[zbin(z[i], zmax)], 1u);
-    __syncthreads();
-    pick_bucket<false>(hist, nullptr, R.rem, sel, selm, false);
-    __syncthreads();
-    const uint32_t zb = sel[0];
-    const unsigned long long aboveA = selm[0];
-    __syncthreads();
-    if (aboveA == ~0ull) {
-        R.all = true;
-        return;
+// The entries of round c that `keep` takes, in index order, by one wave:
+// f(place from `at` on, z, index), from the round's list when it reaches
+// bucket zb, else from the row.
+template <class K, class F>
+__device__ __forceinline__ void round_entries(const uint8_t *ls, const float *Lr, int V, int c, float invT, int zb,
+                                              uint32_t at, K &&keep, F &&f) {
+    const int lane = threadIdx.x & 63;
+    const ListHead hd = *(const ListHead *)ls;
+    const bool list = zb <= hd.last;
+    const float *lz = (const float *)(ls + 16), *src = Lr + (size_t)c * SROUND;
+    const uint16_t *li = (const uint16_t *)(ls + 16 + 4 * LIST_MAX);
+    const int n = list ? hd.n : min(SROUND, V - c * SROUND);
+#pragma unroll 2
+    for (int i0 = 0; i0 < n; i0 += 64) {
+        const int i = i0 + lane;
+        float z = 0.f;
+        int j = i;
+        if (i < n) {
+            if (list) {
+                z = lz[i];
+                j = li[i];
+            } else {
+                z = src[i];
+                if (invT != 1.0f) z = z * invT;
+            }
+        }
+        j += c * SROUND;
+        const bool k = i < n && keep(z, j);
+        const uint64_t m = __ballot(k);
+        if (k) f(at + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u)), z, j);
+        at += __popcll(m);
     }
-    R.rem -= aboveA;
-    R.zb = zb;
-    for (int i = t; i < n; i += SNT)
-        if (id[i] >= 0 && zbin(z[i], zmax) == zb) ck[atomicAdd(ncnt, 1)] = okey(z[i]);
-    __syncthreads();
-    refine_threshold<false>(nullptr, 0, 0, 1.f, zmax, 1.f, true, *ncnt, hist, nullptr, sel, selm, ck, nullptr, R);
 }
 
-// Row blockIdx.x: the chunks' candidates gathered in index order, the row's
-// top-K among them, then draw_candidates as draft_sample_kernel's top-k path.
-__global__ __launch_bounds__(SNT) void topk_draw_kernel(int V, SampleArgs a, SpreadWs ws, const float *__restrict__ u,
-                                                        int32_t *__restrict__ out) {
+// Row blockIdx.x: its threshold and (draw) its token; otherwise the selection
+// is left in the row's RowSel for the kept sums of a min-p after it.
+template <bool COUNT>
+__global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restrict__ L, int V, float invT,
+                                                            SampleArgs a, bool draw, SpreadWs ws,
+                                                            const float *__restrict__ u, int32_t *__restrict__ out) {
     __shared__ float s_redf[2 * SNW];
     __shared__ uint32_t s_redu[SNW];
     __shared__ int s_redi[SNW];
     __shared__ uint32_t s_hist[256];
+    __shared__ unsigned long long s_mass[256];
     __shared__ uint32_t s_sel[2];
     __shared__ unsigned long long s_selm[2];
-    __shared__ float s_gz[SK_MAX];
-    __shared__ int s_gi[SK_MAX];
-    __shared__ int s_cidx[SK_MAX];
-    __shared__ float s_cp[SK_MAX];
-    __shared__ int s_sort[SK_MAX];
-    __shared__ int s_ncnt;
-    const int row = blockIdx.x, t = threadIdx.x;
-    const int nround = (V + SROUND - 1) / SROUND;
-    const float ur = u[row];
-    // chunk c's candidates at slots c * SK_SPREAD + j (j < its count; id -1
-    // beyond): index order, loaded with the statistics, no offsets needed
-    const int n = nround * SK_SPREAD;  // <= SK_MAX
-    for (int i = t; i < n; i += SNT) {  // (count and slot loaded together: the slot is workspace either way)
-        const int c = i / SK_SPREAD, j = i - c * SK_SPREAD;
-        const uint8_t *sl = ws.slot(row, c);
-        const int cnt = *(const int32_t *)(sl + SK_SPREAD * 8);
-        const float zj = ((const float *)sl)[j];
-        const int ij = ((const int32_t *)(sl + SK_SPREAD * 4))[j];
-        const bool live = j < cnt;
-        s_gz[i] = live ? zj : 0.f;
-        s_gi[i] = live ? ij : -1;
+    __shared__ unsigned long long s_cum[SMAX_ROUNDS];  // per round: the packed kept mass and count
+    __shared__ uint32_t s_off[SMAX_ROUNDS];
+    // the threshold bucket's keys, values and indices; then (top-k) the sort
+    // scratch, values and indices of the kept entries
+    __shared__ uint32_t s_ck[SK_MAX];
+    __shared__ float s_cz[SK_MAX];
+    __shared__ int s_ci[SK_MAX];
+    constexpr unsigned long long CMASK = (1ull << CBITS) - 1ull;
+    const int row = blockIdx.x, t = threadIdx.x, wave = t >> 6, lane = t & 63, nround = ws.nround;
+    const float *Lr = L + (size_t)row * V;
+    RowSel *rs = (RowSel *)ws.rowb(row);
+    // the rounds' histograms, wave w those of rounds w, w + 16, ..: buckets
+    // lane + 64 j; the first HC of them stay in registers
+    constexpr int HC = 4;
+    unsigned long long hv[HC][4];
+    auto load_hist = [&](int c, unsigned long long (&h)[4]) {
+        const unsigned long long *p = (const unsigned long long *)ws.slot(row, c) + lane;
+#pragma unroll
+        for (int j = 0; j < 4; j++) h[j] = c < nround ? p[64 * j] : 0ull;
+    };
+#pragma unroll
+    for (int i = 0; i < HC; i++) load_hist(wave + SNW * i, hv[i]);
+    // f(round, its buckets) over this wave's rounds
+    auto rounds = [&](auto &&f) {
+#pragma unroll
+        for (int i = 0; i < HC; i++)
+            if (wave + SNW * i < nround) f(wave + SNW * i, hv[i]);
+#pragma unroll 1
+        for (int c = wave + SNW * HC; c < nround; c += SNW) {
+            unsigned long long h[4];
+            load_hist(c, h);
+            f(c, h);
+        }
+    };
+    const int mode0 = rs->mode;
+    const float zmax = rs->zmax, S = rs->S;
+    const float ur = draw ? u[row] : 1.f;
+    if (t < 256) {
+        s_hist[t] = 0;
+        s_mass[t] = 0;
     }
-    float lm = -__builtin_huge_valf(), nan = 0.f;
-    for (int i = t; i < nround; i += SNT) {
-        const float2 p = ws.part[(size_t)row * nround + i];
-        lm = fmaxf(lm, p.x);
-        if (p.y != p.y) nan = 1.f;
-    }
-    const float zm = block_max(lm, s_redf);  // (its barriers also publish the slots)
-    if (block_max(nan, s_redf) > 0.f || !(zm > -__builtin_huge_valf() && zm < __builtin_huge_valf()) || ur != ur) {
-        if (t == 0) out[row] = V - 1;  // degenerate row (a NaN is kept by the reference's top-k): NaN probabilities
+    __syncthreads();
+    if (mode0 == SEL_DEGEN || ur != ur) {
+        if (draw && t == 0) out[row] = V - 1;
         return;
     }
     if (!(ur > 0.f)) {  // the reference's draw returns index 1 (here 0) when r <= 0
         if (t == 0) out[row] = 0;
         return;
     }
-    Select R;
-    select_lds(s_gz, s_gi, n, zm, (unsigned long long)a.top_k, s_hist, s_sel, s_selm, (uint32_t *)s_sort, &s_ncnt, R);
-    const uint32_t zb = R.zb, tau = R.tau;
-    const int rem = (int)R.rem;
-    // the kept candidates in index order (slots 4 t .. 4 t + 3: n <= SK_MAX)
-    bool g[4], q[4];
-    uint32_t ng = 0, nq = 0;
+    {
+        uint32_t hc[4] = {0, 0, 0, 0};
+        unsigned long long hm[4] = {0, 0, 0, 0};
+        rounds([&](int, const unsigned long long (&h)[4]) {
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const int j = 4 * t + e;
-        const bool live = j < n && s_gi[j] >= 0;
-        const float z = live ? s_gz[j] : 0.f;
-        const uint32_t b = zbin(z, zm), k = okey(z);
-        g[e] = live && (R.all || b < zb || (b == zb && k > tau));
-        q[e] = live && !R.all && b == zb && k == tau;
-        ng += g[e];
-        nq += q[e];
-    }
-    uint32_t tot;
-    const uint32_t ex = block_excl_scan_u(ng | (nq << 16), s_redu, tot);
-    const int eq_before = (int)(ex >> 16);
-    int pos = (int)(ex & 0xffffu) + min(max(rem, 0), eq_before);
-    int er = eq_before;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const int j = 4 * t + e;
-        if (g[e] || (q[e] && er < rem)) {
-            if (pos < SK_MAX) {
-                s_cidx[pos] = s_gi[j];
-                s_cp[pos] = s_gz[j];
+            for (int j = 0; j < 4; j++) {
+                hc[j] += (uint32_t)(h[j] & CMASK);
+                hm[j] += h[j] >> CBITS;
             }
-            pos++;
-        }
-        if (q[e]) er++;
-    }
-    __syncthreads();
-    const int nk = min((int)(tot & 0xffffu) + min(max(rem, 0), (int)(tot >> 16)), SK_MAX);  // == K
-    draw_candidates(nk, a, ur, V, s_cidx, s_cp, s_sort, s_redf, s_redi, out + row);
-}
-
-// Spread top-p and / or min-p (no top-k): the row's statistics from the chunk
-// partials; for top-p the chunks' pass-A histograms (counts and 2^-40 masses
-// of the buckets below the row maximum) merged per row to the threshold
-// bucket, that bucket's elements gathered in index order, the key passes
-// over them (or over the row when the bucket holds more than SK_MAX), the
-// ties at the threshold kept lowest index first; then each chunk's sum of
-// the kept probabilities and one workgroup per row drawing from those sums,
-// as draft_sample_kernel's whole-row path does (the same threshold rules).
-enum : int { SEL_SELECT = 0, SEL_ALL = 1, SEL_DEGEN = 2 };
-struct RowSel {
-    int mode;
-    uint32_t zb, tau;
-    int tie_lim;
-    unsigned long long rem;
-    int nzb;
-    float zmax, S;
-};
-
-__global__ __launch_bounds__(SNT) void chunk_hist_kernel(const float *__restrict__ L, int V, float invT, bool count,
-                                                         SpreadWs ws) {
-    __shared__ float s_redf[2 * SNW];
-    __shared__ uint32_t s_hist[256];
-    __shared__ unsigned long long s_mass[256];
-    const int c = blockIdx.x, row = blockIdx.y, t = threadIdx.x;
-    float zmax, S;
-    const bool ok = row_stats(ws.part + (size_t)row * ws.nround, ws.nround, s_redf, zmax, S, count);
-    if (t < 256) {
-        s_hist[t] = 0;
-        s_mass[t] = 0;
-    }
-    __syncthreads();
-    if (ok) {
-        const float invS = 1.0f / S;
-        float z[4];
-        bool in;
-        load_round(L + (size_t)row * V + (size_t)c * SROUND, min(SROUND, V - c * SROUND), 0, invT, z, in);
-        if (in)
+        });
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const uint32_t b = zbin(z[e], zmax);
-                atomicAdd(&s_hist[b], 1u);
-                if (!count) atomicAdd(&s_mass[b], mass_fx(z[e], zmax, invS));
+        for (int j = 0; j < 4; j++)
+            if (hc[j]) {
+                atomicAdd(&s_hist[lane + 64 * j], hc[j]);
+                if (!COUNT) atomicAdd(&s_mass[lane + 64 * j], hm[j]);
             }
     }
     __syncthreads();
-    uint8_t *sl = ws.slot(row, c);
-    if (t < 256) {
-        ((uint32_t *)sl)[t] = s_hist[t];
-        ((unsigned long long *)(sl + 1024))[t] = s_mass[t];
-    }
-}
-
-// Row blockIdx.x: the merged histograms, the bucket holding the target mass
-// (top_k > 0: the bucket holding the top_k-th element).
-__global__ __launch_bounds__(SNT) void row_pick_kernel(float top_p, int top_k, SpreadWs ws) {
-    __shared__ float s_redf[2 * SNW];
-    __shared__ uint32_t s_hist[256];
-    __shared__ unsigned long long s_mass[256];
-    __shared__ uint32_t s_sel[2];
-    __shared__ unsigned long long s_selm[2];
-    const int row = blockIdx.x, t = threadIdx.x, nround = ws.nround;
-    RowSel *rs = (RowSel *)ws.rowb(row);
-    float zmax, S;
-    if (!row_stats(ws.part + (size_t)row * nround, nround, s_redf, zmax, S, top_k > 0)) {
-        if (t == 0) rs->mode = SEL_DEGEN;
-        return;
-    }
-    if (t < 256) {
-        s_hist[t] = 0;
-        s_mass[t] = 0;
-    }
-    __syncthreads();
-    {  // bucket t % 256 over every fourth chunk from t / 256 (integer sums: any order)
-        const int b = t & 255;
-        uint32_t h = 0;
-        unsigned long long m = 0;
-#pragma unroll 4
-        for (int c = t >> 8; c < nround; c += SNT / 256) {
-            const uint8_t *sl = ws.slot(row, c);
-            h += ((const uint32_t *)sl)[b];
-            if (top_k == 0) m += ((const unsigned long long *)(sl + 1024))[b];
-        }
-        atomicAdd(&s_hist[b], h);
-        if (top_k == 0) atomicAdd(&s_mass[b], m);
-    }
-    __syncthreads();
-    const float tp = fmaxf(top_p, 0.f) * 1099511627776.0f;
+    const float tp = fmaxf(a.top_p, 0.f) * 1099511627776.0f;
     const unsigned long long target =
-        top_k > 0 ? (unsigned long long)top_k : tp < 1.0f ? 1ull : (unsigned long long)ceilf(tp);
-    if (top_k > 0)
-        pick_bucket<false>(s_hist, nullptr, target, s_sel, s_selm, false);
-    else
-        pick_bucket<true>(s_hist, s_mass, target, s_sel, s_selm, false);
-    __syncthreads();
-    if (t == 0) {
-        const uint32_t zb = s_sel[0];
-        const unsigned long long above = s_selm[0];
-        rs->zmax = zmax;
-        rs->S = S;
-        if (above == ~0ull) {
-            rs->mode = SEL_ALL;
-        } else {
-            rs->mode = SEL_SELECT;
-            rs->zb = zb;
-            rs->rem = target - above;
-            rs->nzb = (int)s_hist[zb];
-        }
-    }
-}
-
-// Chunk blockIdx.x of row blockIdx.y: its elements of the threshold bucket
-// (key, z, index) at their index-order place in the row's gather.
-__global__ __launch_bounds__(SNT) void chunk_gather_kernel(const float *__restrict__ L, int V, float invT, SpreadWs ws) {
-    __shared__ uint32_t s_redu[SNW];
-    const int c = blockIdx.x, row = blockIdx.y, t = threadIdx.x;
-    const RowSel *rs = (const RowSel *)ws.rowb(row);
-    if (rs->mode != SEL_SELECT || rs->nzb > SK_MAX) return;
-    const uint32_t zb = rs->zb;
-    const float zmax = rs->zmax;
-    uint32_t tot;
-    const uint32_t before = t < c ? ((const uint32_t *)ws.slot(row, t))[zb] : 0u;  // (c < nround <= SNT)
-    block_excl_scan_u(before, s_redu, tot);
-    const uint32_t off = tot;
-    float z[4];
-    bool in;
-    load_round(L + (size_t)row * V + (size_t)c * SROUND, min(SROUND, V - c * SROUND), 0, invT, z, in);
-    bool q[4];
-    uint32_t nq = 0;
+        COUNT ? (unsigned long long)a.top_k : tp < 1.0f ? 1ull : (unsigned long long)ceilf(tp);
+    if constexpr (COUNT) {
+        // At most 64 entries up to the threshold's bucket (a top-k of tens):
+        // they are gathered in index order and one wave ranks, keeps and
+        // draws. (Every wave finds the bucket by itself.)
+        const uint32_t h[4] = {s_hist[4 * lane], s_hist[4 * lane + 1], s_hist[4 * lane + 2], s_hist[4 * lane + 3]};
+        const uint32_t c0 = h[0], c1 = c0 + h[1], c2 = c1 + h[2], c3 = c2 + h[3];
+        const uint32_t ex = wave_scan_u(c3) - c3, k = (uint32_t)a.top_k;
+        const uint64_t m = __ballot(ex < k && k <= ex + c3);
+        if (m != 0ull && nround <= 64) {
+            const int f = __ffsll((unsigned long long)m) - 1;
+            const int j = ex + c0 >= k ? 0 : ex + c1 >= k ? 1 : ex + c2 >= k ? 2 : 3;
+            const uint32_t nle = __builtin_amdgcn_readlane(ex + (j == 0 ? c0 : j == 1 ? c1 : j == 2 ? c2 : c3), f);
+            const uint32_t zb = 4 * f + __builtin_amdgcn_readlane(j, f);
+            if (nle <= 64u) {
+                rounds([&](int c, const unsigned long long (&x)[4]) {
+                    unsigned long long v = 0;
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-        q[e] = in && zbin(z[e], zmax) == zb;
-        nq += q[e];
-    }
-    uint32_t tq;
-    uint32_t pos = off + block_excl_scan_u(nq, s_redu, tq);
-    uint8_t *g = ws.rowb(row) + ROW_GATHER;
-#pragma unroll
-    for (int e = 0; e < 4; e++)
-        if (q[e] && pos < (uint32_t)SK_MAX) {  // (pos < nzb: the counts of chunk_hist_kernel)
-            ((uint32_t *)g)[pos] = okey(z[e]);
-            ((float *)(g + SK_MAX * 4))[pos] = z[e];
-            ((int32_t *)(g + SK_MAX * 8))[pos] = c * SROUND + 4 * t + e;
-            pos++;
-        }
-}
-
-// Row blockIdx.x: the key passes inside the threshold bucket, then the ties
-// kept at the threshold (the first n_eq in index order; count: top-k, n_eq
-// the units left at tau).
-__global__ __launch_bounds__(SNT) void row_select_kernel(const float *__restrict__ L, int V, float invT, bool count,
-                                                         SpreadWs ws) {
-    __shared__ uint32_t s_redu[SNW];
-    __shared__ int s_redi[SNW];
-    __shared__ uint32_t s_hist[256];
-    __shared__ unsigned long long s_mass[256];
-    __shared__ uint32_t s_sel[2];
-    __shared__ unsigned long long s_selm[2];
-    __shared__ uint32_t s_ck[SK_MAX];
-    __shared__ float s_cz[SK_MAX];
-    __shared__ int s_ci[SK_MAX];
-    const int row = blockIdx.x, t = threadIdx.x, nround = ws.nround;
-    RowSel *rs = (RowSel *)ws.rowb(row);
-    if (rs->mode != SEL_SELECT) return;
-    const float zmax = rs->zmax, S = rs->S;
-    const int nzb = rs->nzb;
-    const bool gathered = nzb <= SK_MAX;
-    const float *Lr = L + (size_t)row * V;
-    if (gathered) {
-        const uint8_t *g = ws.rowb(row) + ROW_GATHER;
-        for (int i = t; i < nzb; i += SNT) {
-            s_ck[i] = ((const uint32_t *)g)[i];
-            s_cz[i] = ((const float *)(g + SK_MAX * 4))[i];
-            s_ci[i] = ((const int32_t *)(g + SK_MAX * 8))[i];
+                    for (int i = 0; i < 4; i++)
+                        if ((uint32_t)(lane + 64 * i) <= zb) v += x[i] & CMASK;
+                    v = wave_sum_u64(v);
+                    if (lane == 0) s_off[c] = (uint32_t)v;
+                });
+                __syncthreads();
+                const uint32_t n = lane < nround ? s_off[lane] : 0u, off = wave_scan_u(n) - n;
+#pragma unroll 1
+                for (int c = wave; c < nround; c += SNW)
+                    if (__builtin_amdgcn_readlane(n, c) != 0)
+                        round_entries(ws.slot(row, c) + SLOT_LIST, Lr, V, c, invT, (int)zb, __builtin_amdgcn_readlane(off, c),
+                                      [&](float z, int) { return zbin(z, zmax) <= zb; },
+                                      [&](uint32_t p, float z, int id) {
+                                          s_cz[p & 63u] = z;  // (p < nle)
+                                          s_ci[p & 63u] = id;
+                                      });
+                __syncthreads();
+                if (wave != 0) return;
+                const bool in = (uint32_t)lane < nle;
+                const float z = in ? s_cz[lane] : 0.f;
+                const int id = in ? s_ci[lane] : 0;
+                const uint32_t key = in ? okey(z) : 0u;
+                uint32_t rank = 0;
+                for (uint32_t i = 0; i < nle; i++) {  // (slots in index order: equals before it rank higher)
+                    const uint32_t ki = __builtin_amdgcn_readlane(key, i);
+                    rank += ki > key || (ki == key && i < (uint32_t)lane);
+                }
+                const bool keep = in && rank < k;
+                const uint64_t km = __ballot(keep);
+                const uint32_t p = __builtin_amdgcn_mbcnt_hi((uint32_t)(km >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)km, 0u));
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                if (keep) {
+                    s_cz[p] = z;
+                    s_ci[p] = id;
+                }
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                draw_candidates_wave(__popcll(km), a, ur, V, s_ci, s_cz, (int *)s_ck, out + row);
+                return;
+            }
         }
     }
+    pick_bucket<!COUNT>(s_hist, s_mass, target, s_sel, s_selm, false);
     __syncthreads();
     Select R;
-    R.zb = rs->zb;
+    R.all = s_selm[0] == ~0ull;
+    R.zb = R.all ? 256u : s_sel[0];
+    R.rem = R.all ? 0ull : target - s_selm[0];
     R.tau = 0u;
-    R.rem = rs->rem;
     R.cnt = 0;
-    R.all = false;
-    if (count)
-        refine_threshold<false>(Lr, V, nround, invT, zmax, 1.f, gathered, nzb, s_hist, s_mass, s_sel, s_selm, s_ck,
-                                s_cz, R);
-    else
-        refine_threshold<true>(Lr, V, nround, invT, zmax, S, gathered, nzb, s_hist, s_mass, s_sel, s_selm, s_ck,
-                               s_cz, R);
-    if (R.all) {
-        if (t == 0) rs->mode = SEL_ALL;
-        return;
-    }
-    const uint32_t zb = R.zb, tau = R.tau;
-    // ties at tau share one probability: keep the first n_eq of them
-    unsigned long long n_eq = R.rem;
-    if (!count) {
-        const float ptau = pexp(okey_inv(tau) - zmax) * (1.0f / S);
-        const unsigned long long mt = (unsigned long long)(ptau * 1099511627776.0f);
-        n_eq = mt ? (R.rem + mt - 1) / mt : (unsigned long long)R.cnt;
-    }
-    if (n_eq < 1) n_eq = 1;
+    const int nzb = R.all ? 0 : (int)s_hist[R.zb];
+    const bool gathered = nzb <= SK_MAX;
+    const uint32_t zb = R.zb;
+    // per round: the packed sum of the buckets above zb, and zb's count
+    rounds([&](int c, const unsigned long long (&h)[4]) {
+        unsigned long long v = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint32_t b = lane + 64 * j;
+            if (b < zb) v += h[j];
+            if (b == zb) s_off[c] = (uint32_t)(h[j] & CMASK);
+        }
+        v = wave_sum_u64(v);
+        if (lane == 0) s_cum[c] = v;
+    });
+    __syncthreads();
+    auto entries = [&](int c, uint32_t at, auto &&keep, auto &&f) {
+        round_entries(ws.slot(row, c) + SLOT_LIST, Lr, V, c, invT, (int)zb, at, keep, f);
+    };
     int tie_lim = V;
-    if (n_eq < R.cnt) {
-        if (gathered) {  // the gather is in index order: slots 4 t .. 4 t + 3
-            bool q[4];
-            uint32_t nq = 0;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int j = 4 * t + e;
-                q[e] = j < nzb && s_ck[j] == tau;
-                nq += q[e];
-            }
+    if (!R.all) {
+        if (gathered) {
             uint32_t tot;
-            int cnum = (int)block_excl_scan_u(nq, s_redu, tot);
-            int cand = INT_MAX;
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                if (q[e]) {
-                    cnum++;
-                    if (cnum == (int)n_eq && cand == INT_MAX) cand = s_ci[4 * t + e] + 1;
-                }
-            tie_lim = block_min_i(cand, s_redi);
-        } else {
-            int run = 0, lim = V;
-            for_rounds(Lr, V, nround, invT, [&](const float (&z)[4], bool in, int r) {
+            const uint32_t cnt = t < nround ? s_off[t] : 0u;  // (nround <= SNT)
+            const uint32_t off = block_excl_scan_u(cnt, s_redu, tot);
+            if (t < nround) s_off[t] = off;
+            __syncthreads();
+            for (int c = wave; c < nround; c += SNW)
+                if (c + 1 < nround ? s_off[c + 1] > s_off[c] : tot > s_off[c])
+                    entries(c, s_off[c], [&](float z, int) { return zbin(z, zmax) == zb; },
+                            [&](uint32_t p, float z, int j) {
+                                if (p < (uint32_t)SK_MAX) {  // (p < nzb: the counts of chunk_hist_kernel)
+                                    s_ck[p] = okey(z);
+                                    s_cz[p] = z;
+                                    s_ci[p] = j;
+                                }
+                            });
+            __syncthreads();
+        }
+        refine_threshold<!COUNT>(Lr, V, nround, invT, zmax, COUNT ? 1.f : S, gathered, nzb, s_hist, s_mass, s_sel,
+                                 s_selm, s_ck, s_cz, R);
+    }
+    if (!R.all) {
+        // ties at tau share one probability: keep the first n_eq of them
+        unsigned long long n_eq = R.rem;
+        if (!COUNT) {
+            const float ptau = pexp(okey_inv(R.tau) - zmax) * (1.0f / S);
+            const unsigned long long mt = (unsigned long long)(ptau * 1099511627776.0f);
+            n_eq = mt ? (R.rem + mt - 1) / mt : (unsigned long long)R.cnt;
+        }
+        if (n_eq < 1) n_eq = 1;
+        const uint32_t tau = R.tau;
+        if (n_eq < R.cnt) {
+            if (gathered) {  // the gather is in index order: slots 4 t .. 4 t + 3
                 bool q[4];
                 uint32_t nq = 0;
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    q[e] = in && zbin(z[e], zmax) == zb && okey(z[e]) == tau;
+                    const int j = 4 * t + e;
+                    q[e] = j < nzb && s_ck[j] == tau;
                     nq += q[e];
                 }
                 uint32_t tot;
-                const uint32_t ex = block_excl_scan_u(nq, s_redu, tot);
+                int cnum = (int)block_excl_scan_u(nq, s_redu, tot);
                 int cand = INT_MAX;
-                int cc = run + (int)ex;
 #pragma unroll
                 for (int e = 0; e < 4; e++)
                     if (q[e]) {
-                        cc++;
-                        if (cc == (int)n_eq && cand == INT_MAX) cand = r * SROUND + 4 * t + e + 1;
+                        cnum++;
+                        if (cnum == (int)n_eq && cand == INT_MAX) cand = s_ci[4 * t + e] + 1;
                     }
-                const int got = block_min_i(cand, s_redi);
-                if (lim == V && got != INT_MAX) lim = got;
-                run += (int)tot;
-            });
-            tie_lim = lim;
+                tie_lim = block_min_i(cand, s_redi);
+            } else {
+                int run = 0, lim = V;
+                for_rounds(Lr, V, nround, invT, [&](const float (&z)[4], bool in, int r) {
+                    bool q[4];
+                    uint32_t nq = 0;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        q[e] = in && zbin(z[e], zmax) == zb && okey(z[e]) == tau;
+                        nq += q[e];
+                    }
+                    uint32_t tot;
+                    const uint32_t ex = block_excl_scan_u(nq, s_redu, tot);
+                    int cand = INT_MAX;
+                    int cc = run + (int)ex;
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (q[e]) {
+                            cc++;
+                            if (cc == (int)n_eq && cand == INT_MAX) cand = r * SROUND + 4 * t + e + 1;
+                        }
+                    const int got = block_min_i(cand, s_redi);
+                    if (lim == V && got != INT_MAX) lim = got;
+                    run += (int)tot;
+                });
+                tie_lim = lim;
+            }
         }
     }
+    const bool all = R.all;
+    const uint32_t tau = R.tau;
+    if (!draw) {
+        if (t == 0) {
+            rs->mode = all ? SEL_ALL : SEL_SELECT;
+            rs->zb = zb;
+            rs->tau = tau;
+            rs->tie_lim = tie_lim;
+        }
+        return;
+    }
+    if (all && zb != 256u) {  // (the refinement fell short: every entry of every bucket)
+        __syncthreads();
+        rounds([&](int c, const unsigned long long (&h)[4]) {
+            const unsigned long long v = wave_sum_u64((h[0] + h[1]) + (h[2] + h[3]));
+            if (lane == 0) s_cum[c] = v;
+        });
+    }
+    // the kept entries of the threshold's bucket join their rounds' sums
+    if (!all) {
+        const float invS = 1.0f / S;
+        auto add = [&](float z, uint32_t k, int j) {
+            if (k > tau || (k == tau && j < tie_lim))
+                atomicAdd(&s_cum[j / SROUND], COUNT ? 1ull : (mass_fx(z, zmax, invS) << CBITS) + 1ull);
+        };
+        if (gathered) {
+            for (int i = t; i < nzb; i += SNT) add(s_cz[i], s_ck[i], s_ci[i]);
+        } else {
+            for_rounds(Lr, V, nround, invT, [&](const float (&z)[4], bool in, int r) {
+                if (in)
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (zbin(z[e], zmax) == zb) add(z[e], okey(z[e]), r * SROUND + 4 * t + e);
+            });
+        }
+    }
+    __syncthreads();
+    if constexpr (COUNT) {
+        uint32_t n;
+        const uint32_t cnt = t < nround ? (uint32_t)(s_cum[t] & CMASK) : 0u;
+        const uint32_t off = block_excl_scan_u(cnt, s_redu, n);
+        for (int i = t; i < nround; i += SNT) s_off[i] = off;
+        __syncthreads();  // (and the gathered bucket is no longer read)
+        for (int c = wave; c < nround; c += SNW)
+            if ((s_cum[c] & CMASK) != 0)
+                entries(c, s_off[c],
+                        [&](float z, int j) { return all || above_threshold(z, j, zmax, zb, tau, tie_lim); },
+                        [&](uint32_t p, float z, int j) {
+                            if (p < (uint32_t)SK_MAX) {
+                                s_cz[p] = z;
+                                s_ci[p] = j;
+                            }
+                        });
+        __syncthreads();
+        draw_candidates(min((int)n, SK_MAX), a, ur, V, s_ci, s_cz, (int *)s_ck, s_redf, s_redi, out + row);
+        return;
+    }
+    // top-p: the round holding u of the kept mass (every wave by itself, 64
+    // rounds at a time), then the entry inside it
+    auto cum64 = [&](int b, unsigned long long carry) {
+        unsigned long long inc = b + lane < nround ? s_cum[b + lane] >> CBITS : 0ull;
+        for (int o = 1; o < 64; o <<= 1) {
+            const unsigned long long y = __shfl_up(inc, o);
+            if (lane >= o) inc += y;
+        }
+        return carry + inc;
+    };
+    unsigned long long total = 0;
+    for (int b = 0; b < nround; b += 64) total = __shfl(cum64(b, total), 63);
+    const double goal = (double)ur * (double)total;
+    unsigned long long below = 0;
+    int rr = -1;
+    for (int b = 0; b < nround && rr < 0; b += 64) {
+        const unsigned long long cum = cum64(b, below);
+        const uint64_t m = __ballot(b + lane < nround && goal <= (double)cum);
+        const int f = m ? __ffsll((unsigned long long)m) - 1 : 64;
+        if (f > 0) below = __shfl(cum, f - 1);
+        if (f < 64) rr = b + f;
+    }
+    if (rr < 0) {  // (u above 1)
+        if (t == 0) out[row] = V - 1;
+        return;
+    }
+    const float invS = 1.0f / S;
+    const float inv = total > 0 ? (float)(1099511627776.0 / (double)total) : 1.0f;
+    const float before = (float)((double)below * (total > 0 ? 1.0 / (double)total : 0.0));
+    float z[4], v[4];
+    bool in;
+    load_round(Lr, V, rr, invT, z, in);
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        v[e] = in && (all || above_threshold(z[e], rr * SROUND + 4 * t + e, zmax, zb, tau, tie_lim))
+                   ? pexp(z[e] - zmax) * invS * inv
+                   : 0.f;
+    float tot;
+    const int hit = first_cdf_hit(v, in ? 4 : 0, before, ur, s_redf, tot);
+    const int local = block_min_i(hit, s_redi);
+    // (the scan inside the round can end a rounding step below the mass that
+    // selected it: then the round's last kept entry)
+    int last = INT_MAX;
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        if (v[e] > 0.f) last = INT_MAX - (4 * t + e);
+    const int lastk = block_min_i(last, s_redi);
     if (t == 0) {
-        rs->tau = tau;
-        rs->tie_lim = tie_lim;
+        const int tok =
+            local != INT_MAX ? rr * SROUND + local : lastk != INT_MAX ? rr * SROUND + (INT_MAX - lastk) : V - 1;
+        out[row] = min(tok, V - 1);
     }
 }
 
@@ -1705,18 +2016,23 @@ struct Keep {
 };
 
 // 1 / the sum of the row's chunk values at byte `off` of their slots (a
-// fixed order), or 1 when it is not positive.
-__device__ float kept_inv(const SpreadWs &ws, int row, int off, float *s_redf) {
-    float l = 0.f;
-    for (int i = threadIdx.x; i < ws.nround; i += SNT) l += *(const float *)(ws.slot(row, i) + off);
-    const float total = block_sum(l, s_redf);
+// fixed order, as row_stats), or 1 when it is not positive.
+__device__ float kept_inv(const SpreadWs &ws, int row, int off) {
+    const int l = threadIdx.x & 63;
+    float acc = 0.f;
+    for (int v = 0; 64 * v < ws.nround; v++) {
+        const int i = 64 * v + l;
+        const float sv = wave_sum(i < ws.nround ? *(const float *)(ws.slot(row, i) + off) : 0.f);
+        if (l == v) acc = sv;
+    }
+    const float total = wave_sum(acc);
     return total > 0.f ? 1.0f / total : 1.0f;
 }
 
 // false for a row without finite statistics (no draw); minp: the min-p
 // stage (its inv1 from the top-p stage's kept sums).
 __device__ bool load_keep(const SpreadWs &ws, int row, bool topp, bool minp, float min_p, float zmax, float S,
-                          float *s_redf, Keep &k) {
+                          Keep &k) {
     k.topp = topp;
     k.minp = minp;
     k.zmax = zmax;
@@ -1733,7 +2049,7 @@ __device__ bool load_keep(const SpreadWs &ws, int row, bool topp, bool minp, flo
         k.zb = rs->zb;
         k.tau = rs->tau;
         k.tie_lim = rs->tie_lim;
-        if (minp) k.inv1 = kept_inv(ws, row, SLOT_CSUM, s_redf);
+        if (minp) k.inv1 = kept_inv(ws, row, SLOT_CSUM);
     }
     k.thr = k.invS * k.inv1 * min_p;
     return true;
@@ -1742,30 +2058,32 @@ __device__ bool load_keep(const SpreadWs &ws, int row, bool topp, bool minp, flo
 // Chunk blockIdx.x of row blockIdx.y: the sum of its kept probabilities,
 // stage 0 (top-p) at SLOT_CSUM, stage 1 (min-p, after top-p if topp) at
 // SLOT_CSUM + 4.
-__global__ __launch_bounds__(SNT) void chunk_keptsum_kernel(const float *__restrict__ L, int V, float invT, bool topp,
+__global__ __launch_bounds__(CNT) void chunk_keptsum_kernel(const float *__restrict__ L, int V, float invT, bool topp,
                                                             int stage, float min_p, SpreadWs ws) {
-    __shared__ float s_redf[2 * SNW];
+    __shared__ float s_red[SNW];
     const int c = blockIdx.x, row = blockIdx.y, t = threadIdx.x;
+    float z[CR][4];
+    load_chunk(L + (size_t)row * V, V, c, invT, z);
     float zmax, S;
-    if (topp) {  // (the statistics row_pick_kernel stored: the same bits)
+    if (topp) {  // (the statistics chunk_hist_kernel stored: the same bits)
         const RowSel *rs = (const RowSel *)ws.rowb(row);
         if (rs->mode == SEL_DEGEN) return;
         zmax = rs->zmax;
         S = rs->S;
-    } else if (!row_stats(ws.part + (size_t)row * ws.nround, ws.nround, s_redf, zmax, S)) {
+    } else if (!row_stats(ws.part + (size_t)row * ws.nround, ws.nround, zmax, S)) {
         return;
     }
     Keep keep;
-    if (!load_keep(ws, row, topp, stage == 1, min_p, zmax, S, s_redf, keep)) return;
-    float z[4];
-    bool in;
-    load_round(L + (size_t)row * V + (size_t)c * SROUND, min(SROUND, V - c * SROUND), 0, invT, z, in);
-    float sum = 0.f;
-    if (in)
+    if (!load_keep(ws, row, topp, stage == 1, min_p, zmax, S, keep)) return;
+    float sum[CR];
 #pragma unroll
-        for (int e = 0; e < 4; e++) sum += keep.p1(z[e], c * SROUND + 4 * t + e);
-    sum = block_sum(sum, s_redf);
-    if (t == 0) *(float *)(ws.slot(row, c) + SLOT_CSUM + 4 * stage) = sum;
+    for (int r = 0; r < CR; r++) {
+        sum[r] = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; e++) sum[r] += keep.p1(z[r][e], c * SROUND + chunk_entry(r) + e);
+    }
+    const float total = chunk_sum(sum, s_red);
+    if (t == 0) *(float *)(ws.slot(row, c) + SLOT_CSUM + 4 * stage) = total;
 }
 
 // Row blockIdx.x: the kept mass of the last stage, each round's share of
@@ -1783,16 +2101,16 @@ __global__ __launch_bounds__(SNT) void keep_draw_kernel(const float *__restrict_
     const float ur = u[row];
     float zmax, S;
     bool ok;
-    if (topp) {  // (the statistics row_pick_kernel stored: the same bits)
+    if (topp) {  // (the statistics chunk_hist_kernel stored: the same bits)
         const RowSel *rs = (const RowSel *)ws.rowb(row);
         ok = rs->mode != SEL_DEGEN;
         zmax = rs->zmax;
         S = rs->S;
     } else {
-        ok = row_stats(ws.part + (size_t)row * nround, nround, s_redf, zmax, S);
+        ok = row_stats(ws.part + (size_t)row * nround, nround, zmax, S);
     }
     Keep keep;
-    if (!ok || !load_keep(ws, row, topp, minp, min_p, zmax, S, s_redf, keep) || ur != ur) {
+    if (!ok || !load_keep(ws, row, topp, minp, min_p, zmax, S, keep) || ur != ur) {
         if (t == 0) out[row] = V - 1;
         return;
     }
@@ -1801,7 +2119,7 @@ __global__ __launch_bounds__(SNT) void keep_draw_kernel(const float *__restrict_
         return;
     }
     const int off = SLOT_CSUM + (minp ? 4 : 0);
-    const float inv = kept_inv(ws, row, off, s_redf);
+    const float inv = kept_inv(ws, row, off);
     for (int i = t; i < nround; i += SNT) s_round[i] = *(const float *)(ws.slot(row, i) + off) * inv;
     __syncthreads();
     if (t == 0) {
@@ -1843,101 +2161,6 @@ __global__ __launch_bounds__(SNT) void keep_draw_kernel(const float *__restrict_
             local != INT_MAX ? rr * SROUND + local : lastk != INT_MAX ? rr * SROUND + (INT_MAX - lastk) : V - 1;
         out[row] = min(tok, V - 1);
     }
-}
-
-// Spread top-k above SK_SPREAD (or over more than SPART_ROUNDS rounds), with
-// any top-p / min-p after it: the k-th element's bucket and key by count
-// (as top-p's threshold), then each chunk's kept entries counted, compacted
-// in index order into the row's gather (k <= SK_MAX), and one workgroup per
-// row runs draft_sample_kernel's candidate draw over them: its tokens.
-__global__ __launch_bounds__(SNT) void chunk_keptcount_kernel(const float *__restrict__ L, int V, float invT,
-                                                              SpreadWs ws) {
-    __shared__ uint32_t s_redu[SNW];
-    const int c = blockIdx.x, row = blockIdx.y, t = threadIdx.x;
-    const RowSel *rs = (const RowSel *)ws.rowb(row);
-    const int mode = rs->mode;
-    if (mode == SEL_DEGEN) return;
-    const uint32_t zb = rs->zb, tau = rs->tau;
-    const int tie_lim = rs->tie_lim;
-    const float zmax = rs->zmax;
-    float z[4];
-    bool in;
-    load_round(L + (size_t)row * V + (size_t)c * SROUND, min(SROUND, V - c * SROUND), 0, invT, z, in);
-    uint32_t n = 0;
-    if (in)
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-            n += mode == SEL_ALL || above_threshold(z[e], c * SROUND + 4 * t + e, zmax, zb, tau, tie_lim);
-    uint32_t tot;
-    block_excl_scan_u(n, s_redu, tot);
-    if (t == 0) *(uint32_t *)(ws.slot(row, c) + SLOT_CSUM) = tot;
-}
-
-__global__ __launch_bounds__(SNT) void chunk_compact_kernel(const float *__restrict__ L, int V, float invT,
-                                                            SpreadWs ws) {
-    __shared__ uint32_t s_redu[SNW];
-    const int c = blockIdx.x, row = blockIdx.y, t = threadIdx.x;
-    const RowSel *rs = (const RowSel *)ws.rowb(row);
-    const int mode = rs->mode;
-    if (mode == SEL_DEGEN) return;
-    const uint32_t zb = rs->zb, tau = rs->tau;
-    const int tie_lim = rs->tie_lim;
-    const float zmax = rs->zmax;
-    uint32_t tot;
-    const uint32_t before = t < c ? *(const uint32_t *)(ws.slot(row, t) + SLOT_CSUM) : 0u;  // (c < nround <= SNT)
-    block_excl_scan_u(before, s_redu, tot);
-    const uint32_t off = tot;
-    float z[4];
-    bool in;
-    load_round(L + (size_t)row * V + (size_t)c * SROUND, min(SROUND, V - c * SROUND), 0, invT, z, in);
-    bool k[4];
-    uint32_t n = 0;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        k[e] = in && (mode == SEL_ALL || above_threshold(z[e], c * SROUND + 4 * t + e, zmax, zb, tau, tie_lim));
-        n += k[e];
-    }
-    uint32_t tk;
-    uint32_t pos = off + block_excl_scan_u(n, s_redu, tk);
-    uint8_t *g = ws.rowb(row) + ROW_GATHER;
-#pragma unroll
-    for (int e = 0; e < 4; e++)
-        if (k[e]) {
-            if (pos < (uint32_t)SK_MAX) {
-                ((float *)(g + SK_MAX * 4))[pos] = z[e];
-                ((int32_t *)(g + SK_MAX * 8))[pos] = c * SROUND + 4 * t + e;
-            }
-            pos++;
-        }
-}
-
-__global__ __launch_bounds__(SNT) void cand_draw_kernel(int V, SampleArgs a, SpreadWs ws, const float *__restrict__ u,
-                                                        int32_t *__restrict__ out) {
-    __shared__ float s_redf[2 * SNW];
-    __shared__ int s_redi[SNW];
-    __shared__ int s_cidx[SK_MAX];
-    __shared__ float s_cp[SK_MAX];
-    __shared__ int s_sort[SK_MAX];
-    const int row = blockIdx.x, t = threadIdx.x, nround = ws.nround;
-    const float ur = u[row];
-    if (((const RowSel *)ws.rowb(row))->mode == SEL_DEGEN || ur != ur) {  // (as the one-row kernel)
-        if (t == 0) out[row] = V - 1;
-        return;
-    }
-    if (!(ur > 0.f)) {  // the reference's draw returns index 1 (here 0) when r <= 0
-        if (t == 0) out[row] = 0;
-        return;
-    }
-    float l = 0.f;
-    for (int c = t; c < nround; c += SNT) l += (float)*(const uint32_t *)(ws.slot(row, c) + SLOT_CSUM);
-    const int n = min((int)block_sum(l, s_redf), SK_MAX);  // (counts below 2^24: exact)
-    const uint8_t *g = ws.rowb(row) + ROW_GATHER;
-    for (int i = t; i < n; i += SNT) {
-        s_cp[i] = ((const float *)(g + SK_MAX * 4))[i];
-        s_cidx[i] = ((const int32_t *)(g + SK_MAX * 8))[i];
-    }
-    __syncthreads();
-    draw_candidates(n, a, ur, V, s_cidx, s_cp, s_sort, s_redf, s_redi, out + row);
 }
 
 // In place on rows of logits: for every distinct id of the row's list in
@@ -1992,76 +2215,53 @@ size_t sample_spread_ws(int rows, int V) {
 // Rows spread over workgroups of one round each (chunk statistics first):
 // plain draws (T > 0, no top-k, top-p or min-p), then one workgroup per row
 // merges them, picks the round and scans it (as draft_sample_kernel's draw);
-// top-k from 1 to SK_SPREAD over at most SPART_ROUNDS rounds: each chunk's
-// top-k, then one workgroup per row draws among the candidates; top-p
-// and / or min-p without top-k (threshold histograms, pick, gather, key
-// passes): the chunks' kept sums per stage, then the draw; a larger top-k
-// (any top-p / min-p after it): its threshold as top-p's but by count, the
-// kept entries compacted, then the candidate draw; T = 0: each chunk's
-// argmax, then the row's. Rows over more than SMAX_ROUNDS rounds run draft_sample_kernel.
+// top-k up to SK_MAX (any top-p / min-p after it) and top-p: histograms and
+// candidate lists, then one workgroup per row for the threshold and the
+// draw; min-p, alone or after top-p: the chunks' kept sums per stage, then
+// the draw; T = 0: each chunk's argmax, then the row's. Rows over more than
+// SMAX_ROUNDS rounds, and a larger top-k, run draft_sample_kernel.
 // ws: sample_spread_ws bytes (8-byte aligned).
 hipError_t launch_sample_spread(const float *L, int rows, int V, float T, int top_k, float top_p, float min_p,
                                 const float *u, int32_t *out, void *ws, hipStream_t st) {
     const int nround = (V + SROUND - 1) / SROUND;
     if (T == 0.f && nround <= SMAX_ROUNDS) {
         float2 *part = (float2 *)ws;
-        chunk_argmax_kernel<<<dim3(nround, rows), SNT, 0, st>>>(L, V, part);
+        chunk_argmax_kernel<<<dim3(nround, rows), CNT, 0, st>>>(L, V, part);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         argmax_draw_kernel<<<rows, SNT, 0, st>>>(V, part, out);
         return hipGetLastError();
     }
-    const bool live = T > 0.f && nround <= SMAX_ROUNDS;
-    const bool plain = live && top_k == 0 && top_p >= 1.0f && min_p <= 0.f;
-    const bool topk = live && top_k >= 1 && top_k <= SK_SPREAD && nround <= SPART_ROUNDS;
-    // top-k beyond the chunk-candidate path: the threshold as top-p's, by
-    // count, its kept entries compacted (up to SK_MAX of them; a larger top-k
-    // takes the one-workgroup kernel's threshold path)
-    const bool bigk = live && top_k > 0 && top_k <= SK_MAX && !topk;
-    const bool topp = live && ((top_k == 0 && top_p < 1.0f) || bigk);
-    const bool minp = live && top_k == 0 && min_p > 0.f;
-    if (!plain && !topk && !topp && !minp) return launch_sample(L, rows, V, T, top_k, top_p, min_p, u, out, st);
-    if (top_k > SK_MAX) return launch_sample(L, rows, V, T, top_k, top_p, min_p, u, out, st);
+    if (!(T > 0.f) || nround > SMAX_ROUNDS || top_k > SK_MAX)
+        return launch_sample(L, rows, V, T, top_k, top_p, min_p, u, out, st);
+    const bool topk = top_k > 0, topp = !topk && top_p < 1.0f, minp = !topk && min_p > 0.f;
     const float invT = 1.0f / T;
     const size_t rc = (size_t)rows * nround;
     uint8_t *w = (uint8_t *)ws;
     const SpreadWs W{(float2 *)w, w + rc * sizeof(float2), w + rc * (sizeof(float2) + SLOT_BYTES), nround};
     const dim3 chunks(nround, rows);
-    chunk_stats_kernel<<<chunks, SNT, 0, st>>>(L, V, invT, W.part);
+    const SampleArgs a{T, top_k, top_p, min_p};
+    chunk_stats_kernel<<<chunks, CNT, 0, st>>>(L, V, invT, W.part);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if (plain) {
-        chunk_draw_kernel<<<rows, SNT, 0, st>>>(L, V, invT, W.part, u, out);
-        return hipGetLastError();
-    }
     if (topk) {
-        chunk_topk_kernel<<<chunks, SNT, 0, st>>>(L, V, invT, top_k, W);
+        chunk_hist_kernel<true><<<chunks, CNT, 0, st>>>(L, V, invT, top_k, 1.f, W);
         if ((e = hipGetLastError()) != hipSuccess) return e;
-        const SampleArgs a{T, top_k, top_p, min_p};
-        topk_draw_kernel<<<rows, SNT, 0, st>>>(V, a, W, u, out);
+        row_threshold_kernel<true><<<rows, SNT, 0, st>>>(L, V, invT, a, true, W, u, out);
         return hipGetLastError();
     }
     if (topp) {
-        chunk_hist_kernel<<<chunks, SNT, 0, st>>>(L, V, invT, bigk, W);
+        chunk_hist_kernel<false><<<chunks, CNT, 0, st>>>(L, V, invT, 0, top_p, W);
         if ((e = hipGetLastError()) != hipSuccess) return e;
-        row_pick_kernel<<<rows, SNT, 0, st>>>(top_p, bigk ? top_k : 0, W);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-        chunk_gather_kernel<<<chunks, SNT, 0, st>>>(L, V, invT, W);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-        row_select_kernel<<<rows, SNT, 0, st>>>(L, V, invT, bigk, W);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
+        row_threshold_kernel<false><<<rows, SNT, 0, st>>>(L, V, invT, a, !minp, W, u, out);
+        if ((e = hipGetLastError()) != hipSuccess || !minp) return e;
     }
-    if (bigk) {
-        chunk_keptcount_kernel<<<chunks, SNT, 0, st>>>(L, V, invT, W);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-        chunk_compact_kernel<<<chunks, SNT, 0, st>>>(L, V, invT, W);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-        const SampleArgs a{T, top_k, top_p, min_p};
-        cand_draw_kernel<<<rows, SNT, 0, st>>>(V, a, W, u, out);
+    if (!topp && !minp) {
+        chunk_draw_kernel<<<rows, SNT, 0, st>>>(L, V, invT, W.part, u, out);
         return hipGetLastError();
     }
-    for (int stage = topp ? 0 : 1; stage <= (minp ? 1 : 0); stage++) {
-        chunk_keptsum_kernel<<<chunks, SNT, 0, st>>>(L, V, invT, topp, stage, min_p, W);
+    for (int stage = topp ? 0 : 1; stage <= 1; stage++) {
+        chunk_keptsum_kernel<<<chunks, CNT, 0, st>>>(L, V, invT, topp, stage, min_p, W);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     keep_draw_kernel<<<rows, SNT, 0, st>>>(L, V, invT, topp, minp, min_p, W, u, out);

@@ -1,0 +1,91 @@
+"""GPU: the spread sampler's thresholds at the edges of its kernels: rounds of
+4096 logits, candidate lists of at most 336 entries a round (rows whose
+entries crowd one bucket overflow them, and a bucket of more than 4096 entries
+is refined over the row), the cuts that leave entries out of the histograms
+(top-k up to 256, top-p up to 1 - 1e-4), ties at the threshold, masked and
+unaligned rows. Top-k tokens equal the one-workgroup kernel's; top-p and
+min-p draws equal the oracle's except where u lies within 1e-5 (the sum of
+the fp32 probabilities' relative errors) of a step of its cumulative
+distribution."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [5, 337, 4095, 4096, 4097, 8190, 70001]
+KINDS = ["gauss", "lm", "flat", "few", "masked"]
+
+
+@pytest.fixture(scope="module")
+def ih():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import inferno_hip
+    assert inferno_hip.quant_kernels_available(), inferno_hip._lib.last_error()
+    return inferno_hip
+
+
+def _rows(kind, rows, V):
+    rng = np.random.default_rng(V * 7 + KINDS.index(kind))
+    if kind == "lm":  # a language model's: falling with the rank
+        L = -1.6 * np.log(rng.permuted(np.tile(np.arange(1.0, V + 1), (rows, 1)), axis=1)) + 0.5 * rng.standard_normal((rows, V))
+    elif kind == "flat":  # one bucket holds every entry, values distinct
+        L = 0.01 * rng.standard_normal((rows, V))
+    elif kind == "few":  # ties everywhere
+        L = rng.integers(0, 6, (rows, V)) * 0.5
+    else:
+        L = 3.0 * rng.standard_normal((rows, V))
+        if kind == "masked":
+            L[rng.random((rows, V)) < 0.7] = -np.inf
+            L[:, V // 2] = 4.0
+    return L.astype(np.float32)
+
+
+def _dev(a):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+@pytest.mark.parametrize("V", SIZES)
+@pytest.mark.parametrize("kind", KINDS)
+def test_topk(ih, kind, V):
+    rows = 5
+    L = _rows(kind, rows, V)
+    d = _dev(L)
+    rng = np.random.default_rng(V)
+    for k in (1, 2, 40, 64, 65, 256, 257, 1000, 4096):
+        if k >= V:
+            continue
+        for kw in (dict(top_k=k), dict(top_k=k, top_p=0.9), dict(top_k=k, top_p=0.95, min_p=0.02)):
+            u = _dev(rng.random(rows).astype(np.float32))
+            a = ih.softmax_sample(d, u, temperature=0.8, **kw).cpu().numpy()
+            b = ih.softmax_sample(d, u, temperature=0.8, spread=False, **kw).cpu().numpy()
+            assert np.array_equal(a, b), (k, kw, a, b)
+
+
+@pytest.mark.parametrize("V", SIZES)
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("kw", [dict(top_p=0.5), dict(top_p=0.95), dict(top_p=0.99985), dict(top_p=0.99995),
+                                dict(top_p=0.9, min_p=0.05), dict(min_p=0.05), dict(), dict(top_p=1e-6)],
+                         ids=lambda kw: ",".join(f"{k}={v}" for k, v in kw.items()) or "plain")
+def test_mass_draws(ih, kind, V, kw):
+    rows = 8
+    L = _rows(kind, rows, V)
+    us = np.random.default_rng(V + 1).random(rows).astype(np.float32)
+    us[0] = np.float32(1 - 2.0 ** -24)
+    got = ih.softmax_sample(_dev(L), _dev(us), temperature=0.9, **kw).cpu().numpy()
+    for r in range(rows):
+        p = O.sample_dist(L[r], temperature=0.9, **kw).astype(np.float64)
+        c = np.cumsum(p)
+        g, want = int(got[r]), O.softmax_sample(L[r], float(us[r]), temperature=0.9, **kw)
+        if g == want:
+            continue
+        edge = 1.0
+        if kw.get("top_p", 1.0) < 1.0:
+            q = np.sort(O.sample_dist(L[r], temperature=0.9).astype(np.float64))[::-1]
+            edge = np.min(np.abs(np.cumsum(q) - kw["top_p"]))
+        before = c[g - 1] if g else 0.0
+        assert edge < 1e-5 or (before - 1e-5 <= us[r] <= c[g] + 1e-5), (r, g, want, us[r], before, c[g])
