@@ -165,28 +165,25 @@ __device__ __forceinline__ void load_unit(const uint8_t *__restrict__ u, int g, 
         r.d = ld_u16(u + 208);
     } else {
         // transpose k covers blocks 2k, 2k+1: lane group g fetches half (g&1)
-        // of block 2k + (g>>1)
+        // of block 2k + (g>>1), and the scales of blocks 2g, 2g+1 (in d[0],
+        // d[1] until finish_unit). Blocks past the row's end read block 0 of
+        // the unit; finish_unit zeroes their scales. (Loads only: a select on
+        // the loaded values here made every item of the ring wait for its own
+        // loads, and the scales took 8 loads a lane instead of 2.)
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             const int b = 2 * k + (g >> 1);
-            const bool live = b < nblk;
-            const uint4 v = ld_u128(u + 34 * (live ? b : 0) + 2 + 16 * (g & 1));
-            r.w0[2 * k] = live ? v.x : 0x80808080u;
-            r.w1[2 * k] = live ? v.y : 0x80808080u;
-            r.w0[2 * k + 1] = live ? v.z : 0x80808080u;
-            r.w1[2 * k + 1] = live ? v.w : 0x80808080u;
+            const uint4 v = ld_u128(u + 34 * (b < nblk ? b : 0) + 2 + 16 * (g & 1));
+            r.w0[2 * k] = v.x; r.w1[2 * k] = v.y; r.w0[2 * k + 1] = v.z; r.w1[2 * k + 1] = v.w;
         }
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
-            const bool live = b < nblk;
-            const uint32_t d = ld_u16(u + 34 * (live ? b : 0));
-            r.d[b] = live ? d : 0u;
-        }
+        r.d[0] = ld_u16(u + 34 * (2 * g < nblk ? 2 * g : 0));
+        r.d[1] = ld_u16(u + 34 * (2 * g + 1 < nblk ? 2 * g + 1 : 0));
     }
 }
 
+// (nblk: as load_unit's)
 template <int QT>
-__device__ __forceinline__ void finish_unit(Unit<QT> &r) {
+__device__ __forceinline__ void finish_unit(Unit<QT> &r, int nblk = 8) {
     if constexpr (QT == QT_Q4_K) {
         // GGUF byte order to the order the decoder reads: bytes 1 and 2 of
         // each quant dword swapped (the packer stores them so)
@@ -206,6 +203,17 @@ __device__ __forceinline__ void finish_unit(Unit<QT> &r) {
         // lane group's half-block; after: dword g of each of the 4 halves
 #pragma unroll
         for (int k = 0; k < 4; k++) xpose4(r.w0[2 * k], r.w1[2 * k], r.w0[2 * k + 1], r.w1[2 * k + 1]);
+        // the four lane groups' scale pairs to every lane of the row
+        const uint32_t p = r.d[0] | (r.d[1] << 16);
+        const auto h = __builtin_amdgcn_permlane32_swap(p, p, false, false);
+        const auto lo = __builtin_amdgcn_permlane16_swap(h[0], h[0], false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(h[1], h[1], false, false);
+        const uint32_t w[4] = {(uint32_t)lo[0], (uint32_t)lo[1], (uint32_t)hi[0], (uint32_t)hi[1]};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            r.d[2 * j] = 2 * j < nblk ? w[j] & 0xffffu : 0u;
+            r.d[2 * j + 1] = 2 * j + 1 < nblk ? w[j] >> 16 : 0u;
+        }
     }
 }
 
@@ -369,7 +377,9 @@ __global__ __launch_bounds__(64 * PACK_WAVES) void pack_kernel(const uint8_t *__
             const uint4 v = b < nblk ? ld_u128(src + 34 * b + 2 + 16 * (g & 1)) : z;
             r.w0[2 * k] = v.x; r.w1[2 * k] = v.y; r.w0[2 * k + 1] = v.z; r.w1[2 * k + 1] = v.w;
         }
-        const uint32_t d = (2 * g < nblk ? ld_u16(src + 68 * g) : 0u) | (2 * g + 1 < nblk ? ld_u16(src + 68 * g + 34) << 16 : 0u);
+        r.d[0] = 2 * g < nblk ? ld_u16(src + 68 * g) : 0u;
+        r.d[1] = 2 * g + 1 < nblk ? ld_u16(src + 68 * g + 34) : 0u;
+        const uint32_t d = r.d[0] | (r.d[1] << 16);
         finish_unit<QT>(r);
 #pragma unroll
         for (int k = 0; k < 4; k++)
@@ -1081,7 +1091,7 @@ void gemm_q_kernel(const uint8_t *__restrict__ W, float *__restrict__ Y, int M, 
     const uint8_t *a_lane = a_lds + lane * (QT == QT_Q6_K ? 8 : 16);
     int cj = 0, cu = 0;  // consume position
     auto consume = [&](Unit<QT> &b) {
-        if constexpr (!PK) finish_unit<QT>(b);
+        if constexpr (!PK) finish_unit<QT>(b, u0 + cu == n_units - 1 ? tail_blk : 8);
         compute_unit<QT, MT, SPLIT>(b, a_lane + (size_t)cu * UNIT_A, x_lds + (size_t)cu * 8 * TOK,
                                     i_lds + (size_t)cu * TOK, g, A);
         if (++cu == nu) {
@@ -1720,7 +1730,7 @@ void gemm_v_kernel(const uint8_t *__restrict__ W, const uint8_t *__restrict__ af
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) acc[mt] = macc[mt] = f4{0.f, 0.f, 0.f, 0.f};
     auto consume = [&](int j, int u, Unit<QT> &b) {
-        if constexpr (!PK) finish_unit<QT>(b);
+        if constexpr (!PK) finish_unit<QT>(b, unit0 + u >= n_units - 1 ? tail_blk : 8);
         compute_v<QT, SPLIT, MT>(b, a[u], inv[u], g, live[u], acc, macc);
         if (u == UPS - 1) {
             float vals[MT * TPL];
@@ -2111,7 +2121,7 @@ void gemm_w_kernel(const uint8_t *__restrict__ W, float *__restrict__ Y, int M, 
     // flush (a batch is complete): wave i sums tile i of the batch in wave
     // order and stores it
     auto consume = [&](int j, int jb, bool flush, Unit<QT> &b) __attribute__((always_inline)) {
-        if constexpr (!PK) finish_unit<QT>(b);
+        if constexpr (!PK) finish_unit<QT>(b, un == n_units - 1 ? tail_blk : 8);
         float vals[NVP];
         unit_vals<QT, SPLIT, MT>(b, a, inv, g, live, *(float(*)[NV])vals);
 #pragma unroll
