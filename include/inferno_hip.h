@@ -328,7 +328,7 @@ int ihip_add(float *y_dev, const float *x_dev, int64_t n, void *stream);
  * IHIP_GEMM_PACKED pack the concatenation). w_down: [H x F]. flags:
  * IHIP_GEMM_F32 / IHIP_GEMM_HALF / IHIP_GEMM_PACKED (the precision and layout
  * of both matmuls). Workspace: ihip_mlp_ws_bytes (holds the [M x 2F] gate/up
- * product). Two input-stage + matmul launches on the stream; the same result
+ * product, or its K-slice partials and down's own workspace). Two input-stage + matmul launches on the stream; the same result
  * bit for bit as ihip_gemm_q_ex with IHIP_ACT_RMSNORM into a [M x 2F] buffer
  * followed by ihip_gemm_q_ex with IHIP_ACT_SILU_MUL and IHIP_GEMM_ACCUM. */
 int ihip_mlp_ws_bytes(int qt_gate_up, int qt_down, int M, int H, int F,
