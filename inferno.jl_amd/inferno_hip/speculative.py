@@ -11,7 +11,9 @@ Token ids are 0-based (the Julia shim adds 1).
 """
 from __future__ import annotations
 
+import ctypes as C
 from dataclasses import dataclass
+from functools import lru_cache
 
 from . import _lib
 from .quantized_kernels import _ptr, _stream, check_tensor
@@ -25,15 +27,27 @@ def _ws(nbytes: int, device):
     return torch.empty(max(nbytes, 16), dtype=torch.uint8, device=device)
 
 
+# (Workspace sizes: functions of their numbers alone, asked once a shape.)
+@lru_cache(maxsize=4096)
+def _accept_ws_bytes(rows: int, V: int) -> int:
+    nb = C.c_size_t()
+    _lib.check(_lib.load().ihip_accept_ws_bytes(rows, V, C.byref(nb)))
+    return int(nb.value)
+
+
+@lru_cache(maxsize=4096)
+def _spec_accept_ws_bytes(steps: int, k: int, V: int, top_k: int, top_p: float, min_p: float) -> int:
+    nb = C.c_size_t()
+    _lib.check(_lib.load().ihip_spec_accept_ex_ws_bytes(steps, k, V, top_k, top_p, min_p, C.byref(nb)))
+    return int(nb.value)
+
+
 def softmax_stats(logits, temperature: float, stream=None):
     """(zmax, zsum) per row of logits [rows, V] for z = logits / T."""
     import torch
-    import ctypes as C
     rows, V = logits.shape
     L = _lib.load()
-    nb = C.c_size_t()
-    _lib.check(L.ihip_accept_ws_bytes(rows, V, C.byref(nb)))
-    ws = _ws(nb.value, logits.device)
+    ws = _ws(_accept_ws_bytes(rows, V), logits.device)
     zmax = torch.empty(rows, dtype=torch.float32, device=logits.device)
     zsum = torch.empty_like(zmax)
     _lib.check(L.ihip_softmax_stats(_ptr(logits), rows, V, temperature, _ptr(zmax), _ptr(zsum), _ptr(ws),
@@ -58,7 +72,6 @@ def spec_accept(target_logits, draft_logits, draft_tokens, temperature: float, u
     (:100-104); the ratio tests and residuals stay unfiltered.
     """
     import torch
-    import ctypes as C
     check_tensor(target_logits, "target_logits", torch.float32)
     if target_logits.dim() == 2:
         target_logits = target_logits.unsqueeze(0)
@@ -77,12 +90,11 @@ def spec_accept(target_logits, draft_logits, draft_tokens, temperature: float, u
     check_tensor(u_res, "u_res", torch.float32, (S,))
     check_tensor(u_bonus, "u_bonus", torch.float32, (S,))
     L = _lib.load()
-    nb = C.c_size_t()
-    _lib.check(L.ihip_spec_accept_ex_ws_bytes(S, k, V, top_k, top_p, min_p, C.byref(nb)))
+    need = _spec_accept_ws_bytes(S, k, V, top_k, top_p, min_p)
     dev = target_logits.device
     if ws is None:
-        ws = _ws(nb.value, dev)
-    check_tensor(ws, "ws", torch.uint8, min_numel=nb.value)
+        ws = _ws(need, dev)
+    check_tensor(ws, "ws", torch.uint8, min_numel=need)
     if out_tok is None:
         out_tok = torch.zeros((S, k + 1), dtype=torch.int32, device=dev)
     if out_n is None:
@@ -108,7 +120,6 @@ def n_tokens(n: int, k: int, mode: int = MODE_STANDARD) -> int:
 def greedy_verify(logits, draft_tokens, stream=None):
     """logits [S, k+1, V], draft_tokens [S, k] -> (out_n [S], argmax [S, k+1])."""
     import torch
-    import ctypes as C
     check_tensor(logits, "logits", torch.float32)
     if logits.dim() == 2:
         logits = logits.unsqueeze(0)
@@ -119,11 +130,9 @@ def greedy_verify(logits, draft_tokens, stream=None):
     k = k1 - 1
     check_tensor(draft_tokens, "draft_tokens", torch.int32, (S, k))
     L = _lib.load()
-    nb = C.c_size_t()
-    _lib.check(L.ihip_accept_ws_bytes(S * k1, V, C.byref(nb)))
-    ws = _ws(nb.value, logits.device)
-    out_n = torch.zeros(S, dtype=torch.int32, device=logits.device)
-    am = torch.zeros((S, k1), dtype=torch.int32, device=logits.device)
+    ws = _ws(_accept_ws_bytes(S * k1, V), logits.device)
+    out_n = torch.empty(S, dtype=torch.int32, device=logits.device)  # (both written in full)
+    am = torch.empty((S, k1), dtype=torch.int32, device=logits.device)
     _lib.check(L.ihip_greedy_verify(_ptr(logits), _ptr(draft_tokens) if k else None, S, k, V, _ptr(out_n),
                                     _ptr(am), _ptr(ws), ws.numel(), _stream(stream)))
     return out_n, am
@@ -143,7 +152,6 @@ def tree_accept(target_logits, draft_logits, node_tokens, parent, temperature: f
     node, or a token outside the vocabulary), which the device reports as
     out_len = -1."""
     import torch
-    import ctypes as C
     check_tensor(target_logits, "target_logits", torch.float32, (None, None))
     n, V = target_logits.shape
     check_tensor(draft_logits, "draft_logits", torch.float32, (n, V))
@@ -151,11 +159,9 @@ def tree_accept(target_logits, draft_logits, node_tokens, parent, temperature: f
     check_tensor(parent, "parent", torch.int32, (n,))
     check_tensor(u, "u", torch.float32, (n,))
     L = _lib.load()
-    nb = C.c_size_t()
-    _lib.check(L.ihip_accept_ws_bytes(3 * n, V, C.byref(nb)))
-    ws = _ws(nb.value, target_logits.device)
-    path = torch.zeros(n, dtype=torch.int32, device=target_logits.device)
-    ln = torch.zeros(1, dtype=torch.int32, device=target_logits.device)
+    ws = _ws(_accept_ws_bytes(3 * n, V), target_logits.device)
+    path = torch.empty(n, dtype=torch.int32, device=target_logits.device)  # (written up to the length)
+    ln = torch.empty(1, dtype=torch.int32, device=target_logits.device)
     _lib.check(L.ihip_tree_accept(_ptr(target_logits), _ptr(draft_logits), _ptr(node_tokens), _ptr(parent), n, V,
                                   temperature, _ptr(u), _ptr(path), _ptr(ln), _ptr(ws), ws.numel(),
                                   _stream(stream)))
