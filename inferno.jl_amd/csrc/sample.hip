@@ -150,7 +150,7 @@ __device__ float block_max(float v, float *red) {
     __syncthreads();
     return wave_max(l < SNW ? red[l] : -__builtin_huge_valf());
 }
-__device__ int block_min_i(int v, int *red) {
+__device__ __forceinline__ int block_min_i(int v, int *red) {
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     v = wave_min_i(v);
     __syncthreads();
@@ -159,7 +159,7 @@ __device__ int block_min_i(int v, int *red) {
     return wave_min_i(l < SNW ? red[l] : INT_MAX);
 }
 // exclusive scan over the block in thread order; *total = block sum
-__device__ uint32_t block_excl_scan_u(uint32_t v, uint32_t *red, uint32_t &total) {
+__device__ __forceinline__ uint32_t block_excl_scan_u(uint32_t v, uint32_t *red, uint32_t &total) {
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     uint32_t inc = v;
     for (int o = 1; o < 64; o <<= 1) {
@@ -178,7 +178,7 @@ __device__ uint32_t block_excl_scan_u(uint32_t v, uint32_t *red, uint32_t &total
     total = tot;
     return base + inc - v;
 }
-__device__ float block_excl_scan_f(float v, float *red, float &total) {
+__device__ __forceinline__ float block_excl_scan_f(float v, float *red, float &total) {
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     float inc = v;
     for (int o = 1; o < 64; o <<= 1) {
@@ -282,7 +282,7 @@ __device__ void block_ms(float &m, float &s, float *red) {
 
 // First j in [0, n) of this thread's 4 values (slot 4t + e) with u <= the
 // inclusive prefix; the block's scan total goes to *total.
-__device__ int first_cdf_hit(const float (&v)[4], int n_here, float before, float u, float *redf, float &total) {
+__device__ __forceinline__ int first_cdf_hit(const float (&v)[4], int n_here, float before, float u, float *redf, float &total) {
     float c[4], run = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; e++) {
@@ -320,14 +320,23 @@ __device__ int block_argmax_key(uint32_t k, int i, uint32_t *s_k, int *s_i, uint
 
 // Threshold selection counted from the top (the k-th largest z, or the z
 // where the probability mass from the top reaches top_p). Pass A buckets
-// w = zmax - z linearly, 8 buckets per unit of log-probability (bucket 255:
-// the tail), which spreads real logits over many buckets; then 4 passes of
-// 8 key bits each refine inside the chosen bucket, over its few elements.
+// logits linearly, 8 buckets per unit of log-probability counted down from
+// the maximum's (bucket 255: the tail), which spreads real logits over many
+// buckets; then 4 passes of 8 key bits each refine inside the chosen bucket,
+// over its few elements. The grid is absolute (zq: floor(8 z), saturated far
+// past float's fraction), so that a part of a row may count from its own
+// maximum: bucket b there is bucket b + zq(row's) - zq(part's) of the row.
 // With MASS the buckets also carry each element's probability in 2^-40
 // fixed point (integer atomics: the same sums in any order).
-__device__ __forceinline__ uint32_t zbin(float z, float zmax) {
-    const float w = (zmax - z) * 8.0f;
-    return w < 255.0f ? (uint32_t)w : 255u;  // (-Inf and NaN: the tail)
+__device__ __forceinline__ int zq(float z) {
+    return (int)floorf(fminf(fmaxf(z * 8.0f, -0x1p29f), 0x1p29f));  // (-Inf and NaN: the lowest)
+}
+__device__ __forceinline__ uint32_t zbin(float z, float zmax) { return (uint32_t)min(zq(zmax) - zq(z), 255); }
+// z's place among the 256 equal parts of its grid cell (never falls as z
+// grows; just below 0 the difference rounds up to 1)
+__device__ __forceinline__ uint32_t zpart(float z) {
+    const float y = fminf(fmaxf(z * 8.0f, -0x1p29f), 0x1p29f);
+    return min((uint32_t)((y - floorf(y)) * 256.0f), 255u);
 }
 
 struct Select {
@@ -341,7 +350,7 @@ struct Select {
 // Wave 0 finds, over the 256 buckets (descending or ascending index), the
 // one holding the rem-th unit (~0ull in *selm when the total is short).
 template <bool MASS>
-__device__ void pick_bucket(const uint32_t *hist, const unsigned long long *mass, unsigned long long rem,
+__device__ __forceinline__ void pick_bucket(const uint32_t *hist, const unsigned long long *mass, unsigned long long rem,
                             uint32_t *sel, unsigned long long *selm, bool descending) {
     const int t = threadIdx.x;
     if (t >= 64) return;
@@ -379,6 +388,43 @@ __device__ void pick_bucket(const uint32_t *hist, const unsigned long long *mass
 // Fixed-point probability mass of z: p = exp(z - zmax) / S in units of 2^-40.
 __device__ __forceinline__ unsigned long long mass_fx(float z, float zmax, float invS) {
     return (unsigned long long)(pexp(z - zmax) * invS * 1099511627776.0f);
+}
+
+// The entries q of a thread's 4 into their buckets b (MASS: their units m);
+// uniform over the wave. A wave whose entries all take one bucket adds once:
+// on a row of equal logits its adds to one address are what a pass waits for.
+template <bool MASS>
+__device__ __forceinline__ void hist_add4(uint32_t *hist, unsigned long long *mass, const bool (&q)[4],
+                                          const uint32_t (&b)[4], const unsigned long long (&m)[4]) {
+    uint32_t b0 = 0, n = 0;
+    unsigned long long sum = 0;
+    bool same = true;
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        if (q[e]) {
+            same &= n == 0 || b[e] == b0;
+            b0 = b[e];
+            n++;
+            if (MASS) sum += m[e];
+        }
+    const uint64_t any = __ballot(n != 0);
+    if (any == 0ull) return;
+    const uint32_t bl = __builtin_amdgcn_readlane(b0, __ffsll((unsigned long long)any) - 1);
+    if (__ballot(n != 0 && (!same || b0 != bl)) == 0ull) {
+        const uint32_t nw = (uint32_t)wave_sum_u64(n);
+        if (MASS) sum = wave_sum_u64(sum);
+        if ((threadIdx.x & 63) == 0) {
+            atomicAdd(&hist[bl], nw);
+            if (MASS) atomicAdd(&mass[bl], sum);
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (q[e]) {
+                atomicAdd(&hist[b[e]], 1u);
+                if (MASS) atomicAdd(&mass[b[e]], m[e]);
+            }
+    }
 }
 
 // Passes B: the exact key inside bucket R.zb, 8 bits a pass from the top,
@@ -466,15 +512,17 @@ __device__ void refine_threshold(const float *__restrict__ row, int V, int nroun
             }
         } else {
             for_rounds(row, V, nround, T, [&](const float (&z)[4], bool in, int) {
-                if (!in) return;
+                bool q[4];
+                uint32_t b[4];
+                unsigned long long m[4];
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     const uint32_t k = okey(z[e]);
-                    if ((k & pmask) != prefix || zbin(z[e], zmax) != zb) continue;
-                    const uint32_t b = (k >> shift) & 255u;
-                    atomicAdd(&hist[b], 1u);
-                    if (MASS) atomicAdd(&mass[b], mass_fx(z[e], zmax, invS));
+                    q[e] = in && (k & pmask) == prefix && zbin(z[e], zmax) == zb;
+                    b[e] = (k >> shift) & 255u;
+                    m[e] = MASS && q[e] ? mass_fx(z[e], zmax, invS) : 0ull;
                 }
+                hist_add4<MASS>(hist, mass, q, b, m);
             });
         }
         __syncthreads();
@@ -1199,7 +1247,7 @@ struct SpreadWs {
 // puts NaN first) and its maximum is then NaN, so this holds with top-k
 // too. count (a top-k threshold, whose softmax is over the kept entries
 // only): S = 1.
-__device__ bool row_stats(const float2 *pr, int nround, float &zmax, float &S, bool count = false) {
+__device__ __forceinline__ bool row_stats(const float2 *pr, int nround, float &zmax, float &S, bool count = false) {
     const int l = threadIdx.x & 63;
     const float ninf = -__builtin_huge_valf();
     const float2 p0 = l < nround ? pr[l] : make_float2(ninf, 0.f);
@@ -1448,27 +1496,26 @@ __global__ __launch_bounds__(SNT) void argmax_draw_kernel(int V, const float2 *_
 // Spread thresholds: top-k (the k-th largest z, by count) and top-p (where
 // the probability mass from the top reaches top_p), by the one-row kernel's
 // rules (buckets below the row maximum, then the key; ties lowest index
-// first). After the statistics, one launch over the rounds:
-//  * hist[256] of the round: per bucket the count and the 2^-40 mass packed as
+// first). One launch over the rounds reads the logits once:
+//  * the round's statistics (part, as chunk_stats_kernel's);
+//  * hist[256] of the round, its buckets counted down from its own maximum
+//    m: per bucket the count and the mass sum exp(z - m) in 2^-38, packed as
 //    mass << 13 | count (one LDS atomic an entry, a copy of the array per
-//    wave). Entries that cannot be kept are left out of it: for top-k <= 256
-//    those in buckets past one whose thread maxima up to it number k (at
-//    least k entries of this round are larger); for top-p <= 1 - 1e-4 those
-//    of probability below (1 - top_p) / (2 V): the mass past the threshold
-//    element exceeds 0.99 (1 - top_p) and no entry there is above it, so it
-//    is at least 0.99 (1 - top_p) / V, ln 1.98 above the cut, more than a
-//    bucket's width: the threshold's bucket is counted in full.
+//    wave; 2^-38 so that 4096 equal entries fit: in a row's 2^-40 the entries
+//    lose at most 4 units, of their round's share, where they lost 1 each). For top-k <= 256 the buckets past one whose thread maxima up to it
+//    number k are left out (at least k entries of this round are larger);
 //  * the candidate list: (z, index) of its entries up to bucket `last`, the
 //    largest that leaves at most LIST_MAX of them, in index order.
-// Then one workgroup per row merges the histograms to the threshold's bucket,
+// Then one workgroup per row takes the row's statistics, brings the
+// histograms to the row's buckets and masses, finds the threshold's bucket,
 // takes that bucket's entries from the lists (from the row, for a round whose
 // list ends before it), finds the threshold among them, and draws: top-k
 // over the kept entries (draw_candidates), top-p by the rounds' kept masses
 // (the buckets above the threshold's, plus its kept entries), then inside
-// the round u falls in. Two launches after the statistics where there were
-// two (top-k <= 64), seven (larger) and five (top-p): 64 rows of 151936 at
-// top-p 0.9 95 -> 38 us (histograms 32 -> 14, pick + gather + select + sums +
-// draw 52 -> 15), one row at top-k 40 + top-p 28.5 -> 18.6 us.
+// the round u falls in; with at most 64 entries up to the threshold's bucket
+// one wave does all of it. Two launches where there were three (top-k <= 64),
+// eight (larger) and six (top-p): 64 rows of 151936 at top-p 0.9 95 -> 33 us,
+// one row at top-k 40 + top-p 28.6 -> 18.7 us.
 enum : int { SEL_SELECT = 0, SEL_ALL = 1, SEL_DEGEN = 2 };
 struct RowSel {
     int mode;
@@ -1482,27 +1529,29 @@ struct ListHead { int n, last; };
 
 template <bool COUNT>
 __global__ __launch_bounds__(CNT) void chunk_hist_kernel(const float *__restrict__ L, int V, float invT, int top_k,
-                                                         float top_p, SpreadWs ws) {
+                                                         SpreadWs ws) {
     __shared__ unsigned long long s_h[CNW][256];
     __shared__ uint32_t s_tm[256];
+    __shared__ float s_m[CNW], s_red[SNW];
     __shared__ int s_wn[CNW];
     const int c = blockIdx.x, row = blockIdx.y, t = threadIdx.x, wave = t >> 6, lane = t & 63;
     float z[CR][4];
     load_chunk(L + (size_t)row * V, V, c, invT, z);
-    float zmax, S;
-    const bool ok = row_stats(ws.part + (size_t)row * ws.nround, ws.nround, zmax, S, COUNT);
-    if (c == 0 && t == 0) {
-        RowSel *rs = (RowSel *)ws.rowb(row);
-        rs->mode = ok ? SEL_SELECT : SEL_DEGEN;
-        rs->zmax = zmax;
-        rs->S = S;
-    }
-    if (!ok) return;  // (the whole workgroup)
 #pragma unroll
     for (int w = 0; w < CNW; w++) s_h[w][t] = 0;
+    s_tm[t] = 0;
     const int n = V - c * SROUND;  // entries of the row from this round on
-    float zcut = -__builtin_huge_valf();  // (top-p: entries below it are left out)
-    uint32_t bcut = 255u;                 // (top-k: buckets past it are)
+    float tm = -__builtin_huge_valf();
+#pragma unroll
+    for (int r = 0; r < CR; r++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) tm = fmaxf(tm, z[r][e]);
+    float m = wave_max(tm);
+    if (lane == 0) s_m[wave] = m;
+    __syncthreads();
+    m = s_m[0];
+#pragma unroll
+    for (int w = 1; w < CNW; w++) m = fmaxf(m, s_m[w]);
     // the buckets 4 lane .. 4 lane + 3 of a wave: how many leading buckets
     // hold at most `most` entries together (every wave by itself)
     auto leading = [&](const uint32_t (&h)[4], uint32_t most) {
@@ -1518,43 +1567,47 @@ __global__ __launch_bounds__(CNT) void chunk_hist_kernel(const float *__restrict
         for (int j = 0; j < 4; j++) k += __popcll(__ballot(inc - run + cum[j] <= most));
         return k;
     };
-    if constexpr (COUNT) {
-        s_tm[t] = 0;
+    uint32_t bcut = 255u;  // (top-k: buckets past it are left out)
+    if (COUNT && top_k <= CNT) {
+        if (chunk_entry(0) < n) atomicAdd(&s_tm[zbin(tm, m)], 1u);
         __syncthreads();
-        if (top_k <= CNT) {
-            float tm = z[0][0];
-#pragma unroll
-            for (int r = 0; r < CR; r++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) tm = fmaxf(tm, z[r][e]);
-            if (chunk_entry(0) < n) atomicAdd(&s_tm[zbin(tm, zmax)], 1u);
-            __syncthreads();
-            const uint32_t h[4] = {s_tm[4 * lane], s_tm[4 * lane + 1], s_tm[4 * lane + 2], s_tm[4 * lane + 3]};
-            bcut = min(255, leading(h, (uint32_t)top_k - 1));  // (the first bucket whose prefix reaches k)
-        }
-    } else {
-        if (top_p <= 1.0f - 1e-4f) zcut = zmax + logf(0.5f * (1.0f - top_p) / (float)V * S) - 1e-3f;
-        __syncthreads();
+        const uint32_t h[4] = {s_tm[4 * lane], s_tm[4 * lane + 1], s_tm[4 * lane + 2], s_tm[4 * lane + 3]};
+        bcut = min(255, leading(h, (uint32_t)top_k - 1));  // (the first bucket whose prefix reaches k)
     }
-    const float invS = 1.0f / S;
+    // the statistics (chunk_stats_kernel's sums; top-k: only whether a NaN is there) and the histogram
     uint32_t bk[CR][4];
     bool in[CR][4];
 #pragma unroll
-    for (int r = 0; r < CR; r++)
+    for (int r = 0; r < CR; r++) {
+        float sw = 0.f;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            bk[r][e] = zbin(z[r][e], zmax);
-            in[r][e] = chunk_entry(r) + e < n && (COUNT ? bk[r][e] <= bcut : z[r][e] >= zcut);
+            const float x = z[r][e];
+            float p = 0.f;
+            if (x != x) sw = __builtin_nanf("");  // (flags the row even when m is -Inf)
+            else if (!COUNT && m > -__builtin_huge_valf()) {
+                p = pexp(x - m);
+                sw += p;
+            }
+            bk[r][e] = zbin(x, m);
+            in[r][e] = chunk_entry(r) + e < n && bk[r][e] <= bcut;
             if (in[r][e])
                 atomicAdd(&s_h[wave][bk[r][e]],
-                          COUNT ? 1ull : (mass_fx(z[r][e], zmax, invS) << CBITS) + 1ull);
+                          COUNT ? 1ull : ((unsigned long long)(p * 0x1p38f) << CBITS) + 1ull);
         }
+        sw = wave_sum(sw);
+        if (lane == 0) s_red[CR * wave + r] = sw;
+    }
     __syncthreads();
     unsigned long long hs = s_h[0][t];
 #pragma unroll
     for (int w = 1; w < CNW; w++) hs += s_h[w][t];
     uint8_t *sl = ws.slot(row, c);
     ((unsigned long long *)sl)[t] = hs;
+    if (wave == 0) {
+        const float sum = wave_sum(lane < SNW ? s_red[lane] : 0.f);
+        if (lane == 0) ws.part[(size_t)row * ws.nround + c] = make_float2(m, sum);
+    }
     s_tm[t] = (uint32_t)hs & ((1u << CBITS) - 1u);
     __syncthreads();
     const uint32_t h[4] = {s_tm[4 * lane], s_tm[4 * lane + 1], s_tm[4 * lane + 2], s_tm[4 * lane + 3]};
@@ -1567,9 +1620,9 @@ __global__ __launch_bounds__(CNT) void chunk_hist_kernel(const float *__restrict
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             in[r][e] = in[r][e] && (int)bk[r][e] <= last;
-            const uint64_t m = __ballot(in[r][e]);
-            before += __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-            all += __popcll(m);
+            const uint64_t mk = __ballot(in[r][e]);
+            before += __builtin_amdgcn_mbcnt_hi((uint32_t)(mk >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mk, 0u));
+            all += __popcll(mk);
         }
         pos[r] = wn + before;
         wn += all;
@@ -1646,6 +1699,7 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
     __shared__ unsigned long long s_mass[256];
     __shared__ uint32_t s_sel[2];
     __shared__ unsigned long long s_selm[2];
+    __shared__ int s_cnt;
     __shared__ unsigned long long s_cum[SMAX_ROUNDS];  // per round: the packed kept mass and count
     __shared__ uint32_t s_off[SMAX_ROUNDS];
     // the threshold bucket's keys, values and indices; then (top-k) the sort
@@ -1658,7 +1712,7 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
     const float *Lr = L + (size_t)row * V;
     RowSel *rs = (RowSel *)ws.rowb(row);
     // the rounds' histograms, wave w those of rounds w, w + 16, ..: buckets
-    // lane + 64 j; the first HC of them stay in registers
+    // lane + 64 j of the round; the first HC of them stay in registers
     constexpr int HC = 4;
     unsigned long long hv[HC][4];
     auto load_hist = [&](int c, unsigned long long (&h)[4]) {
@@ -1668,74 +1722,107 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
     };
 #pragma unroll
     for (int i = 0; i < HC; i++) load_hist(wave + SNW * i, hv[i]);
-    // f(round, its buckets) over this wave's rounds
-    auto rounds = [&](auto &&f) {
-#pragma unroll
-        for (int i = 0; i < HC; i++)
-            if (wave + SNW * i < nround) f(wave + SNW * i, hv[i]);
-#pragma unroll 1
-        for (int c = wave + SNW * HC; c < nround; c += SNW) {
-            unsigned long long h[4];
-            load_hist(c, h);
-            f(c, h);
-        }
-    };
-    const int mode0 = rs->mode;
-    const float zmax = rs->zmax, S = rs->S;
+    const float2 *pr = ws.part + (size_t)row * nround;
     const float ur = draw ? u[row] : 1.f;
+    float zmax, S;
+    const bool ok = row_stats(pr, nround, zmax, S, COUNT);
     if (t < 256) {
         s_hist[t] = 0;
         s_mass[t] = 0;
     }
     __syncthreads();
-    if (mode0 == SEL_DEGEN || ur != ur) {
-        if (draw && t == 0) out[row] = V - 1;
+    if (!ok || ur != ur) {
+        if (t == 0) {
+            if (draw) out[row] = V - 1;
+            else rs->mode = SEL_DEGEN;
+        }
         return;
     }
     if (!(ur > 0.f)) {  // the reference's draw returns index 1 (here 0) when r <= 0
         if (t == 0) out[row] = 0;
         return;
     }
-    {
-        uint32_t hc[4] = {0, 0, 0, 0};
-        unsigned long long hm[4] = {0, 0, 0, 0};
-        rounds([&](int, const unsigned long long (&h)[4]) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                hc[j] += (uint32_t)(h[j] & CMASK);
-                hm[j] += h[j] >> CBITS;
-            }
-        });
+    const float invS = 1.0f / S;
+    // round c's buckets moved down by this many in the row's count
+    auto shift = [&](int c) { return zq(zmax) - zq(pr[c].x); };
+    auto row_bucket = [&](int b, int sh) { return (uint32_t)min(b + min(sh, 255), 255); };
+    // a round's packed buckets with the mass in the row's 2^-40 (top-p)
+    auto to_row = [&](int c, unsigned long long (&h)[4]) {
+        if (COUNT) return;
+        const double f = (double)(pexp(pr[c].x - zmax) * invS) * 4.0;
 #pragma unroll
         for (int j = 0; j < 4; j++)
-            if (hc[j]) {
-                atomicAdd(&s_hist[lane + 64 * j], hc[j]);
-                if (!COUNT) atomicAdd(&s_mass[lane + 64 * j], hm[j]);
+            h[j] = ((unsigned long long)((double)(h[j] >> CBITS) * f) << CBITS) | (h[j] & CMASK);
+    };
+#pragma unroll
+    for (int i = 0; i < HC; i++)
+        if (wave + SNW * i < nround) to_row(wave + SNW * i, hv[i]);
+    // f(round, its shift, its buckets) over this wave's rounds
+    auto rounds = [&](auto &&f) {
+#pragma unroll
+        for (int i = 0; i < HC; i++)
+            if (wave + SNW * i < nround) f(wave + SNW * i, shift(wave + SNW * i), hv[i]);
+#pragma unroll 1
+        for (int c = wave + SNW * HC; c < nround; c += SNW) {
+            unsigned long long h[4];
+            load_hist(c, h);
+            to_row(c, h);
+            f(c, shift(c), h);
+        }
+    };
+    rounds([&](int, int sh, const unsigned long long (&h)[4]) {
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if ((h[j] & CMASK) != 0) {
+                const uint32_t b = row_bucket(lane + 64 * j, sh);
+                atomicAdd(&s_hist[b], (uint32_t)(h[j] & CMASK));
+                if (!COUNT) atomicAdd(&s_mass[b], h[j] >> CBITS);
             }
-    }
+    });
     __syncthreads();
     const float tp = fmaxf(a.top_p, 0.f) * 1099511627776.0f;
     const unsigned long long target =
         COUNT ? (unsigned long long)a.top_k : tp < 1.0f ? 1ull : (unsigned long long)ceilf(tp);
-    if constexpr (COUNT) {
-        // At most 64 entries up to the threshold's bucket (a top-k of tens):
-        // they are gathered in index order and one wave ranks, keeps and
-        // draws. (Every wave finds the bucket by itself.)
+    // the list of a round reaches row bucket zb when its `last` is at least
+    auto reach = [&](int c, uint32_t zb) { return zb == 255u ? 255 : (int)zb - shift(c); };
+    if (draw && nround <= 64) {
+        // At most 64 entries up to the threshold's bucket (a top-k of tens, a
+        // peaked row's nucleus): they are gathered in index order and one
+        // wave ranks, keeps and draws. (Every wave finds the bucket by itself.)
         const uint32_t h[4] = {s_hist[4 * lane], s_hist[4 * lane + 1], s_hist[4 * lane + 2], s_hist[4 * lane + 3]};
-        const uint32_t c0 = h[0], c1 = c0 + h[1], c2 = c1 + h[2], c3 = c2 + h[3];
-        const uint32_t ex = wave_scan_u(c3) - c3, k = (uint32_t)a.top_k;
-        const uint64_t m = __ballot(ex < k && k <= ex + c3);
-        if (m != 0ull && nround <= 64) {
-            const int f = __ffsll((unsigned long long)m) - 1;
-            const int j = ex + c0 >= k ? 0 : ex + c1 >= k ? 1 : ex + c2 >= k ? 2 : 3;
-            const uint32_t nle = __builtin_amdgcn_readlane(ex + (j == 0 ? c0 : j == 1 ? c1 : j == 2 ? c2 : c3), f);
+        uint32_t cc[4], cr = 0;
+        unsigned long long mc[4], mr = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            cr += h[j];
+            cc[j] = cr;
+            mr += COUNT ? (unsigned long long)h[j] : s_mass[4 * lane + j];
+            mc[j] = mr;
+        }
+        const uint32_t ex = wave_scan_u(cr) - cr;
+        unsigned long long mex = 0;
+        if (COUNT) {
+            mex = ex;
+        } else {
+            mex = mr;
+            for (int o = 1; o < 64; o <<= 1) {
+                const unsigned long long y = __shfl_up(mex, o);
+                if (lane >= o) mex += y;
+            }
+            mex -= mr;
+        }
+        const uint64_t hit = __ballot(mex < target && target <= mex + mr);
+        if (hit != 0ull) {
+            const int f = __ffsll((unsigned long long)hit) - 1;
+            const int j = mex + mc[0] >= target ? 0 : mex + mc[1] >= target ? 1 : mex + mc[2] >= target ? 2 : 3;
+            const uint32_t nle = __builtin_amdgcn_readlane(ex + (j == 0 ? cc[0] : j == 1 ? cc[1] : j == 2 ? cc[2] : cc[3]), f);
             const uint32_t zb = 4 * f + __builtin_amdgcn_readlane(j, f);
             if (nle <= 64u) {
-                rounds([&](int c, const unsigned long long (&x)[4]) {
+                rounds([&](int c, int sh, const unsigned long long (&x)[4]) {
                     unsigned long long v = 0;
 #pragma unroll
                     for (int i = 0; i < 4; i++)
-                        if ((uint32_t)(lane + 64 * i) <= zb) v += x[i] & CMASK;
+                        if (row_bucket(lane + 64 * i, sh) <= zb) v += x[i] & CMASK;
                     v = wave_sum_u64(v);
                     if (lane == 0) s_off[c] = (uint32_t)v;
                 });
@@ -1744,8 +1831,8 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
 #pragma unroll 1
                 for (int c = wave; c < nround; c += SNW)
                     if (__builtin_amdgcn_readlane(n, c) != 0)
-                        round_entries(ws.slot(row, c) + SLOT_LIST, Lr, V, c, invT, (int)zb, __builtin_amdgcn_readlane(off, c),
-                                      [&](float z, int) { return zbin(z, zmax) <= zb; },
+                        round_entries(ws.slot(row, c) + SLOT_LIST, Lr, V, c, invT, reach(c, zb),
+                                      __builtin_amdgcn_readlane(off, c), [&](float z, int) { return zbin(z, zmax) <= zb; },
                                       [&](uint32_t p, float z, int id) {
                                           s_cz[p & 63u] = z;  // (p < nle)
                                           s_ci[p & 63u] = id;
@@ -1756,22 +1843,42 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
                 const float z = in ? s_cz[lane] : 0.f;
                 const int id = in ? s_ci[lane] : 0;
                 const uint32_t key = in ? okey(z) : 0u;
-                uint32_t rank = 0;
-                for (uint32_t i = 0; i < nle; i++) {  // (slots in index order: equals before it rank higher)
+                // the units (entries, or mass) ahead of this entry: larger
+                // keys, and equal ones before it (slots are in index order);
+                // kept while they are short of the target
+                const unsigned long long mine = COUNT ? 1ull : mass_fx(z, zmax, invS);
+                unsigned long long ahead = 0;
+                for (uint32_t i = 0; i < nle; i++) {
                     const uint32_t ki = __builtin_amdgcn_readlane(key, i);
-                    rank += ki > key || (ki == key && i < (uint32_t)lane);
+                    const uint32_t mhi = __builtin_amdgcn_readlane((uint32_t)(mine >> 32), i);  // (int: not widened as is)
+                    const uint32_t mlo = __builtin_amdgcn_readlane((uint32_t)mine, i);
+                    const unsigned long long mi = ((unsigned long long)mhi << 32) | mlo;
+                    if (ki > key || (ki == key && i < (uint32_t)lane)) ahead += mi;
                 }
-                const bool keep = in && rank < k;
-                const uint64_t km = __ballot(keep);
-                const uint32_t p = __builtin_amdgcn_mbcnt_hi((uint32_t)(km >> 32),
-                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)km, 0u));
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                if (keep) {
-                    s_cz[p] = z;
-                    s_ci[p] = id;
+                const bool keep = in && ahead < target;
+                if constexpr (COUNT) {
+                    const uint64_t km = __ballot(keep);
+                    const uint32_t p = __builtin_amdgcn_mbcnt_hi((uint32_t)(km >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo((uint32_t)km, 0u));
+                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                    if (keep) {
+                        s_cz[p] = z;
+                        s_ci[p] = id;
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                    draw_candidates_wave(__popcll(km), a, ur, V, s_ci, s_cz, (int *)s_ck, out + row);
+                } else {
+                    unsigned long long cum = keep ? mine : 0ull;
+                    for (int o = 1; o < 64; o <<= 1) {
+                        const unsigned long long y = __shfl_up(cum, o);
+                        if (lane >= o) cum += y;
+                    }
+                    const double goal = (double)ur * (double)__shfl(cum, 63);
+                    const uint64_t got = __ballot(keep && goal <= (double)cum);
+                    const int g = got ? __ffsll((unsigned long long)got) - 1 : 0;
+                    const int tok = __shfl(id, g);
+                    if (lane == 0) out[row] = got ? tok : V - 1;  // (none: u above 1)
                 }
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                draw_candidates_wave(__popcll(km), a, ur, V, s_ci, s_cz, (int *)s_ck, out + row);
                 return;
             }
         }
@@ -1788,22 +1895,26 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
     const bool gathered = nzb <= SK_MAX;
     const uint32_t zb = R.zb;
     // per round: the packed sum of the buckets above zb, and zb's count
-    rounds([&](int c, const unsigned long long (&h)[4]) {
-        unsigned long long v = 0;
+    rounds([&](int c, int sh, const unsigned long long (&h)[4]) {
+        unsigned long long v = 0, q = 0;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const uint32_t b = lane + 64 * j;
+            const uint32_t b = row_bucket(lane + 64 * j, sh);
             if (b < zb) v += h[j];
-            if (b == zb) s_off[c] = (uint32_t)(h[j] & CMASK);
+            if (b == zb) q += h[j] & CMASK;
         }
         v = wave_sum_u64(v);
-        if (lane == 0) s_cum[c] = v;
+        q = wave_sum_u64(q);
+        if (lane == 0) {
+            s_cum[c] = v;
+            s_off[c] = (uint32_t)q;
+        }
     });
     __syncthreads();
     auto entries = [&](int c, uint32_t at, auto &&keep, auto &&f) {
-        round_entries(ws.slot(row, c) + SLOT_LIST, Lr, V, c, invT, (int)zb, at, keep, f);
+        round_entries(ws.slot(row, c) + SLOT_LIST, Lr, V, c, invT, R.all ? 256 : reach(c, zb), at, keep, f);
     };
-    int tie_lim = V;
+    int tie_lim = V, npart = -1;  // (npart >= 0: the threshold's part of the bucket is what was gathered)
     if (!R.all) {
         if (gathered) {
             uint32_t tot;
@@ -1822,9 +1933,71 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
                                 }
                             });
             __syncthreads();
+        } else if (!COUNT && zb < 255u) {
+            // A flat row: the bucket's 256 parts in one pass, then the
+            // threshold's part is gathered (in any order) in a second one,
+            // in which the parts above it join their rounds' sums. (Key
+            // passes over the row, 4 and one for the sums: 64 rows of
+            // V = 151936 at sd 1, top-p 0.9: 191 us, 107 so. A top-k's
+            // flat rows keep the key passes: this code cost its other rows 2 us.)
+            if (t < 256) {
+                s_hist[t] = 0;
+                s_mass[t] = 0;
+            }
+            if (t == 0) s_cnt = 0;
+            __syncthreads();
+            for_rounds(Lr, V, nround, invT, [&](const float (&z)[4], bool in, int) {
+                bool q[4];
+                uint32_t b[4];
+                unsigned long long m[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    q[e] = in && zbin(z[e], zmax) == zb;
+                    b[e] = zpart(z[e]);
+                    m[e] = q[e] ? mass_fx(z[e], zmax, invS) : 0ull;
+                }
+                hist_add4<true>(s_hist, s_mass, q, b, m);
+            });
+            __syncthreads();
+            pick_bucket<true>(s_hist, s_mass, R.rem, s_sel, s_selm, true);
+            __syncthreads();
+            const uint32_t part = s_sel[0];
+            const unsigned long long above = s_selm[0];
+            if (above != ~0ull && s_hist[part] <= (uint32_t)SK_MAX) {  // (uniform)
+                npart = (int)s_hist[part];
+                R.rem -= above;
+                for_rounds(Lr, V, nround, invT, [&](const float (&z)[4], bool in, int r) {
+                    unsigned long long v = 0;
+                    if (in)
+#pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            if (zbin(z[e], zmax) == zb) {
+                                const uint32_t b = zpart(z[e]);
+                                if (b > part) v += (mass_fx(z[e], zmax, invS) << CBITS) + 1ull;
+                                if (b == part) {
+                                    const int p = atomicAdd(&s_cnt, 1);  // (p < npart: the predicate counted above)
+                                    s_ck[p] = okey(z[e]);
+                                    s_cz[p] = z[e];
+                                    s_ci[p] = r * SROUND + 4 * t + e;
+                                }
+                            }
+                    if (!draw) return;
+                    v = wave_sum_u64(v);
+                    if (lane == 0 && v) atomicAdd(&s_cum[r], v);
+                });
+            }
+            __syncthreads();
         }
-        refine_threshold<!COUNT>(Lr, V, nround, invT, zmax, COUNT ? 1.f : S, gathered, nzb, s_hist, s_mass, s_sel,
-                                 s_selm, s_ck, s_cz, R);
+        Select Q = R;  // (a copy: R, captured above, stays in registers)
+        refine_threshold<!COUNT>(Lr, V, nround, invT, zmax, COUNT ? 1.f : S, gathered || npart >= 0,
+                                 gathered ? nzb : npart, s_hist, s_mass, s_sel, s_selm, s_ck, s_cz, Q);
+        R = Q;
+        if (R.all) {  // (the entries' masses a rounding short of the rounds': the whole bucket is kept)
+            R.all = false;
+            R.tau = 0u;
+            R.cnt = 0;
+            R.rem = 1;
+        }
     }
     if (!R.all) {
         // ties at tau share one probability: keep the first n_eq of them
@@ -1889,34 +2062,33 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
     if (!draw) {
         if (t == 0) {
             rs->mode = all ? SEL_ALL : SEL_SELECT;
+            rs->zmax = zmax;
+            rs->S = S;
             rs->zb = zb;
             rs->tau = tau;
             rs->tie_lim = tie_lim;
         }
         return;
     }
-    if (all && zb != 256u) {  // (the refinement fell short: every entry of every bucket)
-        __syncthreads();
-        rounds([&](int c, const unsigned long long (&h)[4]) {
-            const unsigned long long v = wave_sum_u64((h[0] + h[1]) + (h[2] + h[3]));
-            if (lane == 0) s_cum[c] = v;
-        });
-    }
     // the kept entries of the threshold's bucket join their rounds' sums
     if (!all) {
-        const float invS = 1.0f / S;
-        auto add = [&](float z, uint32_t k, int j) {
-            if (k > tau || (k == tau && j < tie_lim))
-                atomicAdd(&s_cum[j / SROUND], COUNT ? 1ull : (mass_fx(z, zmax, invS) << CBITS) + 1ull);
+        auto units = [&](float z, uint32_t k, int j) {
+            return k > tau || (k == tau && j < tie_lim) ? COUNT ? 1ull : (mass_fx(z, zmax, invS) << CBITS) + 1ull : 0ull;
         };
-        if (gathered) {
-            for (int i = t; i < nzb; i += SNT) add(s_cz[i], s_ck[i], s_ci[i]);
+        if (gathered || npart >= 0) {
+            for (int i = t; i < (gathered ? nzb : npart); i += SNT) {
+                const unsigned long long v = units(s_cz[i], s_ck[i], s_ci[i]);
+                if (v) atomicAdd(&s_cum[s_ci[i] / SROUND], v);
+            }
         } else {
             for_rounds(Lr, V, nround, invT, [&](const float (&z)[4], bool in, int r) {
+                unsigned long long v = 0;
                 if (in)
 #pragma unroll
                     for (int e = 0; e < 4; e++)
-                        if (zbin(z[e], zmax) == zb) add(z[e], okey(z[e]), r * SROUND + 4 * t + e);
+                        if (zbin(z[e], zmax) == zb) v += units(z[e], okey(z[e]), r * SROUND + 4 * t + e);
+                v = wave_sum_u64(v);
+                if (lane == 0 && v) atomicAdd(&s_cum[r], v);
             });
         }
     }
@@ -1967,7 +2139,6 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
         if (t == 0) out[row] = V - 1;
         return;
     }
-    const float invS = 1.0f / S;
     const float inv = total > 0 ? (float)(1099511627776.0 / (double)total) : 1.0f;
     const float before = (float)((double)below * (total > 0 ? 1.0 / (double)total : 0.0));
     float z[4], v[4];
@@ -2065,7 +2236,7 @@ __global__ __launch_bounds__(CNT) void chunk_keptsum_kernel(const float *__restr
     float z[CR][4];
     load_chunk(L + (size_t)row * V, V, c, invT, z);
     float zmax, S;
-    if (topp) {  // (the statistics chunk_hist_kernel stored: the same bits)
+    if (topp) {  // (the statistics row_threshold_kernel stored: the same bits)
         const RowSel *rs = (const RowSel *)ws.rowb(row);
         if (rs->mode == SEL_DEGEN) return;
         zmax = rs->zmax;
@@ -2101,7 +2272,7 @@ __global__ __launch_bounds__(SNT) void keep_draw_kernel(const float *__restrict_
     const float ur = u[row];
     float zmax, S;
     bool ok;
-    if (topp) {  // (the statistics chunk_hist_kernel stored: the same bits)
+    if (topp) {  // (the statistics row_threshold_kernel stored: the same bits)
         const RowSel *rs = (const RowSel *)ws.rowb(row);
         ok = rs->mode != SEL_DEGEN;
         zmax = rs->zmax;
@@ -2212,9 +2383,8 @@ size_t sample_spread_ws(int rows, int V) {
     return rc * (sizeof(float2) + SLOT_BYTES) + (size_t)rows * ROW_BYTES;
 }
 
-// Rows spread over workgroups of one round each (chunk statistics first):
-// plain draws (T > 0, no top-k, top-p or min-p), then one workgroup per row
-// merges them, picks the round and scans it (as draft_sample_kernel's draw);
+// Rows spread over workgroups of one round each: plain draws (T > 0, no top-k,
+// top-p or min-p): chunk statistics, then one workgroup per row merges them, picks the round and scans it (as draft_sample_kernel's draw);
 // top-k up to SK_MAX (any top-p / min-p after it) and top-p: histograms and
 // candidate lists, then one workgroup per row for the threshold and the
 // draw; min-p, alone or after top-p: the chunks' kept sums per stage, then
@@ -2241,20 +2411,21 @@ hipError_t launch_sample_spread(const float *L, int rows, int V, float T, int to
     const SpreadWs W{(float2 *)w, w + rc * sizeof(float2), w + rc * (sizeof(float2) + SLOT_BYTES), nround};
     const dim3 chunks(nround, rows);
     const SampleArgs a{T, top_k, top_p, min_p};
-    chunk_stats_kernel<<<chunks, CNT, 0, st>>>(L, V, invT, W.part);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    hipError_t e;
     if (topk) {
-        chunk_hist_kernel<true><<<chunks, CNT, 0, st>>>(L, V, invT, top_k, 1.f, W);
+        chunk_hist_kernel<true><<<chunks, CNT, 0, st>>>(L, V, invT, top_k, W);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         row_threshold_kernel<true><<<rows, SNT, 0, st>>>(L, V, invT, a, true, W, u, out);
         return hipGetLastError();
     }
     if (topp) {
-        chunk_hist_kernel<false><<<chunks, CNT, 0, st>>>(L, V, invT, 0, top_p, W);
+        chunk_hist_kernel<false><<<chunks, CNT, 0, st>>>(L, V, invT, 0, W);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         row_threshold_kernel<false><<<rows, SNT, 0, st>>>(L, V, invT, a, !minp, W, u, out);
         if ((e = hipGetLastError()) != hipSuccess || !minp) return e;
+    } else {
+        chunk_stats_kernel<<<chunks, CNT, 0, st>>>(L, V, invT, W.part);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     if (!topp && !minp) {
         chunk_draw_kernel<<<rows, SNT, 0, st>>>(L, V, invT, W.part, u, out);

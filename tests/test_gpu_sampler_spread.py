@@ -1,8 +1,8 @@
 """GPU: the spread sampler's thresholds at the edges of its kernels: rounds of
 4096 logits, candidate lists of at most 336 entries a round (rows whose
 entries crowd one bucket overflow them, and a bucket of more than 4096 entries
-is refined over the row), the cuts that leave entries out of the histograms
-(top-k up to 256, top-p up to 1 - 1e-4), ties at the threshold, masked and
+is refined over the row, by parts of it first), the cut that leaves entries out
+of the histograms (top-k up to 256), ties at the threshold, masked and
 unaligned rows. Top-k tokens equal the one-workgroup kernel's; top-p and
 min-p draws equal the oracle's except where u lies within 1e-5 (the sum of
 the fp32 probabilities' relative errors) of a step of its cumulative
