@@ -492,6 +492,19 @@ __device__ __forceinline__ double chunk_sum(const double (&w)[PER], double *sh) 
     return s;
 }
 
+// The chunk's sum of a draw slot's weights: csum[slot][c].
+__device__ __forceinline__ void sum_chunk(const Decision &D, size_t slot, int step, int c,
+                                          const float *__restrict__ tgt, const float *__restrict__ drf, int k, int V,
+                                          int nchunk, double *sh, double *__restrict__ csum) {
+    if (D.kind < 0 || D.kind == 3) return;
+    const float *lt = tgt + ((size_t)step * (k + 1) + D.prow) * V;
+    const float *ld = D.kind == 1 ? drf + ((size_t)step * k + D.qrow) * V : nullptr;
+    double w[PER];
+    chunk_weights(D, lt, ld, V, c, false, w);
+    const double sw = chunk_sum(w, sh);
+    if (threadIdx.x == 0) csum[slot * nchunk + c] = sw;
+}
+
 // The decision of verify step `step` (decide_block, computed by every
 // workgroup; the first one publishes it), then csum[step][slot][c] = the
 // sum of w over chunk c (grid: x chunk, y step, z draw slot).
@@ -510,15 +523,32 @@ __global__ __launch_bounds__(NT) void decide_sum_kernel(const float *__restrict_
     const int c = blockIdx.x, step = blockIdx.y;
     decide_block(tgt, drf, draft_tok, k, V, T, u_acc, u_res, u_bonus, mode, part, nchunk, step, gridDim.y,
                  c == 0 && blockIdx.z == 0, bonus_pre, out_tok, out_n, dec, ms, s_dec);
-    const size_t slot = (size_t)step * gridDim.z + blockIdx.z;
-    const Decision D = s_dec[blockIdx.z];
-    if (D.kind < 0 || D.kind == 3) return;
-    const float *lt = tgt + ((size_t)step * (k + 1) + D.prow) * V;
-    const float *ld = D.kind == 1 ? drf + ((size_t)step * k + D.qrow) * V : nullptr;
-    double w[PER];
-    chunk_weights(D, lt, ld, V, c, false, w);
-    const double sw = chunk_sum(w, sh);
-    if (threadIdx.x == 0) csum[slot * nchunk + c] = sw;
+    sum_chunk(s_dec[blockIdx.z], (size_t)step * gridDim.z + blockIdx.z, step, c, tgt, drf, k, V, nchunk, sh, csum);
+}
+
+// The two halves as launches of their own, for more workgroups than run
+// together: the decision once a step (grid: x step), then the chunk sums
+// (decide_sum_kernel's grid), which read it.
+__global__ __launch_bounds__(NT) void decide_kernel(const float *__restrict__ tgt, const float *__restrict__ drf,
+                                                    const int32_t *__restrict__ draft_tok, int k, int V, float T,
+                                                    const float *__restrict__ u_acc,
+                                                    const float *__restrict__ u_res,
+                                                    const float *__restrict__ u_bonus, int mode,
+                                                    const MS *__restrict__ part, int nchunk,
+                                                    const int32_t *__restrict__ bonus_pre,
+                                                    int32_t *__restrict__ out_tok, int32_t *__restrict__ out_n,
+                                                    Decision *__restrict__ dec) {
+    __shared__ MS ms[DECIDE_MAX_ROWS];
+    __shared__ Decision s_dec[2];
+    decide_block(tgt, drf, draft_tok, k, V, T, u_acc, u_res, u_bonus, mode, part, nchunk, blockIdx.x, gridDim.x, true,
+                 bonus_pre, out_tok, out_n, dec, ms, s_dec);
+}
+__global__ __launch_bounds__(NT) void sum_kernel(const float *__restrict__ tgt, const float *__restrict__ drf, int k,
+                                                 int V, const Decision *__restrict__ dec, int nchunk,
+                                                 double *__restrict__ csum) {
+    __shared__ double sh[NT / 64];
+    const size_t slot = (size_t)blockIdx.y * gridDim.z + blockIdx.z;
+    sum_chunk(dec[slot], slot, blockIdx.y, blockIdx.x, tgt, drf, k, V, nchunk, sh, csum);
 }
 
 // First j with u * S <= C_j: the chunk by a prefix over the chunk sums (a
@@ -888,6 +918,16 @@ size_t spec_accept_ws(int steps, int k, int V) {
            (size_t)steps * 2 * nc * sizeof(double) + 256;
 }
 
+// With more chunk-sum workgroups than CUs the decision has a launch of its
+// own: a workgroup that decides first waits ~6 us for 2k + 1 rows' partials
+// while its place on the CU could stream a chunk. Both ways
+// measured at k = 4, V = 151936 (38 workgroups a step; a graph of 20 calls): 4
+// steps 20.1 us in one launch, 21.0 in two; 8 steps 29.5 and 26.7; 64 steps
+// 124.8 and 84.1; V = 32000 (8 a step): 32 steps 27.0 and 28.3, 64 steps 42.8
+// and 36.9. Reference mode, two slots a step: 256 workgroups 19.9 and 21.5,
+// 304 20.1 and 19.2.
+constexpr size_t SPLIT_DECIDE = 256;
+
 // ws: MS part[steps*(k+1) + steps*k][nchunk], Decision dec[steps][slots],
 // double csum[steps][slots][nchunk] (slots = draw_slots(mode)). bonus_pre
 // (nullptr: none): each step's bonus token, drawn beforehand from target row
@@ -906,8 +946,15 @@ hipError_t launch_spec_accept(const float *tgt, const float *drf, const int32_t 
                                                                       drf, Tr, V, nc, nullptr, part);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    decide_sum_kernel<<<dim3(nc, steps, nd), NT, 0, st>>>(tgt, drf, draft_tok, k, V, T, u_acc, u_res, u_bonus,
-                                                          mode, part, nc, bonus_pre, out_tok, out_n, dec, csum);
+    if ((size_t)steps * nc * nd > SPLIT_DECIDE) {
+        decide_kernel<<<steps, NT, 0, st>>>(tgt, drf, draft_tok, k, V, T, u_acc, u_res, u_bonus, mode, part, nc,
+                                            bonus_pre, out_tok, out_n, dec);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        sum_kernel<<<dim3(nc, steps, nd), NT, 0, st>>>(tgt, drf, k, V, dec, nc, csum);
+    } else {
+        decide_sum_kernel<<<dim3(nc, steps, nd), NT, 0, st>>>(tgt, drf, draft_tok, k, V, T, u_acc, u_res, u_bonus,
+                                                              mode, part, nc, bonus_pre, out_tok, out_n, dec, csum);
+    }
     if ((e = hipGetLastError()) != hipSuccess) return e;
     sample_kernel<<<dim3(steps, nd), NT, 0, st>>>(tgt, drf, k, V, dec, nc, csum, bonus_pre, out_tok);
     return hipGetLastError();

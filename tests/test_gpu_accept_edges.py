@@ -112,3 +112,29 @@ def test_tree_malformed_parent(ih, node, parent):
     L = np.zeros((64, 32), np.float32)
     with pytest.raises(ValueError):
         ih.tree_accept(_dev(L), _dev(L), _dev(np.zeros(64, np.int32)), _dev(par), 1.0, _dev(np.zeros(64, np.float32)))
+
+
+@pytest.mark.parametrize("mode,V,steps", [(0, 4 * 4096, 64), (0, 4 * 4096, 65), (0, 4 * 4096 - 7, 129),
+                                          (1, 4 * 4096, 32), (1, 4 * 4096, 33), (0, 3, 257), (1, 5000, 300)])
+@pytest.mark.parametrize("top_k", [0, 5])
+def test_batch_equals_single_steps(ih, mode, V, steps, top_k):
+    """More than 256 chunk-sum workgroups take the decision in a launch of its
+    own: the tokens of a batch on either side are those of its steps one by
+    one, also for an invalid draft id, k's edges and a pre-drawn bonus."""
+    rng = np.random.default_rng(steps * 11 + V)
+    k = 3
+    t = (2.0 * rng.standard_normal((steps, k + 1, V))).astype(np.float32)
+    d = (t[:, :k] + 0.7 * rng.standard_normal((steps, k, V))).astype(np.float32)
+    x = d.argmax(-1).astype(np.int32)
+    x[1, 1] = V  # invalid
+    u = [_dev(rng.random(s).astype(np.float32)) for s in ((steps, k), steps, steps)]
+    t, d, x = _dev(t), _dev(d), _dev(x)
+    kw = dict(mode=mode, top_k=min(top_k, V))
+    tok, n = (a.cpu().numpy() for a in ih.spec_accept(t, d, x, 0.9, *u, **kw))
+    for s in range(steps):
+        o = slice(s, s + 1)
+        tok1, n1 = (a.cpu().numpy() for a in ih.spec_accept(t[o], d[o], x[o], 0.9, *(v[o] for v in u), **kw))
+        assert n[s] == n1[0], (s, n[s], n1[0])
+        m = n[s] + 1 + (mode == 1 and n[s] == k - 1)
+        assert np.array_equal(tok[s, :m], tok1[0, :m]), (s, tok[s], tok1[0])
+    assert n[1] == -1 or n[1] == 0
