@@ -383,8 +383,9 @@ def gemm_partials(qtype: int, m: int, n: int, k: int, flags: int, ws):
 
 
 # (The sizes are functions of their numbers alone: kept, so that a call with
-# its workspace and outputs at hand asks the library once a shape.)
-@lru_cache(maxsize=4096)
+# its workspace and outputs at hand asks the library once a shape; by type
+# too, so that a float the library refuses does not meet an equal size.)
+@lru_cache(maxsize=4096, typed=True)
 def _gemm_ws_bytes(qtype: int, m: int, n: int, k: int, flags: int) -> int:
     nb = C.c_size_t()
     _lib.check(_lib.load().ihip_gemm_q_ws_bytes(qtype, m, n, k, flags, C.byref(nb)))
@@ -396,7 +397,7 @@ def gemm_ws_bytes(qtype: int, m: int, n: int, k: int, flags: int = GEMM_AUTO) ->
     return _gemm_ws_bytes(qtype, m, n, k, flags & ~(GEMM_REUSE | GEMM_DEFER | GEMM_SUM_OUT))
 
 
-@lru_cache(maxsize=4096)
+@lru_cache(maxsize=4096, typed=True)
 def packed_bytes(qtype: int, n: int, k: int) -> int:
     """Size of the packed layout of an [n x k] matrix."""
     nb = C.c_size_t()

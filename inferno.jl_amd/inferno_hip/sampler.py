@@ -17,7 +17,7 @@ from . import _lib
 from .quantized_kernels import _ptr, _stream
 
 
-@lru_cache(maxsize=4096)
+@lru_cache(maxsize=4096, typed=True)
 def sample_ws_bytes(rows: int, V: int) -> int:
     """Workspace bytes of ihip_sample_ex for rows x V."""
     nb = C.c_size_t()

@@ -28,14 +28,14 @@ def _ws(nbytes: int, device):
 
 
 # (Workspace sizes: functions of their numbers alone, asked once a shape.)
-@lru_cache(maxsize=4096)
+@lru_cache(maxsize=4096, typed=True)
 def _accept_ws_bytes(rows: int, V: int) -> int:
     nb = C.c_size_t()
     _lib.check(_lib.load().ihip_accept_ws_bytes(rows, V, C.byref(nb)))
     return int(nb.value)
 
 
-@lru_cache(maxsize=4096)
+@lru_cache(maxsize=4096, typed=True)
 def _spec_accept_ws_bytes(steps: int, k: int, V: int, top_k: int, top_p: float, min_p: float) -> int:
     nb = C.c_size_t()
     _lib.check(_lib.load().ihip_spec_accept_ex_ws_bytes(steps, k, V, top_k, top_p, min_p, C.byref(nb)))
@@ -90,7 +90,7 @@ def spec_accept(target_logits, draft_logits, draft_tokens, temperature: float, u
     check_tensor(u_res, "u_res", torch.float32, (S,))
     check_tensor(u_bonus, "u_bonus", torch.float32, (S,))
     L = _lib.load()
-    need = _spec_accept_ws_bytes(S, k, V, top_k, top_p, min_p)
+    need = _spec_accept_ws_bytes(S, k, V, top_k, float(top_p), float(min_p))
     dev = target_logits.device
     if ws is None:
         ws = _ws(need, dev)

@@ -234,3 +234,15 @@ def test_q8k_exports_report_failure():
     vals = [float(v) for v in f[:-1]]
     assert len(vals) == 5 and all(v != v for v in vals), r.stdout + r.stderr
     assert int(f[-1]) == -19
+
+
+def test_sizes_kept_by_shape_still_refuse_floats(lib):
+    """A size asked before with integers does not answer for an equal float."""
+    from inferno_hip import quantized_kernels as qk
+    from inferno_hip import sampler
+    assert qk.packed_bytes(12, 256, 256) > 0 and qk.gemm_ws_bytes(12, 1, 256, 256) > 0
+    assert sampler.sample_ws_bytes(1, 4096) > 0
+    for call in (lambda: qk.packed_bytes(12, 256.0, 256), lambda: qk.gemm_ws_bytes(12, 1, 256.0, 256),
+                 lambda: sampler.sample_ws_bytes(1, 4096.0)):
+        with pytest.raises(C.ArgumentError):
+            call()
