@@ -1502,8 +1502,9 @@ __global__ __launch_bounds__(SNT) void argmax_draw_kernel(int V, const float2 *_
 //    m: per bucket the count and the mass sum exp(z - m) in 2^-38, packed as
 //    mass << 13 | count (one LDS atomic an entry, a copy of the array per
 //    wave; 2^-38 so that 4096 equal entries fit: in a row's 2^-40 the entries
-//    lose at most 4 units, of their round's share, where they lost 1 each). For top-k <= 256 the buckets past one whose thread maxima up to it
-//    number k are left out (at least k entries of this round are larger);
+//    lose at most 4 units, of their round's share, where they lost 1 each).
+//    For top-k <= 256 the buckets past one (the cut) whose thread maxima up to
+//    it number k are left out (at least k entries of this round are larger);
 //  * the candidate list: (z, index) of its entries up to bucket `last`, the
 //    largest that leaves at most LIST_MAX of them, in index order.
 // Then one workgroup per row takes the row's statistics, brings the
@@ -1525,7 +1526,11 @@ struct RowSel {
 };
 constexpr int LIST_MAX = 336;  // entries: 16 bytes of header, z[LIST_MAX], uint16 index in the round [LIST_MAX]
 constexpr int CBITS = 13;      // count bits of a packed bucket (a round holds 4096 entries)
-struct ListHead { int n, last; };
+struct ListHead {
+    int n, last;
+    int cut;  // the round's last bucket in its histogram
+    float m;  // the round's maximum
+};
 
 template <bool COUNT>
 __global__ __launch_bounds__(CNT) void chunk_hist_kernel(const float *__restrict__ L, int V, float invT, int top_k,
@@ -1636,7 +1641,7 @@ __global__ __launch_bounds__(CNT) void chunk_hist_kernel(const float *__restrict
         total += s_wn[w];
     }
     uint8_t *ls = sl + SLOT_LIST;
-    if (t == 0) *(ListHead *)ls = ListHead{total, last};
+    if (t == 0) *(ListHead *)ls = ListHead{total, last, (int)bcut, m};
     float *lz = (float *)(ls + 16);
     uint16_t *li = (uint16_t *)(ls + 16 + 4 * LIST_MAX);
 #pragma unroll
@@ -1654,7 +1659,10 @@ __global__ __launch_bounds__(CNT) void chunk_hist_kernel(const float *__restrict
 
 // The entries of round c that `keep` takes, in index order, by one wave:
 // f(place from `at` on, z, index), from the round's list when it reaches
-// bucket zb, else from the row.
+// bucket zb, else from the row up to the round's cut: exactly entries that its
+// histogram counts. (Where the threshold's bucket is the row's last, 255,
+// entries past the cut share that bucket, and each would take a place that
+// the counts give to another round's.)
 template <class K, class F>
 __device__ __forceinline__ void round_entries(const uint8_t *ls, const float *Lr, int V, int c, float invT, int zb,
                                               uint32_t at, K &&keep, F &&f) {
@@ -1679,7 +1687,7 @@ __device__ __forceinline__ void round_entries(const uint8_t *ls, const float *Lr
             }
         }
         j += c * SROUND;
-        const bool k = i < n && keep(z, j);
+        const bool k = i < n && (list || (int)zbin(z, hd.m) <= hd.cut) && keep(z, j);
         const uint64_t m = __ballot(k);
         if (k) f(at + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u)), z, j);
         at += __popcll(m);
@@ -1926,7 +1934,7 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
                 if (c + 1 < nround ? s_off[c + 1] > s_off[c] : tot > s_off[c])
                     entries(c, s_off[c], [&](float z, int) { return zbin(z, zmax) == zb; },
                             [&](uint32_t p, float z, int j) {
-                                if (p < (uint32_t)SK_MAX) {  // (p < nzb: the counts of chunk_hist_kernel)
+                                if (p < (uint32_t)SK_MAX) {  // (p < nzb: the entries chunk_hist_kernel counted)
                                     s_ck[p] = okey(z);
                                     s_cz[p] = z;
                                     s_ci[p] = j;

@@ -2,8 +2,9 @@
 4096 logits, candidate lists of at most 336 entries a round (rows whose
 entries crowd one bucket overflow them, and a bucket of more than 4096 entries
 is refined over the row, by parts of it first), the cut that leaves entries out
-of the histograms (top-k up to 256), ties at the threshold, masked and
-unaligned rows. Top-k tokens equal the one-workgroup kernel's; top-p and
+of the histograms (top-k up to 256) with the threshold near the row's maximum
+and past the last bucket's start, ties at the threshold, masked and unaligned
+rows. Top-k tokens equal the one-workgroup kernel's; top-p and
 min-p draws equal the oracle's except where u lies within 1e-5 (the sum of
 the fp32 probabilities' relative errors) of a step of its cumulative
 distribution."""
@@ -64,6 +65,31 @@ def test_topk(ih, kind, V):
             a = ih.softmax_sample(d, u, temperature=0.8, **kw).cpu().numpy()
             b = ih.softmax_sample(d, u, temperature=0.8, spread=False, **kw).cpu().numpy()
             assert np.array_equal(a, b), (k, kw, a, b)
+
+
+@pytest.mark.parametrize("V", [4200, 5000, 6000, 8292, 17384, 50257])
+@pytest.mark.parametrize("k", [20, 40, 100, 200, 256])
+def test_topk_outlier(ih, V, k):
+    """One logit 45 above the rest (z = L / T), in the first, a middle or the
+    short last round: the threshold lies in the last bucket, which every round
+    with a cut shares, and rounds whose counted entries pass the list are read
+    from the row. The uniforms are spread over the mass below the outlier too
+    (an outlier in the last round has every other candidate before it)."""
+    rows = 24
+    rng = np.random.default_rng(V + k)
+    for sd in (0.05, 0.2, 1.0):
+        for T in (0.1, 0.3, 1.0):
+            for at in (1, V // 2, V - 100):
+                z = sd * rng.standard_normal(V)
+                z[at] = z.max() + 45.0
+                L = _dev(np.tile((T * z).astype(np.float32), (rows, 1)))
+                e = np.exp(z - z[at])
+                below = np.sort(e)[::-1][1:k].sum()  # the other candidates' mass
+                u = np.append(below * rng.random(rows - 4), [1e-30, 1e-7, 0.5, 1 - 2.0 ** -24]).astype(np.float32)
+                a = ih.softmax_sample(L, _dev(u), temperature=T, top_k=k).cpu().numpy()
+                b = ih.softmax_sample(L, _dev(u), temperature=T, top_k=k, spread=False).cpu().numpy()
+                assert np.array_equal(a, b), (sd, T, at, a, b)
+                assert b[-2] == at
 
 
 @pytest.mark.parametrize("V", SIZES)
