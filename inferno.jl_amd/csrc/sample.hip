@@ -1499,10 +1499,14 @@ __global__ __launch_bounds__(SNT) void argmax_draw_kernel(int V, const float2 *_
 // first). One launch over the rounds reads the logits once:
 //  * the round's statistics (part, as chunk_stats_kernel's);
 //  * hist[256] of the round, its buckets counted down from its own maximum
-//    m: per bucket the count and the mass sum exp(z - m) in 2^-38, packed as
-//    mass << 13 | count (one LDS atomic an entry, a copy of the array per
-//    wave; 2^-38 so that 4096 equal entries fit: in a row's 2^-40 the entries
-//    lose at most 4 units, of their round's share, where they lost 1 each).
+//    m: per bucket the count and the mass sum exp(z - m), packed as mass << 13
+//    | count (one LDS atomic an entry, a copy of the array per wave). Bucket
+//    b's mass is in units of 2^-mass_exp(b), ~2^-30 of its largest entry's,
+//    so the entries' fp32 exponentials enter exactly (but in bucket 255, the
+//    tail); the row kernel scales each bucket by a double factor to 2^-40 of
+//    the row. (In 2^-38 of m's and an fp32 factor a round, the cumulative
+//    masses were up to 1.0e-7 off against 64 bits, and 9.7e-8 with each
+//    entry's mass cut to the row's 2^-40; so at most 4.6e-8.)
 //    For top-k <= 256 the buckets past one (the cut) whose thread maxima up to
 //    it number k are left out (at least k entries of this round are larger);
 //  * the candidate list: (z, index) of its entries up to bucket `last`, the
@@ -1526,6 +1530,10 @@ struct RowSel {
 };
 constexpr int LIST_MAX = 336;  // entries: 16 bytes of header, z[LIST_MAX], uint16 index in the round [LIST_MAX]
 constexpr int CBITS = 13;      // count bits of a packed bucket (a round holds 4096 entries)
+// Entries of bucket b below m have b - 1 < 8 (m - z) < b + 1 (b < 255), so
+// exp(z - m) 2^mass_exp(b) lies in 2^29 .. 2^31 (46 / 256 is just below
+// log2(e) / 8): its 24 bits are a whole number.
+__device__ __forceinline__ int mass_exp(int b) { return (46 * b + 31 * 256 - 46) >> 8; }
 struct ListHead {
     int n, last;
     int cut;  // the round's last bucket in its histogram
@@ -1598,7 +1606,8 @@ __global__ __launch_bounds__(CNT) void chunk_hist_kernel(const float *__restrict
             in[r][e] = chunk_entry(r) + e < n && bk[r][e] <= bcut;
             if (in[r][e])
                 atomicAdd(&s_h[wave][bk[r][e]],
-                          COUNT ? 1ull : ((unsigned long long)(p * 0x1p38f) << CBITS) + 1ull);
+                          COUNT ? 1ull
+                                : ((unsigned long long)(uint32_t)__builtin_amdgcn_ldexpf(p, mass_exp(bk[r][e])) << CBITS) + 1ull);
         }
         sw = wave_sum(sw);
         if (lane == 0) s_red[CR * wave + r] = sw;
@@ -1754,17 +1763,25 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
     // round c's buckets moved down by this many in the row's count
     auto shift = [&](int c) { return zq(zmax) - zq(pr[c].x); };
     auto row_bucket = [&](int b, int sh) { return (uint32_t)min(b + min(sh, 255), 255); };
-    // a round's packed buckets with the mass in the row's 2^-40 (top-p)
-    auto to_row = [&](int c, unsigned long long (&h)[4]) {
+    // a round's packed buckets with the mass in the row's 2^-40 (top-p), f the
+    // round's factor; those of the rounds in hv by one exp, a round a lane
+    auto factor = [&](int c) {
+        return COUNT || c >= nround ? 0.0 : exp((double)pr[c].x - (double)zmax) / (double)S;
+    };
+    auto to_row = [&](double f, unsigned long long (&h)[4]) {
         if (COUNT) return;
-        const double f = (double)(pexp(pr[c].x - zmax) * invS) * 4.0;
 #pragma unroll
         for (int j = 0; j < 4; j++)
-            h[j] = ((unsigned long long)((double)(h[j] >> CBITS) * f) << CBITS) | (h[j] & CMASK);
+            h[j] = ((unsigned long long)__builtin_ldexp((double)(h[j] >> CBITS) * f, 40 - mass_exp(lane + 64 * j)) << CBITS) |
+                   (h[j] & CMASK);
     };
+    const unsigned long long fl = __builtin_bit_cast(unsigned long long, factor(wave + SNW * (lane & (HC - 1))));
 #pragma unroll
-    for (int i = 0; i < HC; i++)
-        if (wave + SNW * i < nround) to_row(wave + SNW * i, hv[i]);
+    for (int i = 0; i < HC; i++) {
+        const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)fl, i);
+        const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(fl >> 32), i);
+        to_row(__builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo), hv[i]);
+    }
     // f(round, its shift, its buckets) over this wave's rounds
     auto rounds = [&](auto &&f) {
 #pragma unroll
@@ -1774,7 +1791,7 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
         for (int c = wave + SNW * HC; c < nround; c += SNW) {
             unsigned long long h[4];
             load_hist(c, h);
-            to_row(c, h);
+            to_row(factor(c), h);
             f(c, shift(c), h);
         }
     };

@@ -115,3 +115,31 @@ def test_mass_draws(ih, kind, V, kw):
             edge = np.min(np.abs(np.cumsum(q) - kw["top_p"]))
         before = c[g - 1] if g else 0.0
         assert edge < 1e-5 or (before - 1e-5 <= us[r] <= c[g] + 1e-5), (r, g, want, us[r], before, c[g])
+
+
+@pytest.mark.parametrize("V", [4096, 12300])
+@pytest.mark.parametrize("width", [2.0, 30.0, 60.0])
+def test_mass_histograms(ih, V, width):
+    """The buckets a top-p threshold is found in, as chunk_hist_kernel leaves
+    them in the workspace (rows of 4104 bytes a round: statistics, then a slot
+    whose first 2048 bytes are uint64 buckets mass << 13 | count, the mass of
+    bucket b in 2^-x, x = 31 + floor(46 (b - 1) / 256)): each holds its entries'
+    exp(z - m) to the relative error of one fp32 exponential at |z - m| <= 32:
+    2^-20 / 32 of the difference's rounding, 2^-19 of the product's with
+    log2 e, times ln 2, log2 e's own and the hardware's last place: 3e-6."""
+    import torch
+    n = -(-V // 4096)
+    z = (width * np.random.default_rng(V).random(V)).astype(np.float32)
+    ws = torch.zeros(ih.sampler.sample_ws_bytes(1, V), dtype=torch.uint8, device="cuda")
+    ih.softmax_sample(_dev(z[None]), _dev(np.array([0.5], np.float32)), top_p=0.9, ws=ws)
+    slots = ws.cpu().numpy()[8 * n:8 * n + 4096 * n].reshape(n, 4096)
+    for c in range(n):
+        x = z[4096 * c:4096 * (c + 1)]
+        q = np.floor(x * np.float32(8)).astype(int)
+        b = np.minimum(q.max() - q, 255)
+        h = slots[c, :2048].view(np.uint64)
+        assert np.array_equal(h & np.uint64(8191), np.bincount(b, minlength=256))
+        mass = (h >> np.uint64(13)).astype(float) * 2.0 ** -(31.0 + (46 * (np.arange(256) - 1) >> 8))
+        want = np.bincount(b, weights=np.exp(x.astype(float) - float(x.max())), minlength=256)
+        live = want[:255] > 0
+        assert np.max(np.abs(mass[:255][live] / want[:255][live] - 1)) < 3e-6
