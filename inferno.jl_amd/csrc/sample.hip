@@ -332,6 +332,11 @@ __device__ __forceinline__ int zq(float z) {
     return (int)floorf(fminf(fmaxf(z * 8.0f, -0x1p29f), 0x1p29f));  // (-Inf and NaN: the lowest)
 }
 __device__ __forceinline__ uint32_t zbin(float z, float zmax) { return (uint32_t)min(zq(zmax) - zq(z), 255); }
+// The smallest z with zq(z) >= q: bucket b of a row with zq(zmax) = zqm is
+// grid_lo(zqm - b) <= z < grid_lo(zqm - b + 1) (b = 255: no lower bound).
+__device__ __forceinline__ float grid_lo(int q) {
+    return q <= -(1 << 29) ? -__builtin_huge_valf() : q > (1 << 29) ? __builtin_huge_valf() : __int2float_ru(q) * 0.125f;
+}
 // z's place among the 256 equal parts of its grid cell (never falls as z
 // grows; just below 0 the difference rounds up to 1)
 __device__ __forceinline__ uint32_t zpart(float z) {
@@ -620,7 +625,7 @@ __device__ __forceinline__ bool above_threshold(float z, int j, float zmax, uint
 // sum, a sorted slot the count of the candidates before it), without the
 // ~30 barriers of the block form (sort 21, sums and scans 2-3 each), which
 // were most of an 18 us draw of 40 candidates.
-__device__ void draw_candidates_wave(int n, const SampleArgs &a, float ur, int V, const int *s_cidx, float *s_cp,
+__device__ __forceinline__ void draw_candidates_wave(int n, const SampleArgs &a, float ur, int V, const int *s_cidx, float *s_cp,
                                      int *s_sort, int32_t *out_row) {
     const int l = threadIdx.x;
     // first_cdf_hit over slots 4 l + e of the first 16 lanes
@@ -1225,18 +1230,37 @@ __global__ __launch_bounds__(SNT) void draft_sample_kernel(const float *__restri
 // (max, sum exp(z - max))), then a slot of SLOT_BYTES per round of each row
 // (a threshold: uint64 hist[256], at SLOT_LIST the candidate list; top-p /
 // min-p: float sums at SLOT_CSUM, once the list is no longer read), then
-// ROW_BYTES per row (a threshold: the selection state).
+// ROW_BYTES per row (a threshold: the selection state, then the longer lists
+// of a row of few rounds).
 constexpr int SLOT_BYTES = 4096;
 constexpr int SLOT_LIST = 2048;
 constexpr int SLOT_CSUM = 3072;
 constexpr size_t ROW_BYTES = 256 + (size_t)SK_MAX * 12;
+constexpr int LIST_MAX = 336;  // entries of a list in its slot: (2048 - 16) / 6
 struct SpreadWs {
     float2 *part;
     uint8_t *slots, *rows;
     int nround;
+    // a round's list: 16 bytes of header, z[lmax], uint16 index in the round
+    // [lmax]; above LIST_MAX in the row's ROW_BYTES, else in the round's slot
+    int lmax;
     __device__ uint8_t *slot(int row, int c) const { return slots + ((size_t)row * nround + c) * SLOT_BYTES; }
     __device__ uint8_t *rowb(int row) const { return rows + (size_t)row * ROW_BYTES; }
+    __device__ uint8_t *list(int row, int c) const {
+        return lmax > LIST_MAX ? rowb(row) + 256 + (size_t)c * (16 + 6 * lmax) : slot(row, c) + SLOT_LIST;
+    }
 };
+// The entries of a list: LIST_MAX, or for a top-k of many entries a round
+// (twice the mean and 128; a multiple of 8, so that a header stays 8-byte
+// aligned) as many as the row's ROW_BYTES hold for each round (top-k 4000 of
+// 32000: 45 us with lists of LIST_MAX, 32 so). A row of 1 or 2 rounds is read
+// whole instead (gather_far; top-k 4000 of 8192: 31 us, 43 with lists of 4088
+// entries, a wave each).
+constexpr int list_max(int nround, int top_k) {
+    const int want = (2 * top_k / nround + 128) / 8 * 8, room = ((int)(ROW_BYTES - 256) / nround - 16) / 6 / 8 * 8;
+    const int n = want < room ? want : room;
+    return nround > 2 && n > LIST_MAX ? n : LIST_MAX;
+}
 
 // The row's softmax statistics from its rounds' partials (a fixed order: the
 // same bits in every kernel, each wave by itself: the sums of 64 rounds at a
@@ -1507,10 +1531,11 @@ __global__ __launch_bounds__(SNT) void argmax_draw_kernel(int V, const float2 *_
 //    the row. (In 2^-38 of m's and an fp32 factor a round, the cumulative
 //    masses were up to 1.0e-7 off against 64 bits, and 9.7e-8 with each
 //    entry's mass cut to the row's 2^-40; so at most 4.6e-8.)
-//    For top-k <= 256 the buckets past one (the cut) whose thread maxima up to
-//    it number k are left out (at least k entries of this round are larger);
+//    For top-k the buckets past one (the cut) whose entries up to it number k
+//    are left out (at least k entries of this round are larger; for k <= 256
+//    first those past one whose thread maxima number k, before the atomics);
 //  * the candidate list: (z, index) of its entries up to bucket `last`, the
-//    largest that leaves at most LIST_MAX of them, in index order.
+//    largest that leaves at most lmax of them, in index order.
 // Then one workgroup per row takes the row's statistics, brings the
 // histograms to the row's buckets and masses, finds the threshold's bucket,
 // takes that bucket's entries from the lists (from the row, for a round whose
@@ -1528,16 +1553,16 @@ struct RowSel {
     int tie_lim;
     float zmax, S;
 };
-constexpr int LIST_MAX = 336;  // entries: 16 bytes of header, z[LIST_MAX], uint16 index in the round [LIST_MAX]
 constexpr int CBITS = 13;      // count bits of a packed bucket (a round holds 4096 entries)
 // Entries of bucket b below m have b - 1 < 8 (m - z) < b + 1 (b < 255), so
 // exp(z - m) 2^mass_exp(b) lies in 2^29 .. 2^31 (46 / 256 is just below
 // log2(e) / 8): its 24 bits are a whole number.
 __device__ __forceinline__ int mass_exp(int b) { return (46 * b + 31 * 256 - 46) >> 8; }
 struct ListHead {
-    int n, last;
+    int n;    // entries
     int cut;  // the round's last bucket in its histogram
     float m;  // the round's maximum
+    int pad;
 };
 
 template <bool COUNT>
@@ -1616,8 +1641,6 @@ __global__ __launch_bounds__(CNT) void chunk_hist_kernel(const float *__restrict
     unsigned long long hs = s_h[0][t];
 #pragma unroll
     for (int w = 1; w < CNW; w++) hs += s_h[w][t];
-    uint8_t *sl = ws.slot(row, c);
-    ((unsigned long long *)sl)[t] = hs;
     if (wave == 0) {
         const float sum = wave_sum(lane < SNW ? s_red[lane] : 0.f);
         if (lane == 0) ws.part[(size_t)row * ws.nround + c] = make_float2(m, sum);
@@ -1625,7 +1648,13 @@ __global__ __launch_bounds__(CNT) void chunk_hist_kernel(const float *__restrict
     s_tm[t] = (uint32_t)hs & ((1u << CBITS) - 1u);
     __syncthreads();
     const uint32_t h[4] = {s_tm[4 * lane], s_tm[4 * lane + 1], s_tm[4 * lane + 2], s_tm[4 * lane + 3]};
-    const int last = leading(h, LIST_MAX) - 1;
+    int last = leading(h, ws.lmax) - 1;
+    if (COUNT) {  // (the first bucket whose prefix reaches k ends both)
+        bcut = min(bcut, (uint32_t)leading(h, (uint32_t)top_k - 1));
+        last = min(last, (int)bcut);
+        if ((uint32_t)t > bcut) hs = 0;
+    }
+    ((unsigned long long *)ws.slot(row, c))[t] = hs;
     // places in index order: (wave, group, lane, entry)
     int pos[CR], wn = 0;
 #pragma unroll
@@ -1649,16 +1678,16 @@ __global__ __launch_bounds__(CNT) void chunk_hist_kernel(const float *__restrict
         base += w < wave ? s_wn[w] : 0;
         total += s_wn[w];
     }
-    uint8_t *ls = sl + SLOT_LIST;
-    if (t == 0) *(ListHead *)ls = ListHead{total, last, (int)bcut, m};
+    uint8_t *ls = ws.list(row, c);
+    if (t == 0) *(ListHead *)ls = ListHead{total, (int)bcut, m, 0};
     float *lz = (float *)(ls + 16);
-    uint16_t *li = (uint16_t *)(ls + 16 + 4 * LIST_MAX);
+    uint16_t *li = (uint16_t *)(ls + 16 + 4 * ws.lmax);
 #pragma unroll
     for (int r = 0; r < CR; r++) {
         int q = base + pos[r];
 #pragma unroll
         for (int e = 0; e < 4; e++)
-            if (in[r][e]) {  // (total <= LIST_MAX)
+            if (in[r][e]) {  // (total <= lmax)
                 lz[q] = z[r][e];
                 li[q] = (uint16_t)(chunk_entry(r) + e);
                 q++;
@@ -1666,40 +1695,138 @@ __global__ __launch_bounds__(CNT) void chunk_hist_kernel(const float *__restrict
     }
 }
 
-// The entries of round c that `keep` takes, in index order, by one wave:
-// f(place from `at` on, z, index), from the round's list when it reaches
-// bucket zb, else from the row up to the round's cut: exactly entries that its
-// histogram counts. (Where the threshold's bucket is the row's last, 255,
-// entries past the cut share that bucket, and each would take a place that
-// the counts give to another round's.)
-template <class K, class F>
-__device__ __forceinline__ void round_entries(const uint8_t *ls, const float *Lr, int V, int c, float invT, int zb,
-                                              uint32_t at, K &&keep, F &&f) {
-    const int lane = threadIdx.x & 63;
-    const ListHead hd = *(const ListHead *)ls;
-    const bool list = zb <= hd.last;
-    const float *lz = (const float *)(ls + 16), *src = Lr + (size_t)c * SROUND;
-    const uint16_t *li = (const uint16_t *)(ls + 16 + 4 * LIST_MAX);
-    const int n = list ? hd.n : min(SROUND, V - c * SROUND);
-#pragma unroll 2
-    for (int i0 = 0; i0 < n; i0 += 64) {
-        const int i = i0 + lane;
-        float z = 0.f;
-        int j = i;
-        if (i < n) {
-            if (list) {
-                z = lz[i];
-                j = li[i];
-            } else {
-                z = src[i];
-                if (invT != 1.0f) z = z * invT;
+// The gathers: entries lo <= z < hi that also(z, index) holds for, in index
+// order, of the row's rounds c, round c's from place at(c) on: f(place, z,
+// index). gather_lists takes them from the lists of the rounds need(c) holds
+// for (the same in a wave), a wave a round, head and first entries in one
+// load round. (64 entries after 64, after the head, a gather took 7 to 11 us,
+// most of it latency; now 3 to 5. The lists of 2 or 3 rounds at a time are no
+// faster: their code is longer, and one workgroup's time here is also that of
+// fetching its code.) LONG: lists of more than LIST_MAX entries too.
+constexpr int LE = (LIST_MAX + 63) / 64;
+template <bool LONG, class N, class A, class K, class F>
+__device__ __forceinline__ void gather_lists(const SpreadWs &ws, int row, float lo, float hi, N &&need, A &&at, K &&also,
+                                             F &&f) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+#pragma unroll 1
+    for (int c = wave; c < ws.nround; c += SNW) {
+        if (!need(c)) continue;
+        const uint8_t *ls = ws.list(row, c);
+        const float *lz = (const float *)(ls + 16);
+        const uint16_t *li = (const uint16_t *)(ls + 16 + 4 * ws.lmax);
+        const int nl = ((const ListHead *)ls)->n;
+        uint32_t q = at(c);
+        int n = 1;
+#pragma unroll 1
+        for (int i0 = 0; LONG ? i0 < n : i0 == 0; i0 += 64 * LE) {
+            float z[LE];
+            int j[LE];
+#pragma unroll
+            for (int e = 0; e < LE; e++) {  // (places past n: loaded, not used)
+                const int i = min(i0 + 64 * e + lane, ws.lmax - 1);
+                z[e] = lz[i];
+                j[e] = li[i];
+            }
+            n = __builtin_amdgcn_readfirstlane(nl);
+#pragma unroll
+            for (int e = 0; e < LE; e++) {
+                if (i0 + 64 * e >= n) break;
+                const int id = c * SROUND + j[e];
+                const bool k = i0 + 64 * e + lane < n && z[e] >= lo && z[e] < hi && also(z[e], id);
+                const uint64_t m = __ballot(k);
+                if (k)
+                    f(q + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u)), z[e],
+                      id);
+                q += __popcll(m);
             }
         }
-        j += c * SROUND;
-        const bool k = i < n && (list || (int)zbin(z, hd.m) <= hd.cut) && keep(z, j);
-        const uint64_t m = __ballot(k);
-        if (k) f(at + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u)), z, j);
-        at += __popcll(m);
+    }
+}
+
+// gather_far reads the rounds whose bit is set in far (their lists end before
+// the threshold's bucket) from the row, FB at a time by the whole workgroup,
+// the next FB in flight, down to the round's cut (CUT): exactly the entries
+// that its histogram counts. (Where the threshold's bucket is the row's last,
+// 255, entries past the cut share that bucket, and each would take a place
+// that the counts give to another round's.) s_w: 2 x 64 words. (A wave a
+// round, one round of 4096 took 7 to 12 us; now 2.)
+constexpr int FB = 4;
+template <bool CUT, class A, class K, class F>
+__device__ __forceinline__ void gather_far(const SpreadWs &ws, int row, const float *__restrict__ Lr, int V, float invT,
+                                           float lo, float hi, const uint32_t *far, uint32_t *s_w, A &&at, K &&also,
+                                           F &&f) {
+    static_assert(FB * SNW == 64, "a wave scans a batch's counts");
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    auto next = [&](int c) {  // the first far round from c on (nround: none)
+        while (c < ws.nround) {
+            const uint32_t w = __builtin_amdgcn_readfirstlane(far[c >> 5]) >> (c & 31);
+            if (w != 0u) return c + __ffs(w) - 1;
+            c = (c | 31) + 1;
+        }
+        return ws.nround;
+    };
+    float x[FB][4], xl[FB];
+    int xc[FB];
+    auto load = [&](int c) {
+#pragma unroll
+        for (int b = 0; b < FB; b++) {
+            xc[b] = c = next(c);
+            xl[b] = lo;
+            if (c >= ws.nround) continue;
+            bool in;
+            load_round(Lr, V, c, invT, x[b], in);
+            if (CUT) {
+                const ListHead hd = *(const ListHead *)ws.list(row, c);
+                if (hd.cut < 255) xl[b] = fmaxf(lo, grid_lo(zq(hd.m) - hd.cut));
+            }
+            c++;
+        }
+    };
+    load(0);
+    for (int it = 0; xc[0] < ws.nround; it ^= 64) {
+        float z[FB][4], lb[FB];
+        int cb[FB];
+#pragma unroll
+        for (int b = 0; b < FB; b++) {
+            cb[b] = xc[b];
+            lb[b] = xl[b];
+#pragma unroll
+            for (int e = 0; e < 4; e++) z[b][e] = x[b][e];
+        }
+        load(cb[FB - 1] + 1);
+        bool k[FB][4];
+        uint32_t before[FB];
+#pragma unroll
+        for (int b = 0; b < FB; b++) {
+            uint32_t all = 0;
+            before[b] = 0;
+            if (cb[b] < ws.nround) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int j = cb[b] * SROUND + 4 * (int)threadIdx.x + e;
+                    k[b][e] = j < V && z[b][e] >= lb[b] && z[b][e] < hi && also(z[b][e], j);
+                    const uint64_t m = __ballot(k[b][e]);
+                    before[b] += __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                    all += __popcll(m);
+                }
+            }
+            if (lane == 0) s_w[it + SNW * b + wave] = all;
+        }
+        __syncthreads();  // (the other half of s_w is free: every wave has passed its reads)
+        const uint32_t v = s_w[it + lane];
+        uint32_t inc = v;  // the scan within a round's 16 waves
+        inc += __builtin_amdgcn_update_dpp(0, (int)inc, 0x111, 0xF, 0xF, true);
+        inc += __builtin_amdgcn_update_dpp(0, (int)inc, 0x112, 0xF, 0xF, true);
+        inc += __builtin_amdgcn_update_dpp(0, (int)inc, 0x114, 0xF, 0xF, true);
+        inc += __builtin_amdgcn_update_dpp(0, (int)inc, 0x118, 0xF, 0xF, true);
+#pragma unroll
+        for (int b = 0; b < FB; b++) {
+            if (cb[b] >= ws.nround) break;
+            uint32_t q = at(cb[b]) + __builtin_amdgcn_readlane(inc - v, SNW * b + wave) + before[b];
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (k[b][e]) f(q++, z[b][e], cb[b] * SROUND + 4 * (int)threadIdx.x + e);
+        }
     }
 }
 
@@ -1719,6 +1846,8 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
     __shared__ int s_cnt;
     __shared__ unsigned long long s_cum[SMAX_ROUNDS];  // per round: the packed kept mass and count
     __shared__ uint32_t s_off[SMAX_ROUNDS];
+    __shared__ uint32_t s_w[128];
+    __shared__ uint32_t s_far[SMAX_ROUNDS / 32];  // rounds whose list ends before the threshold's bucket
     // the threshold bucket's keys, values and indices; then (top-k) the sort
     // scratch, values and indices of the kept entries
     __shared__ uint32_t s_ck[SK_MAX];
@@ -1741,12 +1870,15 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
     for (int i = 0; i < HC; i++) load_hist(wave + SNW * i, hv[i]);
     const float2 *pr = ws.part + (size_t)row * nround;
     const float ur = draw ? u[row] : 1.f;
+    // the maxima of the rounds in hv, a round a lane
+    const float ml = pr[min(wave + SNW * (lane & (HC - 1)), nround - 1)].x;
     float zmax, S;
     const bool ok = row_stats(pr, nround, zmax, S, COUNT);
     if (t < 256) {
         s_hist[t] = 0;
         s_mass[t] = 0;
     }
+    if (t < SMAX_ROUNDS / 32) s_far[t] = 0;
     __syncthreads();
     if (!ok || ur != ur) {
         if (t == 0) {
@@ -1760,24 +1892,24 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
         return;
     }
     const float invS = 1.0f / S;
-    // round c's buckets moved down by this many in the row's count
-    auto shift = [&](int c) { return zq(zmax) - zq(pr[c].x); };
+    // a round of maximum m: its buckets' places in the row's count, and its
+    // packed buckets with the mass in the row's 2^-40 (top-p; f: the round's
+    // factor). (Shifts and factors of the rounds in hv: a round a lane.)
+    const int zqm = zq(zmax);
+    auto bucket_lo = [&](uint32_t b) { return b >= 255u ? -__builtin_huge_valf() : grid_lo(zqm - (int)b); };
     auto row_bucket = [&](int b, int sh) { return (uint32_t)min(b + min(sh, 255), 255); };
-    // a round's packed buckets with the mass in the row's 2^-40 (top-p), f the
-    // round's factor; those of the rounds in hv by one exp, a round a lane
-    auto factor = [&](int c) {
-        return COUNT || c >= nround ? 0.0 : exp((double)pr[c].x - (double)zmax) / (double)S;
-    };
+    auto factor = [&](float m) { return COUNT ? 0.0 : exp((double)m - (double)zmax) / (double)S; };
     auto to_row = [&](double f, unsigned long long (&h)[4]) {
-        if (COUNT) return;
 #pragma unroll
         for (int j = 0; j < 4; j++)
             h[j] = ((unsigned long long)__builtin_ldexp((double)(h[j] >> CBITS) * f, 40 - mass_exp(lane + 64 * j)) << CBITS) |
                    (h[j] & CMASK);
     };
-    const unsigned long long fl = __builtin_bit_cast(unsigned long long, factor(wave + SNW * (lane & (HC - 1))));
+    const int shl = zqm - zq(ml);
+    const unsigned long long fl = __builtin_bit_cast(unsigned long long, factor(ml));
 #pragma unroll
     for (int i = 0; i < HC; i++) {
+        if (COUNT || wave + SNW * i >= nround) break;
         const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)fl, i);
         const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(fl >> 32), i);
         to_row(__builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo), hv[i]);
@@ -1786,13 +1918,14 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
     auto rounds = [&](auto &&f) {
 #pragma unroll
         for (int i = 0; i < HC; i++)
-            if (wave + SNW * i < nround) f(wave + SNW * i, shift(wave + SNW * i), hv[i]);
+            if (wave + SNW * i < nround) f(wave + SNW * i, __builtin_amdgcn_readlane(shl, i), hv[i]);
 #pragma unroll 1
         for (int c = wave + SNW * HC; c < nround; c += SNW) {
             unsigned long long h[4];
             load_hist(c, h);
-            to_row(factor(c), h);
-            f(c, shift(c), h);
+            const float m = pr[c].x;
+            if (!COUNT) to_row(factor(m), h);
+            f(c, zqm - zq(m), h);
         }
     };
     rounds([&](int, int sh, const unsigned long long (&h)[4]) {
@@ -1808,8 +1941,6 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
     const float tp = fmaxf(a.top_p, 0.f) * 1099511627776.0f;
     const unsigned long long target =
         COUNT ? (unsigned long long)a.top_k : tp < 1.0f ? 1ull : (unsigned long long)ceilf(tp);
-    // the list of a round reaches row bucket zb when its `last` is at least
-    auto reach = [&](int c, uint32_t zb) { return zb == 255u ? 255 : (int)zb - shift(c); };
     if (draw && nround <= 64) {
         // At most 64 entries up to the threshold's bucket (a top-k of tens, a
         // peaked row's nucleus): they are gathered in index order and one
@@ -1853,15 +1984,13 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
                 });
                 __syncthreads();
                 const uint32_t n = lane < nround ? s_off[lane] : 0u, off = wave_scan_u(n) - n;
-#pragma unroll 1
-                for (int c = wave; c < nround; c += SNW)
-                    if (__builtin_amdgcn_readlane(n, c) != 0)
-                        round_entries(ws.slot(row, c) + SLOT_LIST, Lr, V, c, invT, reach(c, zb),
-                                      __builtin_amdgcn_readlane(off, c), [&](float z, int) { return zbin(z, zmax) <= zb; },
-                                      [&](uint32_t p, float z, int id) {
-                                          s_cz[p & 63u] = z;  // (p < nle)
-                                          s_ci[p & 63u] = id;
-                                      });
+                gather_lists<false>(  // (at most 64 entries a round: every list reaches; top-k <= 64: none is long)
+                    ws, row, bucket_lo(zb), __builtin_huge_valf(), [&](int c) { return __builtin_amdgcn_readlane(n, c) != 0; },
+                    [&](int c) { return (uint32_t)__builtin_amdgcn_readlane(off, c); }, [&](float, int) { return true; },
+                    [&](uint32_t p, float z, int id) {
+                        s_cz[p & 63u] = z;  // (p < nle)
+                        s_ci[p & 63u] = id;
+                    });
                 __syncthreads();
                 if (wave != 0) return;
                 const bool in = (uint32_t)lane < nle;
@@ -1933,11 +2062,16 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
         if (lane == 0) {
             s_cum[c] = v;
             s_off[c] = (uint32_t)q;
+            if ((v & CMASK) + q > (unsigned long long)ws.lmax) atomicOr(&s_far[c >> 5], 1u << (c & 31));
         }
     });
     __syncthreads();
-    auto entries = [&](int c, uint32_t at, auto &&keep, auto &&f) {
-        round_entries(ws.slot(row, c) + SLOT_LIST, Lr, V, c, invT, R.all ? 256 : reach(c, zb), at, keep, f);
+    // from the bucket's lower bound to hi, each round at its s_off
+    auto gather = [&](float hi, auto &&need, auto &&also, auto &&f) {
+        auto at = [&](int c) { return s_off[c]; };
+        gather_lists<COUNT>(ws, row, bucket_lo(zb), hi, [&](int c) { return ((s_far[c >> 5] >> (c & 31)) & 1u) == 0u && need(c); },
+                     at, also, f);
+        gather_far<COUNT>(ws, row, Lr, V, invT, bucket_lo(zb), hi, s_far, s_w, at, also, f);
     };
     int tie_lim = V, npart = -1;  // (npart >= 0: the threshold's part of the bucket is what was gathered)
     if (!R.all) {
@@ -1947,16 +2081,17 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
             const uint32_t off = block_excl_scan_u(cnt, s_redu, tot);
             if (t < nround) s_off[t] = off;
             __syncthreads();
-            for (int c = wave; c < nround; c += SNW)
-                if (c + 1 < nround ? s_off[c + 1] > s_off[c] : tot > s_off[c])
-                    entries(c, s_off[c], [&](float z, int) { return zbin(z, zmax) == zb; },
-                            [&](uint32_t p, float z, int j) {
-                                if (p < (uint32_t)SK_MAX) {  // (p < nzb: the entries chunk_hist_kernel counted)
-                                    s_ck[p] = okey(z);
-                                    s_cz[p] = z;
-                                    s_ci[p] = j;
-                                }
-                            });
+            gather(
+                grid_lo(zqm - (int)zb + 1),
+                [&](int c) { return c + 1 < nround ? s_off[c + 1] > s_off[c] : tot > s_off[c]; },
+                [&](float, int) { return true; },
+                [&](uint32_t p, float z, int j) {
+                    if (p < (uint32_t)SK_MAX) {  // (p < nzb: the entries chunk_hist_kernel counted)
+                        s_ck[p] = okey(z);
+                        s_cz[p] = z;
+                        s_ci[p] = j;
+                    }
+                });
             __syncthreads();
         } else if (!COUNT && zb < 255u) {
             // A flat row: the bucket's 256 parts in one pass, then the
@@ -2124,16 +2259,18 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
         const uint32_t off = block_excl_scan_u(cnt, s_redu, n);
         for (int i = t; i < nround; i += SNT) s_off[i] = off;
         __syncthreads();  // (and the gathered bucket is no longer read)
-        for (int c = wave; c < nround; c += SNW)
-            if ((s_cum[c] & CMASK) != 0)
-                entries(c, s_off[c],
-                        [&](float z, int j) { return all || above_threshold(z, j, zmax, zb, tau, tie_lim); },
-                        [&](uint32_t p, float z, int j) {
-                            if (p < (uint32_t)SK_MAX) {
-                                s_cz[p] = z;
-                                s_ci[p] = j;
-                            }
-                        });
+        gather(
+            __builtin_huge_valf(), [&](int c) { return (s_cum[c] & CMASK) != 0; },
+            [&](float z, int j) {  // (a bucket above zb has the larger keys)
+                const uint32_t k = okey(z);
+                return k > tau || (k == tau && j < tie_lim);
+            },
+            [&](uint32_t p, float z, int j) {
+                if (p < (uint32_t)SK_MAX) {
+                    s_cz[p] = z;
+                    s_ci[p] = j;
+                }
+            });
         __syncthreads();
         draw_candidates(min((int)n, SK_MAX), a, ur, V, s_ci, s_cz, (int *)s_ck, s_redf, s_redi, out + row);
         return;
@@ -2433,7 +2570,7 @@ hipError_t launch_sample_spread(const float *L, int rows, int V, float T, int to
     const float invT = 1.0f / T;
     const size_t rc = (size_t)rows * nround;
     uint8_t *w = (uint8_t *)ws;
-    const SpreadWs W{(float2 *)w, w + rc * sizeof(float2), w + rc * (sizeof(float2) + SLOT_BYTES), nround};
+    const SpreadWs W{(float2 *)w, w + rc * sizeof(float2), w + rc * (sizeof(float2) + SLOT_BYTES), nround, list_max(nround, topk ? top_k : 0)};
     const dim3 chunks(nround, rows);
     const SampleArgs a{T, top_k, top_p, min_p};
     hipError_t e;

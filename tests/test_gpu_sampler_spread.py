@@ -1,5 +1,5 @@
 """GPU: the spread sampler's thresholds at the edges of its kernels: rounds of
-4096 logits, candidate lists of at most 336 entries a round (rows whose
+4096 logits, candidate lists of 336 entries a round and longer (rows whose
 entries crowd one bucket overflow them, and a bucket of more than 4096 entries
 is refined over the row, by parts of it first), the cut that leaves entries out
 of the histograms (top-k up to 256) with the threshold near the row's maximum
@@ -30,13 +30,17 @@ def ih():
 
 
 def _rows(kind, rows, V):
-    rng = np.random.default_rng(V * 7 + KINDS.index(kind))
+    rng = np.random.default_rng(V * 7 + (KINDS + ["wide", "crowded"]).index(kind))
     if kind == "lm":  # a language model's: falling with the rank
         L = -1.6 * np.log(rng.permuted(np.tile(np.arange(1.0, V + 1), (rows, 1)), axis=1)) + 0.5 * rng.standard_normal((rows, V))
     elif kind == "flat":  # one bucket holds every entry, values distinct
         L = 0.01 * rng.standard_normal((rows, V))
     elif kind == "few":  # ties everywhere
         L = rng.integers(0, 6, (rows, V)) * 0.5
+    elif kind in ("wide", "crowded"):  # a threshold past the lists, in every round or in the first
+        L = 2.0 * rng.standard_normal((rows, V))
+        if kind == "crowded":
+            L = -np.sort(-L, axis=1)
     else:
         L = 3.0 * rng.standard_normal((rows, V))
         if kind == "masked":
@@ -92,12 +96,38 @@ def test_topk_outlier(ih, V, k):
                 assert b[-2] == at
 
 
+@pytest.mark.parametrize("V", [4097, 9000, 12289, 30000, 98305])
+@pytest.mark.parametrize("at", ["first", "last", "spread"])
+def test_topk_crowded(ih, V, at):
+    """Candidates crowded into the first or the last rounds, or even: a round
+    passes any list (its entries come from the row, beside rounds with none),
+    the lists of rows of 3 rounds and more are the longer ones for the larger
+    k, and the last round is short. Values distinct and in runs of equals."""
+    rows = 6
+    rng = np.random.default_rng(V)
+    z = 2.0 * rng.standard_normal((rows, V))
+    if at != "spread":
+        z = np.sort(z, axis=1) if at == "last" else -np.sort(-z, axis=1)
+    z[3:] = np.round(4 * z[3:]) / 4
+    d = _dev(z.astype(np.float32))
+    for k in (90, 300, 700, 1500, 3000, 4096):
+        if k < V:
+            u = _dev(rng.random(rows).astype(np.float32))
+            a = ih.softmax_sample(d, u, top_k=k).cpu().numpy()
+            b = ih.softmax_sample(d, u, top_k=k, spread=False).cpu().numpy()
+            assert np.array_equal(a, b), (k, a, b)
+
+
 @pytest.mark.parametrize("V", SIZES)
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("kw", [dict(top_p=0.5), dict(top_p=0.95), dict(top_p=0.99985), dict(top_p=0.99995),
                                 dict(top_p=0.9, min_p=0.05), dict(min_p=0.05), dict(), dict(top_p=1e-6)],
                          ids=lambda kw: ",".join(f"{k}={v}" for k, v in kw.items()) or "plain")
 def test_mass_draws(ih, kind, V, kw):
+    _mass_draws(ih, kind, V, kw)
+
+
+def _mass_draws(ih, kind, V, kw):
     rows = 8
     L = _rows(kind, rows, V)
     us = np.random.default_rng(V + 1).random(rows).astype(np.float32)
@@ -115,6 +145,14 @@ def test_mass_draws(ih, kind, V, kw):
             edge = np.min(np.abs(np.cumsum(q) - kw["top_p"]))
         before = c[g - 1] if g else 0.0
         assert edge < 1e-5 or (before - 1e-5 <= us[r] <= c[g] + 1e-5), (r, g, want, us[r], before, c[g])
+
+
+@pytest.mark.parametrize("V", [4095, 9000, 30000, 70001])
+@pytest.mark.parametrize("kind", ["wide", "crowded"])
+@pytest.mark.parametrize("kw", [dict(top_p=0.9), dict(top_p=0.9, min_p=0.02)],
+                         ids=lambda kw: ",".join(f"{k}={v}" for k, v in kw.items()))
+def test_mass_draws_past_lists(ih, kind, V, kw):
+    _mass_draws(ih, kind, V, kw)
 
 
 @pytest.mark.parametrize("V", [4096, 12300])
