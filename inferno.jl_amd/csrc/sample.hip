@@ -1228,8 +1228,8 @@ __global__ __launch_bounds__(SNT) void draft_sample_kernel(const float *__restri
 
 // Workspace of the spread draws: float2 part[rows][nround] (each round's
 // (max, sum exp(z - max))), then a slot of SLOT_BYTES per round of each row
-// (a threshold: uint64 hist[256], at SLOT_LIST the candidate list; top-p /
-// min-p: float sums at SLOT_CSUM, once the list is no longer read), then
+// (a threshold: uint64 hist[256], at SLOT_LIST the candidate list; min-p: a
+// float sum at SLOT_CSUM, once the list is no longer read), then
 // ROW_BYTES per row (a threshold: the selection state, then the longer lists
 // of a row of few rounds).
 constexpr int SLOT_BYTES = 4096;
@@ -1551,7 +1551,7 @@ struct RowSel {
     int mode;
     uint32_t zb, tau;
     int tie_lim;
-    float zmax, S;
+    float zmax, S, inv1;  // inv1: 1 / the nucleus mass
 };
 constexpr int CBITS = 13;      // count bits of a packed bucket (a round holds 4096 entries)
 // Entries of bucket b below m have b - 1 < 8 (m - z) < b + 1 (b < 255), so
@@ -1831,7 +1831,8 @@ __device__ __forceinline__ void gather_far(const SpreadWs &ws, int row, const fl
 }
 
 // Row blockIdx.x: its threshold and (draw) its token; otherwise the selection
-// is left in the row's RowSel for the kept sums of a min-p after it.
+// and the nucleus mass are left in the row's RowSel for a min-p after it. (A
+// launch over the rounds for that mass: 5 us of 46 for one row.)
 template <bool COUNT>
 __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restrict__ L, int V, float invT,
                                                             SampleArgs a, bool draw, SpreadWs ws,
@@ -2141,7 +2142,6 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
                                     s_ci[p] = r * SROUND + 4 * t + e;
                                 }
                             }
-                    if (!draw) return;
                     v = wave_sum_u64(v);
                     if (lane == 0 && v) atomicAdd(&s_cum[r], v);
                 });
@@ -2219,17 +2219,6 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
     }
     const bool all = R.all;
     const uint32_t tau = R.tau;
-    if (!draw) {
-        if (t == 0) {
-            rs->mode = all ? SEL_ALL : SEL_SELECT;
-            rs->zmax = zmax;
-            rs->S = S;
-            rs->zb = zb;
-            rs->tau = tau;
-            rs->tie_lim = tie_lim;
-        }
-        return;
-    }
     // the kept entries of the threshold's bucket join their rounds' sums
     if (!all) {
         auto units = [&](float z, uint32_t k, int j) {
@@ -2287,6 +2276,18 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
     };
     unsigned long long total = 0;
     for (int b = 0; b < nround; b += 64) total = __shfl(cum64(b, total), 63);
+    if (!draw) {
+        if (t == 0) {
+            rs->mode = all ? SEL_ALL : SEL_SELECT;
+            rs->zmax = zmax;
+            rs->S = S;
+            rs->zb = zb;
+            rs->tau = tau;
+            rs->tie_lim = tie_lim;
+            rs->inv1 = total > 0 ? (float)(1099511627776.0 / (double)total) : 1.0f;
+        }
+        return;
+    }
     const double goal = (double)ur * (double)total;
     unsigned long long below = 0;
     int rr = -1;
@@ -2328,86 +2329,75 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
     }
 }
 
-// An entry's probability through the cuts: p = exp(z - zmax) / S, 0 when
-// top-p (the row's selection) drops it; with min-p, renormalized by the
-// nucleus mass (inv1 = 1 / its total; 1 without top-p) and 0 below
-// thr = inv1 / S * min_p (the largest probability times min_p).
+// An entry's probability through the cuts of a min-p draw: p = exp(z - zmax)
+// / S; after top-p 0 for what its selection drops, else divided by the nucleus
+// mass (inv1 = 1 / it; 1 without top-p); 0 below thr = inv1 / S * min_p (the
+// largest probability times min_p).
 struct Keep {
-    bool topp, minp, all;
+    bool topp, all;
     uint32_t zb, tau;
     int tie_lim;
     float zmax, invS, inv1, thr;
     __device__ float p1(float z, int j) const {
         if (topp && !(all || above_threshold(z, j, zmax, zb, tau, tie_lim))) return 0.f;
         float p = pexp(z - zmax) * invS;
-        if (minp) {
-            if (topp) p = p * inv1;
-            if (p < thr) return 0.f;
-        }
-        return p;
+        if (topp) p = p * inv1;
+        return p < thr ? 0.f : p;
     }
 };
 
-// 1 / the sum of the row's chunk values at byte `off` of their slots (a
-// fixed order, as row_stats), or 1 when it is not positive.
-__device__ float kept_inv(const SpreadWs &ws, int row, int off) {
+// 1 / the sum of the row's chunk values at SLOT_CSUM of their slots (a fixed
+// order, as row_stats), or 1 when it is not positive.
+__device__ float kept_inv(const SpreadWs &ws, int row) {
     const int l = threadIdx.x & 63;
     float acc = 0.f;
     for (int v = 0; 64 * v < ws.nround; v++) {
         const int i = 64 * v + l;
-        const float sv = wave_sum(i < ws.nround ? *(const float *)(ws.slot(row, i) + off) : 0.f);
+        const float sv = wave_sum(i < ws.nround ? *(const float *)(ws.slot(row, i) + SLOT_CSUM) : 0.f);
         if (l == v) acc = sv;
     }
     const float total = wave_sum(acc);
     return total > 0.f ? 1.0f / total : 1.0f;
 }
 
-// false for a row without finite statistics (no draw); minp: the min-p
-// stage (its inv1 from the top-p stage's kept sums).
-__device__ bool load_keep(const SpreadWs &ws, int row, bool topp, bool minp, float min_p, float zmax, float S,
-                          Keep &k) {
+// The row's statistics (after top-p those row_threshold_kernel stored) and
+// cuts; false for a row without finite ones (no draw).
+__device__ __forceinline__ bool load_keep(const SpreadWs &ws, int row, bool topp, float min_p, Keep &k) {
+    float S;
     k.topp = topp;
-    k.minp = minp;
-    k.zmax = zmax;
-    k.invS = 1.0f / S;
-    k.all = false;
-    k.zb = 256u;
-    k.tau = 0u;
-    k.tie_lim = 0;
-    k.inv1 = 1.0f;
     if (topp) {
         const RowSel *rs = (const RowSel *)ws.rowb(row);
         if (rs->mode == SEL_DEGEN) return false;
+        k.zmax = rs->zmax;
+        S = rs->S;
         k.all = rs->mode == SEL_ALL;
         k.zb = rs->zb;
         k.tau = rs->tau;
         k.tie_lim = rs->tie_lim;
-        if (minp) k.inv1 = kept_inv(ws, row, SLOT_CSUM);
+        k.inv1 = rs->inv1;
+    } else {
+        if (!row_stats(ws.part + (size_t)row * ws.nround, ws.nround, k.zmax, S)) return false;
+        k.all = false;
+        k.zb = 256u;
+        k.tau = 0u;
+        k.tie_lim = 0;
+        k.inv1 = 1.0f;
     }
+    k.invS = 1.0f / S;
     k.thr = k.invS * k.inv1 * min_p;
     return true;
 }
 
-// Chunk blockIdx.x of row blockIdx.y: the sum of its kept probabilities,
-// stage 0 (top-p) at SLOT_CSUM, stage 1 (min-p, after top-p if topp) at
-// SLOT_CSUM + 4.
+// Chunk blockIdx.x of row blockIdx.y: the sum of its kept probabilities at
+// SLOT_CSUM.
 __global__ __launch_bounds__(CNT) void chunk_keptsum_kernel(const float *__restrict__ L, int V, float invT, bool topp,
-                                                            int stage, float min_p, SpreadWs ws) {
+                                                            float min_p, SpreadWs ws) {
     __shared__ float s_red[SNW];
     const int c = blockIdx.x, row = blockIdx.y, t = threadIdx.x;
     float z[CR][4];
     load_chunk(L + (size_t)row * V, V, c, invT, z);
-    float zmax, S;
-    if (topp) {  // (the statistics row_threshold_kernel stored: the same bits)
-        const RowSel *rs = (const RowSel *)ws.rowb(row);
-        if (rs->mode == SEL_DEGEN) return;
-        zmax = rs->zmax;
-        S = rs->S;
-    } else if (!row_stats(ws.part + (size_t)row * ws.nround, ws.nround, zmax, S)) {
-        return;
-    }
     Keep keep;
-    if (!load_keep(ws, row, topp, stage == 1, min_p, zmax, S, keep)) return;
+    if (!load_keep(ws, row, topp, min_p, keep)) return;
     float sum[CR];
 #pragma unroll
     for (int r = 0; r < CR; r++) {
@@ -2416,15 +2406,14 @@ __global__ __launch_bounds__(CNT) void chunk_keptsum_kernel(const float *__restr
         for (int e = 0; e < 4; e++) sum[r] += keep.p1(z[r][e], c * SROUND + chunk_entry(r) + e);
     }
     const float total = chunk_sum(sum, s_red);
-    if (t == 0) *(float *)(ws.slot(row, c) + SLOT_CSUM + 4 * stage) = total;
+    if (t == 0) *(float *)(ws.slot(row, c) + SLOT_CSUM) = total;
 }
 
-// Row blockIdx.x: the kept mass of the last stage, each round's share of
-// it, the round holding u, then the index inside it (as chunk_draw_kernel
-// over the kept entries).
+// Row blockIdx.x: the kept mass, each round's share of it, the round holding
+// u, then the index inside it (as chunk_draw_kernel over the kept entries).
 __global__ __launch_bounds__(SNT) void keep_draw_kernel(const float *__restrict__ L, int V, float invT, bool topp,
-                                                        bool minp, float min_p, SpreadWs ws,
-                                                        const float *__restrict__ u, int32_t *__restrict__ out) {
+                                                        float min_p, SpreadWs ws, const float *__restrict__ u,
+                                                        int32_t *__restrict__ out) {
     __shared__ float s_redf[2 * SNW];
     __shared__ int s_redi[SNW];
     __shared__ float s_round[SMAX_ROUNDS];
@@ -2432,18 +2421,8 @@ __global__ __launch_bounds__(SNT) void keep_draw_kernel(const float *__restrict_
     __shared__ int s_rr;
     const int row = blockIdx.x, t = threadIdx.x, nround = ws.nround;
     const float ur = u[row];
-    float zmax, S;
-    bool ok;
-    if (topp) {  // (the statistics row_threshold_kernel stored: the same bits)
-        const RowSel *rs = (const RowSel *)ws.rowb(row);
-        ok = rs->mode != SEL_DEGEN;
-        zmax = rs->zmax;
-        S = rs->S;
-    } else {
-        ok = row_stats(ws.part + (size_t)row * nround, nround, zmax, S);
-    }
     Keep keep;
-    if (!ok || !load_keep(ws, row, topp, minp, min_p, zmax, S, keep) || ur != ur) {
+    if (!load_keep(ws, row, topp, min_p, keep) || ur != ur) {
         if (t == 0) out[row] = V - 1;
         return;
     }
@@ -2451,9 +2430,8 @@ __global__ __launch_bounds__(SNT) void keep_draw_kernel(const float *__restrict_
         if (t == 0) out[row] = 0;
         return;
     }
-    const int off = SLOT_CSUM + (minp ? 4 : 0);
-    const float inv = kept_inv(ws, row, off);
-    for (int i = t; i < nround; i += SNT) s_round[i] = *(const float *)(ws.slot(row, i) + off) * inv;
+    const float inv = kept_inv(ws, row);
+    for (int i = t; i < nround; i += SNT) s_round[i] = *(const float *)(ws.slot(row, i) + SLOT_CSUM) * inv;
     __syncthreads();
     if (t == 0) {
         float cum = 0.f;
@@ -2549,7 +2527,7 @@ size_t sample_spread_ws(int rows, int V) {
 // top-p or min-p): chunk statistics, then one workgroup per row merges them, picks the round and scans it (as draft_sample_kernel's draw);
 // top-k up to SK_MAX (any top-p / min-p after it) and top-p: histograms and
 // candidate lists, then one workgroup per row for the threshold and the
-// draw; min-p, alone or after top-p: the chunks' kept sums per stage, then
+// draw; min-p, alone or after top-p: the chunks' kept sums, then
 // the draw; T = 0: each chunk's argmax, then the row's. Rows over more than
 // SMAX_ROUNDS rounds, and a larger top-k, run draft_sample_kernel.
 // ws: sample_spread_ws bytes (8-byte aligned).
@@ -2593,11 +2571,9 @@ hipError_t launch_sample_spread(const float *L, int rows, int V, float T, int to
         chunk_draw_kernel<<<rows, SNT, 0, st>>>(L, V, invT, W.part, u, out);
         return hipGetLastError();
     }
-    for (int stage = topp ? 0 : 1; stage <= 1; stage++) {
-        chunk_keptsum_kernel<<<chunks, CNT, 0, st>>>(L, V, invT, topp, stage, min_p, W);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-    }
-    keep_draw_kernel<<<rows, SNT, 0, st>>>(L, V, invT, topp, minp, min_p, W, u, out);
+    chunk_keptsum_kernel<<<chunks, CNT, 0, st>>>(L, V, invT, topp, min_p, W);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    keep_draw_kernel<<<rows, SNT, 0, st>>>(L, V, invT, topp, min_p, W, u, out);
     return hipGetLastError();
 }
 
