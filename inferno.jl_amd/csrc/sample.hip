@@ -322,7 +322,7 @@ __device__ int block_argmax_key(uint32_t k, int i, uint32_t *s_k, int *s_i, uint
 // where the probability mass from the top reaches top_p). Pass A buckets
 // logits linearly, 8 buckets per unit of log-probability counted down from
 // the maximum's (bucket 255: the tail), which spreads real logits over many
-// buckets; then 4 passes of 8 key bits each refine inside the chosen bucket,
+// buckets; then passes of 8 key bits each refine inside the chosen bucket,
 // over its few elements. The grid is absolute (zq: floor(8 z), saturated far
 // past float's fraction), so that a part of a row may count from its own
 // maximum: bucket b there is bucket b + zq(row's) - zq(part's) of the row.
@@ -432,76 +432,91 @@ __device__ __forceinline__ void hist_add4(uint32_t *hist, unsigned long long *ma
     }
 }
 
-// Passes B: the exact key inside bucket R.zb, 8 bits a pass from the top,
-// R.rem units still to reach; over the nzb gathered keys and values (ck, cz)
-// when gathered, else over the row. R.tau, R.rem and R.cnt on return, or
-// R.all when (MASS) truncated masses fall just short of the target. At most
-// SPAIR_MAX gathered elements are ranked directly instead: tau is the key
-// whose larger keys hold less than R.rem units and which with its equals
-// reaches it (integer sums: the key the passes would find; MASS: the
-// elements' units staged in mass[], which holds 256).
+// The threshold inside bucket R.zb, R.rem units still to reach: R.tau, R.rem
+// and R.cnt on return, or R.all when (MASS) truncated masses fall just short of
+// the target.
+// At most SPAIR_MAX gathered elements (keys ck, values cz) are ranked
+// directly: tau is the key whose larger keys hold less than R.rem units and
+// which with its equals reaches it (integer sums: the key the passes below
+// would find; MASS: the elements' units staged in mass[], which holds 256).
 constexpr int SPAIR_MAX = 128;
 template <bool MASS>
-__device__ void refine_threshold(const float *__restrict__ row, int V, int nround, float T, float zmax, float S,
-                                 bool gathered, int nzb, uint32_t *hist, unsigned long long *mass, uint32_t *sel,
-                                 unsigned long long *selm, const uint32_t *ck, const float *cz, Select &R) {
+__device__ void refine_pairs(float zmax, float S, int nzb, unsigned long long *mass, uint32_t *sel,
+                             unsigned long long *selm, const uint32_t *ck, const float *cz, Select &R) {
+    const int t = threadIdx.x;
+    const float invS = 1.0f / S;
+    if (t == 0) {
+        sel[0] = 0u;
+        sel[1] = 0u;
+        selm[0] = ~0ull;
+    }
+    if (MASS && t < nzb) mass[t] = mass_fx(cz[t], zmax, invS);  // (each element's units, once)
+    __syncthreads();
+    // element i = t / P compared with every P-th element from t % P (at
+    // most 16 comparisons a lane); the P lanes of an element (adjacent,
+    // in one wave) then add their sums
+    int lp = 0;
+    while (nzb > (16 << lp)) lp++;  // (nzb <= SPAIR_MAX: P = 2^lp <= 8)
+    const int P = 1 << lp, i = t >> lp;
+    const bool act = i < nzb;
+    const uint32_t ki = act ? ck[i] : 0u;
+    unsigned long long gt = 0, eq = 0;
+    uint32_t ne = 0;
+    if (act)
+        for (int j = t & (P - 1); j < nzb; j += P) {
+            const uint32_t kj = ck[j];
+            const unsigned long long mj = MASS ? mass[j] : 1ull;
+            if (kj > ki) {
+                gt += mj;
+            } else if (kj == ki) {
+                eq += mj;
+                ne++;
+            }
+        }
+    for (int o = 1; o < P; o <<= 1) {
+        gt += __shfl_xor(gt, o);
+        eq += __shfl_xor(eq, o);
+        ne += __shfl_xor(ne, o);
+    }
+    if (act && (t & (P - 1)) == 0 && gt < R.rem && R.rem <= gt + eq) {  // (every element of key ki writes the same)
+        sel[0] = ki;
+        sel[1] = ne;
+        selm[0] = gt;
+    }
+    __syncthreads();
+    const uint32_t tau = sel[0], cnt = sel[1];
+    const unsigned long long above = selm[0];
+    __syncthreads();
+    if (above == ~0ull) {
+        R.all = true;
+        return;
+    }
+    R.rem -= above;
+    R.cnt = cnt;
+    R.tau = tau;
+}
+
+// Passes B: the key 8 bits a pass from the highest that differs in the bucket
+// (a cell of the grid: 14 to 20 bits for |z| of 1 to 64, not 32), over the
+// nzb gathered elements when gathered, until one is left, else over the row.
+// (Four passes of the whole key: 611 elements 9.4 us, 3000 14.7; now 5 and 8.)
+template <bool MASS>
+__device__ __noinline__ void refine_passes(const float *__restrict__ row, int V, int nround, float T, float zmax, float S,
+                                           bool gathered, int nzb, uint32_t *hist, unsigned long long *mass,
+                                           uint32_t *sel, unsigned long long *selm, const uint32_t *ck, const float *cz,
+                                           Select &R) {
     const int t = threadIdx.x;
     const uint32_t zb = R.zb;
     const float invS = 1.0f / S;
-    if (gathered && nzb <= SPAIR_MAX) {
-        if (t == 0) {
-            sel[0] = 0u;
-            sel[1] = 0u;
-            selm[0] = ~0ull;
-        }
-        if (MASS && t < nzb) mass[t] = mass_fx(cz[t], zmax, invS);  // (each element's units, once)
-        __syncthreads();
-        // element i = t / P compared with every P-th element from t % P (at
-        // most 16 comparisons a lane); the P lanes of an element (adjacent,
-        // in one wave) then add their sums
-        int lp = 0;
-        while (nzb > (16 << lp)) lp++;  // (nzb <= SPAIR_MAX: P = 2^lp <= 8)
-        const int P = 1 << lp, i = t >> lp;
-        const bool act = i < nzb;
-        const uint32_t ki = act ? ck[i] : 0u;
-        unsigned long long gt = 0, eq = 0;
-        uint32_t ne = 0;
-        if (act)
-            for (int j = t & (P - 1); j < nzb; j += P) {
-                const uint32_t kj = ck[j];
-                const unsigned long long mj = MASS ? mass[j] : 1ull;
-                if (kj > ki) {
-                    gt += mj;
-                } else if (kj == ki) {
-                    eq += mj;
-                    ne++;
-                }
-            }
-        for (int o = 1; o < P; o <<= 1) {
-            gt += __shfl_xor(gt, o);
-            eq += __shfl_xor(eq, o);
-            ne += __shfl_xor(ne, o);
-        }
-        if (act && (t & (P - 1)) == 0 && gt < R.rem && R.rem <= gt + eq) {  // (every element of key ki writes the same)
-            sel[0] = ki;
-            sel[1] = ne;
-            selm[0] = gt;
-        }
-        __syncthreads();
-        const uint32_t tau = sel[0], cnt = sel[1];
-        const unsigned long long above = selm[0];
-        __syncthreads();
-        if (above == ~0ull) {
-            R.all = true;
-            return;
-        }
-        R.rem -= above;
-        R.cnt = cnt;
-        R.tau = tau;
-        return;
-    }
-    uint32_t prefix = 0, pmask = 0;
-    for (int shift = 24; shift >= 0; shift -= 8) {
+    // the bits below the highest in which two keys of the bucket can differ
+    const int zqm = zq(zmax);
+    const float lo = zb >= 255u ? -__builtin_huge_valf() : grid_lo(zqm - (int)zb);
+    const uint32_t khi = okey(grid_lo(zqm - (int)zb + 1)) - 1u, klo = okey(lo == 0.f ? -0.f : lo);
+    const int nbits = max(32 - __clz(klo ^ khi), 1);
+    uint32_t pmask = nbits == 32 ? 0u : ~0u << nbits, prefix = khi & pmask;
+    for (int top = nbits; top > 0; top -= 8) {
+        const int shift = max(top - 8, 0);
+        const uint32_t digit = (1u << (top - shift)) - 1u;
         if (t < 256) {
             hist[t] = 0;
             if (MASS) mass[t] = 0;
@@ -511,7 +526,7 @@ __device__ void refine_threshold(const float *__restrict__ row, int V, int nroun
             for (int i = t; i < nzb; i += SNT) {
                 const uint32_t k = ck[i];
                 if ((k & pmask) != prefix) continue;
-                const uint32_t b = (k >> shift) & 255u;
+                const uint32_t b = (k >> shift) & digit;
                 atomicAdd(&hist[b], 1u);
                 if (MASS) atomicAdd(&mass[b], mass_fx(cz[i], zmax, invS));
             }
@@ -524,7 +539,7 @@ __device__ void refine_threshold(const float *__restrict__ row, int V, int nroun
                 for (int e = 0; e < 4; e++) {
                     const uint32_t k = okey(z[e]);
                     q[e] = in && (k & pmask) == prefix && zbin(z[e], zmax) == zb;
-                    b[e] = (k >> shift) & 255u;
+                    b[e] = (k >> shift) & digit;
                     m[e] = MASS && q[e] ? mass_fx(z[e], zmax, invS) : 0ull;
                 }
                 hist_add4<MASS>(hist, mass, q, b, m);
@@ -543,10 +558,27 @@ __device__ void refine_threshold(const float *__restrict__ row, int V, int nroun
         }
         R.rem -= above;
         prefix |= b << shift;
-        pmask |= 255u << shift;
+        pmask |= digit << shift;
         R.cnt = cb;
+        if (gathered && cb == 1u && shift > 0) {  // (one element: its key)
+            for (int i = t; i < nzb; i += SNT)
+                if ((ck[i] & pmask) == prefix) sel[0] = ck[i];
+            __syncthreads();
+            prefix = sel[0];
+            __syncthreads();
+            break;
+        }
     }
     R.tau = prefix;
+}
+
+template <bool MASS>
+__device__ __forceinline__ void refine_threshold(const float *__restrict__ row, int V, int nround, float T, float zmax,
+                                                 float S, bool gathered, int nzb, uint32_t *hist,
+                                                 unsigned long long *mass, uint32_t *sel, unsigned long long *selm,
+                                                 const uint32_t *ck, const float *cz, Select &R) {
+    if (gathered && nzb <= SPAIR_MAX) refine_pairs<MASS>(zmax, S, nzb, mass, sel, selm, ck, cz, R);
+    else refine_passes<MASS>(row, V, nround, T, zmax, S, gathered, nzb, hist, mass, sel, selm, ck, cz, R);
 }
 
 // The B passes read only the elements of bucket zb: when it holds at most
