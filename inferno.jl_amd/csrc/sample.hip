@@ -130,6 +130,7 @@ __device__ __forceinline__ uint32_t wave_scan_u(uint32_t v) {
     v += __builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, true);  // row_bcast:31 into rows 2, 3
     return v;
 }
+__device__ __forceinline__ uint32_t wave_sum_u(uint32_t v) { return __builtin_amdgcn_readlane(wave_scan_u(v), 63); }
 __device__ __forceinline__ int wave_min_i(int v) {
     for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o));
     return v;
@@ -1584,7 +1585,9 @@ struct RowSel {
     uint32_t zb, tau;
     int tie_lim;
     float zmax, S, inv1;  // inv1: 1 / the nucleus mass
+    uint32_t arrived;     // workgroups whose part of a gather has landed
 };
+constexpr int ROW_PART = 256;  // then (a split gather) the bucket's entries: value, index
 constexpr int CBITS = 13;      // count bits of a packed bucket (a round holds 4096 entries)
 // Entries of bucket b below m have b - 1 < 8 (m - z) < b + 1 (b < 255), so
 // exp(z - m) 2^mass_exp(b) lies in 2^29 .. 2^31 (46 / 256 is just below
@@ -1711,7 +1714,10 @@ __global__ __launch_bounds__(CNT) void chunk_hist_kernel(const float *__restrict
         total += s_wn[w];
     }
     uint8_t *ls = ws.list(row, c);
-    if (t == 0) *(ListHead *)ls = ListHead{total, (int)bcut, m, 0};
+    if (t == 0) {
+        *(ListHead *)ls = ListHead{total, (int)bcut, m, 0};
+        if (!COUNT && c == 0) ((RowSel *)ws.rowb(row))->arrived = 0;
+    }
     float *lz = (float *)(ls + 16);
     uint16_t *li = (uint16_t *)(ls + 16 + 4 * ws.lmax);
 #pragma unroll
@@ -1776,24 +1782,29 @@ __device__ __forceinline__ void gather_lists(const SpreadWs &ws, int row, float 
 }
 
 // gather_far reads the rounds whose bit is set in far (their lists end before
-// the threshold's bucket) from the row, FB at a time by the whole workgroup,
+// the threshold's bucket) and that mine(c) holds for from the row, FB at a time by the whole workgroup,
 // the next FB in flight, down to the round's cut (CUT): exactly the entries
 // that its histogram counts. (Where the threshold's bucket is the row's last,
 // 255, entries past the cut share that bucket, and each would take a place
 // that the counts give to another round's.) s_w: 2 x 64 words. (A wave a
 // round, one round of 4096 took 7 to 12 us; now 2.)
 constexpr int FB = 4;
-template <bool CUT, class A, class K, class F>
+template <bool CUT, class M, class A, class K, class F>
 __device__ __forceinline__ void gather_far(const SpreadWs &ws, int row, const float *__restrict__ Lr, int V, float invT,
-                                           float lo, float hi, const uint32_t *far, uint32_t *s_w, A &&at, K &&also,
-                                           F &&f) {
+                                           float lo, float hi, const uint32_t *far, uint32_t *s_w, M &&mine, A &&at,
+                                           K &&also, F &&f) {
     static_assert(FB * SNW == 64, "a wave scans a batch's counts");
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    auto next = [&](int c) {  // the first far round from c on (nround: none)
+    auto next = [&](int c) {  // the first far round that is mine from c on (nround: none)
         while (c < ws.nround) {
             const uint32_t w = __builtin_amdgcn_readfirstlane(far[c >> 5]) >> (c & 31);
-            if (w != 0u) return c + __ffs(w) - 1;
-            c = (c | 31) + 1;
+            if (w == 0u) {
+                c = (c | 31) + 1;
+                continue;
+            }
+            c += __ffs(w) - 1;
+            if (mine(c)) return c;
+            c++;
         }
         return ws.nround;
     };
@@ -1865,7 +1876,13 @@ __device__ __forceinline__ void gather_far(const SpreadWs &ws, int row, const fl
 // Row blockIdx.x: its threshold and (draw) its token; otherwise the selection
 // and the nucleus mass are left in the row's RowSel for a min-p after it. (A
 // launch over the rounds for that mass: 5 us of 46 for one row.)
-template <bool COUNT>
+// SPLIT (top-p; grid y, 0: 1): every workgroup of a row finds the bucket by
+// itself; where more than FB rounds' lists end before it, each takes the rounds
+// c with c mod SPLIT = blockIdx.y into the row's workspace, and the last to
+// arrive goes on with the bucket (no workgroup waits for another); everywhere
+// else only the first goes on. The entries and the count cross XCDs through
+// device-scope atomics, a wave's stores done before its workgroup counts in.
+template <bool COUNT, int SPLIT>
 __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restrict__ L, int V, float invT,
                                                             SampleArgs a, bool draw, SpreadWs ws,
                                                             const float *__restrict__ u, int32_t *__restrict__ out) {
@@ -1888,6 +1905,7 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
     __shared__ int s_ci[SK_MAX];
     constexpr unsigned long long CMASK = (1ull << CBITS) - 1ull;
     const int row = blockIdx.x, t = threadIdx.x, wave = t >> 6, lane = t & 63, nround = ws.nround;
+    const int g = SPLIT > 0 ? (int)blockIdx.y : 0;
     const float *Lr = L + (size_t)row * V;
     RowSel *rs = (RowSel *)ws.rowb(row);
     // the rounds' histograms, wave w those of rounds w, w + 16, ..: buckets
@@ -1914,14 +1932,14 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
     if (t < SMAX_ROUNDS / 32) s_far[t] = 0;
     __syncthreads();
     if (!ok || ur != ur) {
-        if (t == 0) {
+        if (t == 0 && g == 0) {
             if (draw) out[row] = V - 1;
             else rs->mode = SEL_DEGEN;
         }
         return;
     }
     if (!(ur > 0.f)) {  // the reference's draw returns index 1 (here 0) when r <= 0
-        if (t == 0) out[row] = 0;
+        if (t == 0 && g == 0) out[row] = 0;
         return;
     }
     const float invS = 1.0f / S;
@@ -2007,13 +2025,14 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
             const uint32_t nle = __builtin_amdgcn_readlane(ex + (j == 0 ? cc[0] : j == 1 ? cc[1] : j == 2 ? cc[2] : cc[3]), f);
             const uint32_t zb = 4 * f + __builtin_amdgcn_readlane(j, f);
             if (nle <= 64u) {
+                if (SPLIT > 0 && g != 0) return;
                 rounds([&](int c, int sh, const unsigned long long (&x)[4]) {
-                    unsigned long long v = 0;
+                    uint32_t v = 0;
 #pragma unroll
                     for (int i = 0; i < 4; i++)
-                        if (row_bucket(lane + 64 * i, sh) <= zb) v += x[i] & CMASK;
-                    v = wave_sum_u64(v);
-                    if (lane == 0) s_off[c] = (uint32_t)v;
+                        if (row_bucket(lane + 64 * i, sh) <= zb) v += (uint32_t)x[i] & (uint32_t)CMASK;
+                    v = wave_sum_u(v);
+                    if (lane == 0) s_off[c] = v;
                 });
                 __syncthreads();
                 const uint32_t n = lane < nround ? s_off[lane] : 0u, off = wave_scan_u(n) - n;
@@ -2083,28 +2102,36 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
     const uint32_t zb = R.zb;
     // per round: the packed sum of the buckets above zb, and zb's count
     rounds([&](int c, int sh, const unsigned long long (&h)[4]) {
-        unsigned long long v = 0, q = 0;
+        unsigned long long v = 0;
+        uint32_t q = 0;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const uint32_t b = row_bucket(lane + 64 * j, sh);
             if (b < zb) v += h[j];
-            if (b == zb) q += h[j] & CMASK;
+            if (b == zb) q += (uint32_t)h[j] & (uint32_t)CMASK;
         }
-        v = wave_sum_u64(v);
-        q = wave_sum_u64(q);
+        v = COUNT ? wave_sum_u((uint32_t)v) : wave_sum_u64(v);
+        q = wave_sum_u(q);
         if (lane == 0) {
             s_cum[c] = v;
-            s_off[c] = (uint32_t)q;
+            s_off[c] = q;
             if ((v & CMASK) + q > (unsigned long long)ws.lmax) atomicOr(&s_far[c >> 5], 1u << (c & 31));
         }
     });
     __syncthreads();
+    bool split = false;
+    if (SPLIT > 0) {
+        if (gathered && !R.all) split = wave_sum_u64(lane < SMAX_ROUNDS / 32 ? __popc(s_far[lane]) : 0) > (unsigned long long)FB;
+        if (!split && g != 0) return;
+    }
     // from the bucket's lower bound to hi, each round at its s_off
     auto gather = [&](float hi, auto &&need, auto &&also, auto &&f) {
         auto at = [&](int c) { return s_off[c]; };
-        gather_lists<COUNT>(ws, row, bucket_lo(zb), hi, [&](int c) { return ((s_far[c >> 5] >> (c & 31)) & 1u) == 0u && need(c); },
-                     at, also, f);
-        gather_far<COUNT>(ws, row, Lr, V, invT, bucket_lo(zb), hi, s_far, s_w, at, also, f);
+        auto mine = [&](int c) { return SPLIT == 0 || !split || (c & (SPLIT - 1)) == g; };
+        gather_lists<COUNT>(ws, row, bucket_lo(zb), hi,
+                            [&](int c) { return ((s_far[c >> 5] >> (c & 31)) & 1u) == 0u && need(c) && mine(c); }, at, also,
+                            f);
+        gather_far<COUNT>(ws, row, Lr, V, invT, bucket_lo(zb), hi, s_far, s_w, mine, at, also, f);
     };
     int tie_lim = V, npart = -1;  // (npart >= 0: the threshold's part of the bucket is what was gathered)
     if (!R.all) {
@@ -2114,17 +2141,37 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
             const uint32_t off = block_excl_scan_u(cnt, s_redu, tot);
             if (t < nround) s_off[t] = off;
             __syncthreads();
+            unsigned long long *gp = (unsigned long long *)(ws.rowb(row) + ROW_PART);
+            auto keep1 = [&](uint32_t p, float z, int j) {
+                s_ck[p] = okey(z);
+                s_cz[p] = z;
+                s_ci[p] = j;
+            };
             gather(
                 grid_lo(zqm - (int)zb + 1),
                 [&](int c) { return c + 1 < nround ? s_off[c + 1] > s_off[c] : tot > s_off[c]; },
                 [&](float, int) { return true; },
                 [&](uint32_t p, float z, int j) {
-                    if (p < (uint32_t)SK_MAX) {  // (p < nzb: the entries chunk_hist_kernel counted)
-                        s_ck[p] = okey(z);
-                        s_cz[p] = z;
-                        s_ci[p] = j;
-                    }
+                    if (p >= (uint32_t)SK_MAX) return;  // (p < nzb: the entries chunk_hist_kernel counted)
+                    if (SPLIT > 0 && split)
+                        __hip_atomic_store(gp + p, ((unsigned long long)(uint32_t)j << 32) | __float_as_uint(z), __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+                    else
+                        keep1(p, z, j);
                 });
+            if (SPLIT > 0 && split) {
+                wait_stores_done();
+                __syncthreads();
+                if (t == 0)
+                    s_cnt = (int)__hip_atomic_fetch_add(&rs->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __syncthreads();
+                if (s_cnt != SPLIT - 1) return;
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+                for (int i = t; i < nzb; i += SNT) {
+                    const unsigned long long v = __hip_atomic_load(gp + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    keep1(i, __uint_as_float((uint32_t)v), (int)(v >> 32));
+                }
+            }
             __syncthreads();
         } else if (!COUNT && zb < 255u) {
             // A flat row: the bucket's 256 parts in one pass, then the
@@ -2159,6 +2206,7 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
             if (above != ~0ull && s_hist[part] <= (uint32_t)SK_MAX) {  // (uniform)
                 npart = (int)s_hist[part];
                 R.rem -= above;
+                unsigned long long vt = 0;
                 for_rounds(Lr, V, nround, invT, [&](const float (&z)[4], bool in, int r) {
                     unsigned long long v = 0;
                     if (in)
@@ -2174,9 +2222,15 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
                                     s_ci[p] = r * SROUND + 4 * t + e;
                                 }
                             }
+                    if (!draw) {  // (the row's sum alone is asked for)
+                        vt += v >> CBITS;
+                        return;
+                    }
                     v = wave_sum_u64(v);
                     if (lane == 0 && v) atomicAdd(&s_cum[r], v);
                 });
+                vt = wave_sum_u64(vt);
+                if (lane == 0 && vt) atomicAdd(&s_cum[0], vt << CBITS);
             }
             __syncthreads();
         }
@@ -2550,6 +2604,13 @@ hipError_t launch_sample(const float *L, int rows, int V, float T, int top_k, fl
     return hipGetLastError();
 }
 
+// A top-p's rows have 16 or 8 workgroups each while those of all rows are at
+// most as many as there are CUs. V = 151936, top-p 0.9, by 1 workgroup and so:
+// Gaussian sd 2 (38 rounds past their lists) 1 row 68.4 and 43.7 us, 16 rows
+// 73.0 and 47.5, 32 rows 77.7 and 58.8; a language model's logits (no round past
+// its list) 14.5 and 14.6, 19.0 and 19.2, 21.0 and 21.4 (by 16: 27.5).
+constexpr int SPLIT_CU = 256;
+
 size_t sample_spread_ws(int rows, int V) {
     const size_t rc = (size_t)rows * ((V + SROUND - 1) / SROUND);
     return rc * (sizeof(float2) + SLOT_BYTES) + (size_t)rows * ROW_BYTES;
@@ -2587,13 +2648,18 @@ hipError_t launch_sample_spread(const float *L, int rows, int V, float T, int to
     if (topk) {
         chunk_hist_kernel<true><<<chunks, CNT, 0, st>>>(L, V, invT, top_k, W);
         if ((e = hipGetLastError()) != hipSuccess) return e;
-        row_threshold_kernel<true><<<rows, SNT, 0, st>>>(L, V, invT, a, true, W, u, out);
+        row_threshold_kernel<true, 0><<<rows, SNT, 0, st>>>(L, V, invT, a, true, W, u, out);
         return hipGetLastError();
     }
     if (topp) {
         chunk_hist_kernel<false><<<chunks, CNT, 0, st>>>(L, V, invT, 0, W);
         if ((e = hipGetLastError()) != hipSuccess) return e;
-        row_threshold_kernel<false><<<rows, SNT, 0, st>>>(L, V, invT, a, !minp, W, u, out);
+        if (rows <= SPLIT_CU / 16)
+            row_threshold_kernel<false, 16><<<dim3(rows, 16), SNT, 0, st>>>(L, V, invT, a, !minp, W, u, out);
+        else if (rows <= SPLIT_CU / 8)
+            row_threshold_kernel<false, 8><<<dim3(rows, 8), SNT, 0, st>>>(L, V, invT, a, !minp, W, u, out);
+        else
+            row_threshold_kernel<false, 0><<<rows, SNT, 0, st>>>(L, V, invT, a, !minp, W, u, out);
         if ((e = hipGetLastError()) != hipSuccess || !minp) return e;
     } else {
         chunk_stats_kernel<<<chunks, CNT, 0, st>>>(L, V, invT, W.part);

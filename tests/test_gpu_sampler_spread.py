@@ -127,8 +127,7 @@ def test_mass_draws(ih, kind, V, kw):
     _mass_draws(ih, kind, V, kw)
 
 
-def _mass_draws(ih, kind, V, kw):
-    rows = 8
+def _mass_draws(ih, kind, V, kw, rows=8):
     L = _rows(kind, rows, V)
     us = np.random.default_rng(V + 1).random(rows).astype(np.float32)
     us[0] = np.float32(1 - 2.0 ** -24)
@@ -151,8 +150,9 @@ def _mass_draws(ih, kind, V, kw):
 @pytest.mark.parametrize("kind", ["wide", "crowded"])
 @pytest.mark.parametrize("kw", [dict(top_p=0.9), dict(top_p=0.9, min_p=0.02)],
                          ids=lambda kw: ",".join(f"{k}={v}" for k, v in kw.items()))
-def test_mass_draws_past_lists(ih, kind, V, kw):
-    _mass_draws(ih, kind, V, kw)
+@pytest.mark.parametrize("rows", [8, 32, 40])  # 16, 8 and 1 workgroups a row
+def test_mass_draws_past_lists(ih, kind, V, kw, rows):
+    _mass_draws(ih, kind, V, kw, rows)
 
 
 @pytest.mark.parametrize("V", [4096, 12300])
