@@ -6,6 +6,7 @@ gfx950 device, calls raise.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import os
 
 PKG_ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -16,6 +17,32 @@ IHIP_OK = 0
 STATUS_NAMES = {0: "OK", -14: "EFAULT", -22: "EINVAL", -12: "ENOMEM", -19: "ENODEV", -1000: "EHIP"}
 
 _vp, _i, _i64, _u64, _f, _sz = C.c_void_p, C.c_int, C.c_int64, C.c_uint64, C.c_float, C.c_size_t
+
+
+class _NotPlain(Exception):
+    pass
+
+
+def kept_by_size(f):
+    """f, a size the library works out from plain numbers, asked once for each
+    ints and floats (typed: an equal float does not answer for an int). Other
+    arguments (an array, a tensor, whose value may change) go to f each time."""
+    plain = {int, float}
+
+    @functools.lru_cache(maxsize=4096, typed=True)
+    def kept(*args):
+        if not plain.issuperset(map(type, args)):
+            raise _NotPlain  # (what raises is not kept)
+        return f(*args)
+
+    @functools.wraps(f)
+    def call(*args, **kw):
+        try:
+            return kept(*args, **kw)
+        except (_NotPlain, TypeError):  # (TypeError: unhashable, or a keyword)
+            return f(*args, **kw)
+    return call
+
 
 # name -> (restype, argtypes)
 SIGNATURES = {

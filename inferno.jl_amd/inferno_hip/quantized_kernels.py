@@ -15,7 +15,6 @@ all M verify tokens against one pass over the weights.
 from __future__ import annotations
 
 import ctypes as C
-from functools import lru_cache
 
 import numpy as np
 
@@ -383,21 +382,17 @@ def gemm_partials(qtype: int, m: int, n: int, k: int, flags: int, ws):
 
 
 # (The sizes are functions of their numbers alone: kept, so that a call with
-# its workspace and outputs at hand asks the library once a shape; by type
-# too, so that a float the library refuses does not meet an equal size.)
-@lru_cache(maxsize=4096, typed=True)
-def _gemm_ws_bytes(qtype: int, m: int, n: int, k: int, flags: int) -> int:
+# its workspace and outputs at hand asks the library once a shape.)
+@_lib.kept_by_size
+def gemm_ws_bytes(qtype: int, m: int, n: int, k: int, flags: int = GEMM_AUTO) -> int:
+    """Workspace bytes ihip_gemm_q needs for this call shape."""
     nb = C.c_size_t()
-    _lib.check(_lib.load().ihip_gemm_q_ws_bytes(qtype, m, n, k, flags, C.byref(nb)))
+    _lib.check(_lib.load().ihip_gemm_q_ws_bytes(qtype, m, n, k, flags & ~(GEMM_REUSE | GEMM_DEFER | GEMM_SUM_OUT),
+                                                    C.byref(nb)))
     return max(int(nb.value), 16)
 
 
-def gemm_ws_bytes(qtype: int, m: int, n: int, k: int, flags: int = GEMM_AUTO) -> int:
-    """Workspace bytes ihip_gemm_q needs for this call shape."""
-    return _gemm_ws_bytes(qtype, m, n, k, flags & ~(GEMM_REUSE | GEMM_DEFER | GEMM_SUM_OUT))
-
-
-@lru_cache(maxsize=4096, typed=True)
+@_lib.kept_by_size
 def packed_bytes(qtype: int, n: int, k: int) -> int:
     """Size of the packed layout of an [n x k] matrix."""
     nb = C.c_size_t()

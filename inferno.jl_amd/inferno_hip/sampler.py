@@ -11,13 +11,12 @@ shim adds 1). There is no CPU fallback.
 from __future__ import annotations
 
 import ctypes as C
-from functools import lru_cache
 
 from . import _lib
 from .quantized_kernels import _ptr, _stream
 
 
-@lru_cache(maxsize=4096, typed=True)
+@_lib.kept_by_size
 def sample_ws_bytes(rows: int, V: int) -> int:
     """Workspace bytes of ihip_sample_ex for rows x V."""
     nb = C.c_size_t()

@@ -13,7 +13,6 @@ from __future__ import annotations
 
 import ctypes as C
 from dataclasses import dataclass
-from functools import lru_cache
 
 from . import _lib
 from .quantized_kernels import _ptr, _stream, check_tensor
@@ -28,14 +27,14 @@ def _ws(nbytes: int, device):
 
 
 # (Workspace sizes: functions of their numbers alone, asked once a shape.)
-@lru_cache(maxsize=4096, typed=True)
+@_lib.kept_by_size
 def _accept_ws_bytes(rows: int, V: int) -> int:
     nb = C.c_size_t()
     _lib.check(_lib.load().ihip_accept_ws_bytes(rows, V, C.byref(nb)))
     return int(nb.value)
 
 
-@lru_cache(maxsize=4096, typed=True)
+@_lib.kept_by_size
 def _spec_accept_ws_bytes(steps: int, k: int, V: int, top_k: int, top_p: float, min_p: float) -> int:
     nb = C.c_size_t()
     _lib.check(_lib.load().ihip_spec_accept_ex_ws_bytes(steps, k, V, top_k, top_p, min_p, C.byref(nb)))

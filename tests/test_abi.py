@@ -246,3 +246,18 @@ def test_sizes_kept_by_shape_still_refuse_floats(lib):
                  lambda: sampler.sample_ws_bytes(1, 4096.0)):
         with pytest.raises(C.ArgumentError):
             call()
+
+
+def test_sizes_of_arrays_and_tensors(lib):
+    """Sizes are kept by plain numbers alone: a 0-d array is taken as before,
+    and a tensor filled anew is asked for again."""
+    import numpy as np
+    import torch
+    from inferno_hip import quantized_kernels as qk
+    from inferno_hip import sampler
+    assert qk.packed_bytes(12, np.array(256), 256) == qk.packed_bytes(12, 256, 256)
+    assert qk.gemm_ws_bytes(12, np.array(1), 256, 256) == qk.gemm_ws_bytes(12, 1, 256, 256)
+    rows = torch.tensor(1)
+    assert sampler.sample_ws_bytes(rows, 4096) == sampler.sample_ws_bytes(1, 4096)
+    rows.fill_(4)
+    assert sampler.sample_ws_bytes(rows, 4096) == sampler.sample_ws_bytes(4, V=4096)
