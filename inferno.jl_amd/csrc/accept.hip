@@ -242,6 +242,26 @@ __device__ __forceinline__ MS load_part(const MS *__restrict__ part, int c, int 
     return c < nchunk ? part[c] : make_ms(-__builtin_huge_valf(), 0.0);
 }
 
+// The same by one thread, eight partials in flight.
+__device__ MS thread_merge(const MS *__restrict__ part, int nchunk) {
+    const float ninf = -__builtin_huge_valf();
+    float m = ninf;
+    double s = 0.0;
+    for (int pass = 0; pass < 2; pass++)
+        for (int c = 0; c < nchunk; c += 8) {
+            MS v[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[j] = part[min(c + j, nchunk - 1)];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                if (c + j >= nchunk || !(v[j].m > ninf)) continue;
+                if (pass == 0) m = fmaxf(m, v[j].m);
+                else s += v[j].s * rescale(v[j].m, m);
+            }
+        }
+    return make_ms(m, s);
+}
+
 // One wave per row.
 __global__ __launch_bounds__(NT) void stats_merge_kernel(const MS *__restrict__ part, int rows, int nchunk,
                                                          float *__restrict__ zmax, float *__restrict__ zsum) {
@@ -751,7 +771,8 @@ __global__ __launch_bounds__(64) void greedy_kernel(const float2 *__restrict__ p
 // node, smallest index on ties, ends the path. Node state lives in LDS up to
 // TREE_LDS nodes; a larger tree is walked by one thread from the workspace.
 // (One thread walking 64 nodes in LDS, each row merged by one thread: 29 us;
-// now 8 us.)
+// now 8 us. Above TREE_LDS nodes the rows are merged a thread each: a wave a
+// row, 5000 nodes of V = 512 took 2.36 ms, 1.99 so.)
 constexpr int TREE_NT = 1024;
 constexpr int TREE_LDS = 4096;
 constexpr int TREE_FAIL = -(1 << 24);
@@ -778,11 +799,15 @@ __global__ __launch_bounds__(TREE_NT) void tree_kernel(const float *__restrict__
         }
         __syncthreads();
     }
-    for (int r = wave; r < 2 * n; r += TREE_NT / 64) {
-        if (in_lds && !s_used[r < n ? r : r - n]) continue;
-        const MS *p = part + (size_t)r * nchunk;
-        const MS v = wave_merge(load_part(p, lane, nchunk), load_part(p, lane + 64, nchunk), p, nchunk);
-        if (lane == 0) ms[r] = v;
+    if (in_lds) {
+        for (int r = wave; r < 2 * n; r += TREE_NT / 64) {
+            if (!s_used[r < n ? r : r - n]) continue;
+            const MS *p = part + (size_t)r * nchunk;
+            const MS v = wave_merge(load_part(p, lane, nchunk), load_part(p, lane + 64, nchunk), p, nchunk);
+            if (lane == 0) ms[r] = v;
+        }
+    } else {  // (all rows, more than 8192: a thread each)
+        for (int r = t; r < 2 * n; r += TREE_NT) ms[r] = thread_merge(part + (size_t)r * nchunk, nchunk);
     }
     __syncthreads();
     // 1 passed, 0 failed, -1 malformed
