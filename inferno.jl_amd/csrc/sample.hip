@@ -629,11 +629,13 @@ __device__ void select_threshold(const float *__restrict__ row, int V, int nroun
     if (gathered) {
         if (t == 0) *ncnt = 0;
         __syncthreads();
+        const int zqm = zq(zmax);
+        const float lo = zb >= 255u ? -__builtin_huge_valf() : grid_lo(zqm - (int)zb), hi = grid_lo(zqm - (int)zb + 1);
         for_rounds(row, V, nround, T, [&](const float (&z)[4], bool in, int) {
             if (!in) return;
 #pragma unroll
             for (int e = 0; e < 4; e++)
-                if (zbin(z[e], zmax) == zb) {
+                if (z[e] >= lo && z[e] < hi) {
                     const int p = atomicAdd(ncnt, 1);  // < nzb: the predicate pass A counted
                     ck[p] = okey(z[e]);
                     cz[p] = z[e];
@@ -899,7 +901,7 @@ __global__ __launch_bounds__(SNT) void draft_sample_kernel(const float *__restri
         Select R;
         select_threshold<false>(Lr, V, nround, invT, zm, 1.f, (unsigned long long)K, s_hist, s_mass, s_sel, s_selm,
                                 (uint32_t *)s_cidx, s_cp, &s_ncnt, R);
-        const uint32_t zb = R.zb, tau = R.tau;
+        const uint32_t tau = R.tau;  // (the keys of a bucket above tau's are larger)
         const int rem = (int)R.rem;  // elements equal to tau that are kept, lowest index first
         int run_kept = 0, run_eq = 0;
         for_rounds(Lr, V, nround, invT, [&](const float (&z)[4], bool in, int r) {
@@ -907,10 +909,9 @@ __global__ __launch_bounds__(SNT) void draft_sample_kernel(const float *__restri
             uint32_t ng = 0, nq = 0;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const uint32_t b = zbin(z[e], zm);
                 const uint32_t k = okey(z[e]);
-                g[e] = in && (b < zb || (b == zb && k > tau));
-                q[e] = in && b == zb && k == tau;
+                g[e] = in && k > tau;
+                q[e] = in && k == tau;
                 ng += g[e];
                 nq += q[e];
             }
