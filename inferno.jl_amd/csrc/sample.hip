@@ -1899,11 +1899,12 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
     __shared__ uint32_t s_off[SMAX_ROUNDS];
     __shared__ uint32_t s_w[128];
     __shared__ uint32_t s_far[SMAX_ROUNDS / 32];  // rounds whose list ends before the threshold's bucket
-    // the threshold bucket's keys, values and indices; then (top-k) the sort
+    // the threshold bucket's keys, values and indices (top-k: the bucket's keys,
+    // the values and indices of it and those above it); then (top-k) the sort
     // scratch, values and indices of the kept entries
     __shared__ uint32_t s_ck[SK_MAX];
-    __shared__ float s_cz[SK_MAX];
-    __shared__ int s_ci[SK_MAX];
+    __shared__ float s_cz[COUNT ? 2 * SK_MAX : SK_MAX];
+    __shared__ int s_ci[COUNT ? 2 * SK_MAX : SK_MAX];
     constexpr unsigned long long CMASK = (1ull << CBITS) - 1ull;
     const int row = blockIdx.x, t = threadIdx.x, wave = t >> 6, lane = t & 63, nround = ws.nround;
     const int g = SPLIT > 0 ? (int)blockIdx.y : 0;
@@ -2101,7 +2102,9 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
     const int nzb = R.all ? 0 : (int)s_hist[R.zb];
     const bool gathered = nzb <= SK_MAX;
     const uint32_t zb = R.zb;
-    // per round: the packed sum of the buckets above zb, and zb's count
+    const bool upto = COUNT && gathered && !R.all;
+    // per round: the packed sum of the buckets above zb, and zb's count (upto:
+    // theirs together)
     rounds([&](int c, int sh, const unsigned long long (&h)[4]) {
         unsigned long long v = 0;
         uint32_t q = 0;
@@ -2115,7 +2118,7 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
         q = wave_sum_u(q);
         if (lane == 0) {
             s_cum[c] = v;
-            s_off[c] = q;
+            s_off[c] = upto ? (uint32_t)v + q : q;
             if ((v & CMASK) + q > (unsigned long long)ws.lmax) atomicOr(&s_far[c >> 5], 1u << (c & 31));
         }
     });
@@ -2134,9 +2137,70 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
                             f);
         gather_far<COUNT>(ws, row, Lr, V, invT, bucket_lo(zb), hi, s_far, s_w, mine, at, also, f);
     };
+    if (COUNT && upto) {
+        // The entries up to the threshold's bucket (fewer than k above it, at
+        // most SK_MAX in it) gathered once, in index order; the threshold among
+        // the bucket's; then the candidates closed up in place. (A gather of
+        // the bucket and another of the candidates: one row of 151936 at top-k
+        // 200 27.9 us and 1000 31.5, 24.8 and 27.2 so.)
+        constexpr int PT = 2 * SK_MAX / SNT;
+        const int nle = (int)(target - R.rem) + nzb;
+        const float hi = grid_lo(zqm - (int)zb + 1);
+        uint32_t tot;
+        const uint32_t off = block_excl_scan_u(t < nround ? s_off[t] : 0u, s_redu, tot);  // (nround <= SNT)
+        if (t < nround) s_off[t] = off;
+        if (t == 0) s_cnt = 0;
+        __syncthreads();
+        gather(
+            __builtin_huge_valf(), [&](int c) { return c + 1 < nround ? s_off[c + 1] > s_off[c] : tot > s_off[c]; },
+            [&](float, int) { return true; },
+            [&](uint32_t p, float z, int j) {
+                if (p < 2u * SK_MAX) {  // (p < nle: the entries chunk_hist_kernel counted)
+                    s_cz[p] = z;
+                    s_ci[p] = j;
+                }
+            });
+        __syncthreads();
+        for (int i = t; i < nle; i += SNT)
+            if (s_cz[i] < hi) s_ck[atomicAdd(&s_cnt, 1)] = okey(s_cz[i]);  // (nzb of them)
+        __syncthreads();
+        refine_threshold<false>(Lr, V, nround, invT, zmax, 1.f, true, nzb, s_hist, s_mass, s_sel, s_selm, s_ck, s_cz, R);
+        const uint32_t rem = (uint32_t)R.rem;  // elements equal to tau that are kept, lowest index first
+        float z[PT];
+        int id[PT];
+        bool gt[PT], eq[PT];
+        uint32_t ng = 0, nq = 0;
+#pragma unroll
+        for (int e = 0; e < PT; e++) {
+            const int j = PT * t + e;
+            const bool in = j < nle;
+            z[e] = in ? s_cz[j] : 0.f;
+            id[e] = in ? s_ci[j] : 0;
+            const uint32_t k = okey(z[e]);  // (a bucket above zb has the larger keys)
+            gt[e] = in && k > R.tau;
+            eq[e] = in && k == R.tau;
+            ng += gt[e];
+            nq += eq[e];
+        }
+        const uint32_t ex = block_excl_scan_u(ng | (nq << 16), s_redu, tot);
+        uint32_t er = ex >> 16, pos = (ex & 0xffffu) + min(rem, er);
+#pragma unroll
+        for (int e = 0; e < PT; e++) {
+            if (gt[e] || (eq[e] && er < rem)) {
+                s_cz[pos] = z[e];
+                s_ci[pos] = id[e];
+                pos++;
+            }
+            er += eq[e];
+        }
+        __syncthreads();
+        draw_candidates((int)(tot & 0xffffu) + (int)min(rem, tot >> 16), a, ur, V, s_ci, s_cz, (int *)s_ck, s_redf, s_redi,
+                        out + row);
+        return;
+    }
     int tie_lim = V, npart = -1;  // (npart >= 0: the threshold's part of the bucket is what was gathered)
     if (!R.all) {
-        if (gathered) {
+        if (!COUNT && gathered) {
             uint32_t tot;
             const uint32_t cnt = t < nround ? s_off[t] : 0u;  // (nround <= SNT)
             const uint32_t off = block_excl_scan_u(cnt, s_redu, tot);
@@ -2236,8 +2300,8 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
             __syncthreads();
         }
         Select Q = R;  // (a copy: R, captured above, stays in registers)
-        refine_threshold<!COUNT>(Lr, V, nround, invT, zmax, COUNT ? 1.f : S, gathered || npart >= 0,
-                                 gathered ? nzb : npart, s_hist, s_mass, s_sel, s_selm, s_ck, s_cz, Q);
+        refine_threshold<!COUNT>(Lr, V, nround, invT, zmax, COUNT ? 1.f : S, !COUNT && (gathered || npart >= 0),
+                                 !COUNT && gathered ? nzb : npart, s_hist, s_mass, s_sel, s_selm, s_ck, s_cz, Q);
         R = Q;
         if (R.all) {  // (the entries' masses a rounding short of the rounds': the whole bucket is kept)
             R.all = false;
@@ -2257,7 +2321,7 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
         if (n_eq < 1) n_eq = 1;
         const uint32_t tau = R.tau;
         if (n_eq < R.cnt) {
-            if (gathered) {  // the gather is in index order: slots 4 t .. 4 t + 3
+            if (!COUNT && gathered) {  // the gather is in index order: slots 4 t .. 4 t + 3
                 bool q[4];
                 uint32_t nq = 0;
 #pragma unroll
@@ -2311,7 +2375,7 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
         auto units = [&](float z, uint32_t k, int j) {
             return k > tau || (k == tau && j < tie_lim) ? COUNT ? 1ull : (mass_fx(z, zmax, invS) << CBITS) + 1ull : 0ull;
         };
-        if (gathered || npart >= 0) {
+        if (!COUNT && (gathered || npart >= 0)) {
             for (int i = t; i < (gathered ? nzb : npart); i += SNT) {
                 const unsigned long long v = units(s_cz[i], s_ck[i], s_ci[i]);
                 if (v) atomicAdd(&s_cum[s_ci[i] / SROUND], v);
