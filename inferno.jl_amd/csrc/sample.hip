@@ -660,7 +660,7 @@ __device__ __forceinline__ bool above_threshold(float z, int j, float zmax, uint
 // sum, a sorted slot the count of the candidates before it), without the
 // ~30 barriers of the block form (sort 21, sums and scans 2-3 each), which
 // were most of an 18 us draw of 40 candidates.
-__device__ __forceinline__ void draw_candidates_wave(int n, const SampleArgs &a, float ur, int V, const int *s_cidx, float *s_cp,
+__device__ __forceinline__ void draw_candidates_wave(int n, SampleArgs a, float ur, int V, const int *s_cidx, float *s_cp,
                                      int *s_sort, int32_t *out_row) {
     const int l = threadIdx.x;
     // first_cdf_hit over slots 4 l + e of the first 16 lanes
@@ -729,7 +729,7 @@ __device__ __forceinline__ void draw_candidates_wave(int n, const SampleArgs &a,
 // exp(-Inf) = 0), top-p by a bitonic sort of their probabilities, min-p,
 // then the inverse CDF in index order.
 // (n <= 64: by wave 0 alone, draw_candidates_wave.)
-__device__ void draw_candidates(int n, const SampleArgs &a, float ur, int V, int *s_cidx, float *s_cp, int *s_sort,
+__device__ void draw_candidates(int n, SampleArgs a, float ur, int V, int *s_cidx, float *s_cp, int *s_sort,
                                 float *s_redf, int *s_redi, int32_t *out_row) {
     const int t = threadIdx.x;
     if (n <= 64) {
