@@ -512,7 +512,8 @@ __device__ __noinline__ void refine_passes(const float *__restrict__ row, int V,
     // the bits below the highest in which two keys of the bucket can differ
     const int zqm = zq(zmax);
     const float lo = zb >= 255u ? -__builtin_huge_valf() : grid_lo(zqm - (int)zb);
-    const uint32_t khi = okey(grid_lo(zqm - (int)zb + 1)) - 1u, klo = okey(lo == 0.f ? -0.f : lo);
+    const float hi = grid_lo(zqm - (int)zb + 1);
+    const uint32_t khi = okey(hi) - 1u, klo = okey(lo == 0.f ? -0.f : lo);
     const int nbits = max(32 - __clz(klo ^ khi), 1);
     uint32_t pmask = nbits == 32 ? 0u : ~0u << nbits, prefix = khi & pmask;
     for (int top = nbits; top > 0; top -= 8) {
@@ -539,7 +540,7 @@ __device__ __noinline__ void refine_passes(const float *__restrict__ row, int V,
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     const uint32_t k = okey(z[e]);
-                    q[e] = in && (k & pmask) == prefix && zbin(z[e], zmax) == zb;
+                    q[e] = in && (k & pmask) == prefix && z[e] >= lo && z[e] < hi;
                     b[e] = (k >> shift) & digit;
                     m[e] = MASS && q[e] ? mass_fx(z[e], zmax, invS) : 0ull;
                 }
@@ -2251,13 +2252,14 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
             }
             if (t == 0) s_cnt = 0;
             __syncthreads();
+            const float lo = bucket_lo(zb), hi = grid_lo(zqm - (int)zb + 1);
             for_rounds(Lr, V, nround, invT, [&](const float (&z)[4], bool in, int) {
                 bool q[4];
                 uint32_t b[4];
                 unsigned long long m[4];
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    q[e] = in && zbin(z[e], zmax) == zb;
+                    q[e] = in && z[e] >= lo && z[e] < hi;
                     b[e] = zpart(z[e]);
                     m[e] = q[e] ? mass_fx(z[e], zmax, invS) : 0ull;
                 }
@@ -2277,7 +2279,7 @@ __global__ __launch_bounds__(SNT) void row_threshold_kernel(const float *__restr
                     if (in)
 #pragma unroll
                         for (int e = 0; e < 4; e++)
-                            if (zbin(z[e], zmax) == zb) {
+                            if (z[e] >= lo && z[e] < hi) {
                                 const uint32_t b = zpart(z[e]);
                                 if (b > part) v += (mass_fx(z[e], zmax, invS) << CBITS) + 1ull;
                                 if (b == part) {
