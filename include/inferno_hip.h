@@ -468,11 +468,11 @@ int ihip_sample(const float *logits_dev, int rows, int V, float T, int top_k,
  * plain draws (T > 0, no top-k, top-p or min-p: the speculative defaults)
  * spread each row over workgroups of 4096 logits (their softmax
  * statistics, then the draw inside the round that holds u); so do top-k up to
- * 4096 and top-p (each chunk's threshold histogram and candidate list,
- * then one workgroup per row for the threshold and the draw: with top-k
- * ihip_sample's tokens; a top-k above 4096 takes ihip_sample's path),
- * min-p (the chunks' kept sums)
- * and T = 0 (each chunk's first argmax: the tokens of ihip_sample). The
+ * 4096 and top-p (each chunk's threshold histogram and candidate list, then
+ * the threshold and the draw by one workgroup per row, for top-p of up to 32
+ * rows by 16 or 8: with top-k ihip_sample's tokens; a top-k above 4096 takes
+ * ihip_sample's path), min-p (the chunks' kept sums) and T = 0 (each chunk's
+ * first argmax: the tokens of ihip_sample). The
  * same limits and the same softmax_sample
  * (src/ModelCPU.jl:1123-1200) and the same contract: draws match the exact
  * cumulative distribution except within rounding of a step. */

@@ -11,7 +11,7 @@
 //  * T = 0: Julia's argmax (the first NaN above every number, +0.0 above
 //    -0.0, the first of equals) by an integer key.
 //  * top-k (1 <= k <= 4096, k < V): exact radix select of the k-th largest
-//    z = L / T (8 bits a pass on an order-preserving key), ties at the
+//    z = L / T (buckets, then an order-preserving key's bits), ties at the
 //    threshold kept lowest index first (the stable descending sortperm);
 //    the k candidates are compacted into LDS in index order, and softmax,
 //    top-p (a bitonic sort by probability, then a scan), min-p and the draw
@@ -27,7 +27,7 @@
 //  * with a workspace, every setting spreads each row over workgroups of
 //    one round (chunk statistics, each chunk's argmax, threshold histograms
 //    and candidate lists, kept sums), and one workgroup per row finishes
-//    each stage from them.
+//    each stage from them (16 or 8 where a few rows' top-p is flat).
 // Sums and scans are trees, where the reference accumulates sequentially:
 // the drawn token can differ only where u falls within rounding of a CDF
 // step.
@@ -1571,16 +1571,17 @@ __global__ __launch_bounds__(SNT) void argmax_draw_kernel(int V, const float2 *_
 //    first those past one whose thread maxima number k, before the atomics);
 //  * the candidate list: (z, index) of its entries up to bucket `last`, the
 //    largest that leaves at most lmax of them, in index order.
-// Then one workgroup per row takes the row's statistics, brings the
-// histograms to the row's buckets and masses, finds the threshold's bucket,
-// takes that bucket's entries from the lists (from the row, for a round whose
-// list ends before it), finds the threshold among them, and draws: top-k
-// over the kept entries (draw_candidates), top-p by the rounds' kept masses
-// (the buckets above the threshold's, plus its kept entries), then inside
-// the round u falls in; with at most 64 entries up to the threshold's bucket
-// one wave does all of it. Two launches where there were three (top-k <= 64),
-// eight (larger) and six (top-p): 64 rows of 151936 at top-p 0.9 95 -> 33 us,
-// one row at top-k 40 + top-p 28.6 -> 18.7 us.
+// Then one workgroup per row (SPLIT: more) takes the row's statistics, brings
+// the histograms to the row's buckets and masses, finds the threshold's
+// bucket, takes that bucket's entries (top-k: and those above it) from the
+// lists (from the row, for a round whose list ends before it), finds the
+// threshold among them, and draws: top-k over the kept entries
+// (draw_candidates), top-p by the rounds' kept masses (the buckets above the
+// threshold's, plus its kept entries), then inside the round u falls in; with
+// at most 64 entries up to the threshold's bucket one wave does all of it.
+// Two launches where there were three (top-k <= 64), eight (larger) and six
+// (top-p): 64 rows of 151936 at top-p 0.9 95 -> 28 us, one row at top-k 40 +
+// top-p 28.6 -> 18.1 us, at top-k 1000 34.7 -> 26.9.
 enum : int { SEL_SELECT = 0, SEL_ALL = 1, SEL_DEGEN = 2 };
 struct RowSel {
     int mode;
@@ -2684,11 +2685,12 @@ size_t sample_spread_ws(int rows, int V) {
 }
 
 // Rows spread over workgroups of one round each: plain draws (T > 0, no top-k,
-// top-p or min-p): chunk statistics, then one workgroup per row merges them, picks the round and scans it (as draft_sample_kernel's draw);
-// top-k up to SK_MAX (any top-p / min-p after it) and top-p: histograms and
-// candidate lists, then one workgroup per row for the threshold and the
-// draw; min-p, alone or after top-p: the chunks' kept sums, then
-// the draw; T = 0: each chunk's argmax, then the row's. Rows over more than
+// top-p or min-p): chunk statistics, then one workgroup per row merges them,
+// picks the round and scans it (as draft_sample_kernel's draw); top-k up to
+// SK_MAX (any top-p / min-p after it) and top-p: histograms and candidate
+// lists, then the threshold and the draw per row; min-p, alone or after top-p:
+// the chunks' kept sums, then the draw; T = 0: each chunk's argmax, then the
+// row's. Rows over more than
 // SMAX_ROUNDS rounds, and a larger top-k, run draft_sample_kernel.
 // ws: sample_spread_ws bytes (8-byte aligned).
 hipError_t launch_sample_spread(const float *L, int rows, int V, float T, int top_k, float top_p, float min_p,
