@@ -1288,9 +1288,9 @@ struct SpreadWs {
 // The entries of a list: LIST_MAX, or for a top-k of many entries a round
 // (twice the mean and 128; a multiple of 8, so that a header stays 8-byte
 // aligned) as many as the row's ROW_BYTES hold for each round (top-k 4000 of
-// 32000: 45 us with lists of LIST_MAX, 32 so). A row of 1 or 2 rounds is read
-// whole instead (gather_far; top-k 4000 of 8192: 31 us, 43 with lists of 4088
-// entries, a wave each).
+// 32000: 31.5 us with lists of LIST_MAX, 24.6 so; 64 rows of 50257 46.7 and
+// 31.1). A row of 1 or 2 rounds is read whole instead (gather_far; top-k 4000
+// of 8192: 25.4 us, 32.6 with lists of 4088 entries, a wave each).
 constexpr int list_max(int nround, int top_k) {
     const int want = (2 * top_k / nround + 128) / 8 * 8, room = ((int)(ROW_BYTES - 256) / nround - 16) / 6 / 8 * 8;
     const int n = want < room ? want : room;
